@@ -317,8 +317,8 @@ int rt_rope_kv_append(rt_ctx* ctx, float* q, float* k, const float* v, float* k_
 int rt_attention(rt_ctx* ctx, const float* q, const float* k_cache, const float* v_cache, float* out, int M, int H,
                  int Hkv, int hd, int Lmax, const int* pos);
 
-/* Decode form of rt_attention for one query (M = 1, flash-decoding): the keys are split
- * over workgroups of 64; each writes a partial softmax result to `workspace` (at least
+/* Decode form of rt_attention for one query (M = 1, flash-decoding): the keys, in blocks of
+ * 64, are dealt to at most 10 workgroups per query head; each writes a partial softmax result to `workspace` (at least
  * rt_attention_decode_workspace(H, hd, Lmax) bytes of device memory, no initialisation
  * needed), then a second launch combines them into out [H*hd].  head_dim 64 or 128.
  * rt_attention_decode_partials stops after the first launch; a fused plan with source

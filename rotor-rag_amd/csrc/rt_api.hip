@@ -1384,8 +1384,10 @@ int rt_plan_attach_attention(rt_plan* plan, float* k_cache, float* v_cache, cons
     t.Lmax = Lmax;
     t.S = attn_splits(Lmax);
     // the group's query heads two to a workgroup where they split evenly: the tiles' arithmetic
-    // (one CU per workgroup) then spreads over twice the CUs
-    t.hpw = Gq % 2 == 0 && Gq >= 4 ? Gq / 2 : Gq;
+    // (one CU per workgroup) then spreads over twice the CUs.  With two tiles per head the
+    // workgroup's Gq tiles hold half the heads (or one, of an odd group).
+    t.T = attn_tiles(Lmax);
+    t.hpw = Gq % 2 == 0 && (Gq >= 4 || t.T == 2) ? Gq / 2 : t.T == 2 ? 1 : Gq;
     t.natt = (unsigned)(Hkv * t.S * (Gq / t.hpw));
     t.wrap = t.natt * (0xFFFFFFFFu / t.natt) - 1u;
     t.qrows = H * hd;
@@ -1404,7 +1406,7 @@ int rt_plan_attention_combine(rt_plan* plan, float* out, double* ssq) {
     if (out) {
         if (!plan->att_on) return fail(RT_EINVAL, std::string(who) + ": attach the attention first "
                                                                      "(rt_plan_attach_attention)");
-        if (plan->att.S > kAttnSMax)
+        if (attn_blocks(plan->att.Lmax) > kAttnSMax)
             return fail(RT_EINVAL, std::string(who) + ": at most " + std::to_string(kAttnSMax) +
                                        " key blocks (Lmax <= " + std::to_string(64 * kAttnSMax) + ")");
         if (((uintptr_t)out & 15u) || ((uintptr_t)ssq & 7u))

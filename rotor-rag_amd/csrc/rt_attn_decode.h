@@ -1,15 +1,21 @@
-// Decode attention over one block of 64 keys for one query head: the work of a
-// 256-thread tile, shared by the split-L attention kernel (rt_model.hip) and by the qkv
+// Decode attention over one split of the keys for one query head: the work of one or two
+// 256-thread tiles, shared by the split-L attention kernel (rt_model.hip) and by the qkv
 // GEMV launch that runs the attention partials in its trailing workgroups (rt_gemv.hip).
 //
 // Reference: MultiHeadAttention.forward (src/rotor/transformer.py:206-292: KV concat
 // :250-252, GQA repeat :260-263, scores/softmax/AV :267-281); this build adds RoPE and a
 // causal mask (the benchmark configuration).
 //
-// The tile (h, s) handles keys [64 s, 64 s + 64) of query head h for the single query at
-// position pos and writes a partial result wp[0..HD+2): the unnormalised output
-// sum_j e^(s_j - m) V_j (HD values), the block maximum m and the sum of exponentials z
-// (m = -inf, z = 0 for an empty block).  The partials are combined by attn_combine_kernel,
+// The keys go in blocks of 64, dealt to S = attn_splits(Lmax) splits: split s of query head h
+// takes blocks s, s + S, ..  Up to 640 keys (S = the block count) that is one block for one
+// tile; past that S stays at 10 and the split's blocks go alternately to its attn_tiles = 2
+// tiles, each with an online softmax over its own, tile 1's (m, z, o) merged into tile 0's.
+// The fixed S is what o_proj's prologue pays for: every one of its 40 workgroups combines all
+// S partials of all heads (32 splits at Lmax 2048: 31.4 us a launch; 10: 8.2 us), and the
+// launch itself no longer runs a workgroup per 64 keys of Lmax, mostly past the position.
+// The split writes a partial result wp[0..HD+2) for the single query at position pos: the
+// unnormalised output sum_j e^(s_j - m) V_j (HD values), the maximum m and the sum of
+// exponentials z (m = -inf, z = 0 for an empty split).  The partials are combined by attn_combine_kernel,
 // by the prologue of the o_proj GEMV (rt_rowquant.h, kAttnNorm) or in the qkv launch; all
 // use the operation order of attn_combine_element, so they give identical values.
 #pragma once
@@ -18,7 +24,7 @@
 
 namespace rt {
 
-constexpr int kAttnBlock = 64;  // keys per split
+
 
 // Workgroup barrier for the tile's LDS hand-offs: waits for this wave's LDS accesses only.
 // __syncthreads() also waits for the wave's outstanding global stores (its fence), which
@@ -39,6 +45,14 @@ struct AttnTileLds {
     float pr[kAttnBlock];
     float ored[256];
 };
+
+// attn_tile2's further words, after the tiles: this block's factor of the running output, the
+// tile's m and z.  (In AttnTileLds itself, 12 bytes more left the next tile's arrays 4-byte
+// aligned, its LDS reads 4 bytes wide and the launch 0.4 us longer.)
+struct AttnRun {
+    float alpha, m, z, pad;
+};
+typedef __attribute__((address_space(3))) AttnRun lds_run;
 
 // The tile's LDS is reached through a local-address-space pointer: through a generic one,
 // a select between an LDS value and a register of the key block (the new key) becomes a
@@ -70,6 +84,39 @@ __device__ __forceinline__ void attn_kv_load(const float* __restrict__ Kc, const
     for (int i = 0; i < KV::VN; ++i) kv.v[i] = V[(size_t)min(j0 + g + i * KV::G, Lmax - 1) * HD];
 }
 
+// The same shares of one block after another (attn_tile2), keys and values apart: buffer loads
+// from the block's first key, one VGPR offset for all of them, the dimension's row in the
+// scalar offset (K) or the key group in the range-checked vector offset (V: keys past Lmax
+// read as zeros).  Per-load 64-bit addresses, kept over the loop of blocks, made it spill.
+template <int HD>
+__device__ __forceinline__ void attn_k_load(const float* __restrict__ Kc, int kh, int j0, int Lmax, int t,
+                                            AttnKV<HD>& kv) {
+    using KV = AttnKV<HD>;
+    const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int jb = min(j0, Lmax - 1);
+    const float* K = Kc + ((size_t)kh * HD + (size_t)wave * KV::KD) * Lmax + jb;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)K, 0, 0xFFFFFFFFu, kBufDword3);
+    const int off = 4 * min(lane, Lmax - 1 - jb);
+    int row = Lmax * 4;
+    asm volatile("" : "+s"(row));  // (the row offsets are not kept in SGPRs from block to block)
+#pragma unroll
+    for (int i = 0; i < KV::KD; ++i)
+        kv.k[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, off, i * row, 0));
+}
+template <int HD>
+__device__ __forceinline__ void attn_v_load(const float* __restrict__ Vc, int kh, int j0, int Lmax, int t,
+                                            AttnKV<HD>& kv) {
+    using KV = AttnKV<HD>;
+    const int jb = min(j0, Lmax - 1);
+    const float* V = Vc + ((size_t)kh * Lmax + jb) * HD;
+    const unsigned range = (unsigned)min(Lmax - jb, kAttnBlock) * HD * 4u;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)V, 0, range, kBufDword3);
+    // key g + i G, dim d of t = g HD + d
+#pragma unroll
+    for (int i = 0; i < KV::VN; ++i)
+        kv.v[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, 4 * t + i * KV::G * HD * 4, 0, 0));
+}
+
 // The RoPE factors (cos, sin) of rotation pair t (t < HD / 2) at position pos: loaded by
 // the caller as early as the position is known (the tile's first step waits for them).
 template <int HD>
@@ -82,7 +129,7 @@ __device__ __forceinline__ void attn_rope_load(const float* __restrict__ rope, i
     }
 }
 
-// The tile's work once the position is known and the block holds at least one key
+// The one-block tile's work once the position is known and the block holds at least one key
 // (pos >= j0).  Every thread of the workgroup passes the tile's four barriers.
 // qh: the head's query (HD values); kn, vn: the head's KV group's new key and value (ROPE),
 // in global memory or in LDS (SRC, a pointer type); c, sn: attn_rope_load's factors (ROPE).
@@ -225,7 +272,162 @@ __device__ __forceinline__ void attn_tile(SRC qh, SRC kn, SRC vn, float c, float
         }
 }
 
-// The partial of an empty block (no key at or before the position): m = -inf, z = 0; with
+// The work of tile `tile` (0 or 1) of a split of several blocks (Lmax > 640), once the position
+// is known and the split holds at least one key (pos >= js, its first block's first key).  The
+// two tiles take the split's blocks in turn, a pair a round, with an online softmax each; every
+// thread of the workgroup passes the same barriers, and a tile whose block of the last round
+// lies past the position sits that round out.  kv holds the tile's first block (keys
+// js + 64 S tile ..) on entry; the next block's keys are requested once this one's scores are
+// taken, its values once this one's sums are.  sm1, run1: the head's tile 1, whose
+// (m, z, o) tile 0 merges at the end.  The other arguments are attn_tile's.  (One form for both
+// cost the one-block launch 0.5 us: the loop's block arithmetic, the late store of m and z and
+// the new value's own addition.)
+template <int HD, bool ROPE, typename SRC>
+__device__ __forceinline__ void attn_tile2(SRC qh, SRC kn, SRC vn, float c, float sn, float* __restrict__ Kc,
+                                          float* __restrict__ Vc, int kh, bool writer, int Lmax, int pos, int js, int S,
+                                          int tile, float scale, float* __restrict__ wp, int t, AttnLdsPtr<HD> sm,
+                                          AttnLdsPtr<HD> sm1, lds_run* run, lds_run* run1, AttnKV<HD>& kv) {
+#pragma clang fp contract(off)  // every operation rounds on its own, fmaf where written
+    using KV = AttnKV<HD>;
+    constexpr int T = 2, BL = kAttnBlock, half = HD / 2, G = KV::G, KD = KV::KD, VN = KV::VN;
+    constexpr int CH = VN >= 8 ? 8 : VN;
+    static_assert(VN % CH == 0 && CH % 2 == 0, "runs of key pairs");
+    const int lane = t & 63, wave = t >> 6, d = t % HD, g = t / HD;
+    const int step = S * BL * T;                                    // keys from one round's block to the next
+    const int rounds = (pos - js) / step + 1;
+    int j0 = js + tile * S * BL;                              // this tile's block
+    // the tile's last block ends with the new key
+    const bool any_new = ROPE && pos >= j0 && (pos - j0) % step < BL;
+    if (ROPE) {
+        if (t < half) {
+            const int i = t;
+            const float x1 = qh[i], x2 = qh[i + half];
+            sm->qs[i] = x1 * c - x2 * sn;
+            sm->qs[i + half] = x2 * c + x1 * sn;
+            if (any_new) {
+                const float k1 = kn[i], k2 = kn[i + half];
+                sm->ks[i] = k1 * c - k2 * sn;
+                sm->ks[i + half] = k2 * c + k1 * sn;
+            }
+        }
+        if (any_new)
+            for (int e = t; e < HD; e += 256) sm->vs[e] = vn[e];
+    } else {
+        for (int e = t; e < HD; e += 256) sm->qs[e] = qh[e];
+    }
+    attn_lds_barrier();
+    float o0 = 0.f, o1 = 0.f, mrun = -INFINITY, zrun = 0.f;  // mrun, zrun: wave 0's (zrun in lane 63)
+    for (int r = 0; r < rounds; ++r, j0 += step) {
+        const bool live = j0 <= pos;                   // the tile's block holds a key
+        const bool more = j0 + step <= pos;            // and so does its next one
+        const int nk = min(BL, pos + 1 - j0);          // keys of this block
+        const bool holds_new = any_new && live && pos < j0 + BL;  // this block ends with the new key
+        const int lp = pos - j0;                       // its lane / key index in the block
+        // scores, as attn_tile's
+        if (live) {
+            if (holds_new && lane == lp) {
+#pragma unroll
+                for (int i = 0; i < KD; ++i) kv.k[i] = sm->ks[wave * KD + i];
+            }
+            float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
+#pragma unroll
+            for (int i = 0; i < KD; i += 4) {
+                const int dd = wave * KD + i;
+                a0 = fmaf(sm->qs[dd + 0], kv.k[i + 0], a0);
+                a1 = fmaf(sm->qs[dd + 1], kv.k[i + 1], a1);
+                a2 = fmaf(sm->qs[dd + 2], kv.k[i + 2], a2);
+                a3 = fmaf(sm->qs[dd + 3], kv.k[i + 3], a3);
+            }
+            sm->part[wave][lane] = (a0 + a1) + (a2 + a3);
+            if (more) attn_k_load<HD>(Kc, kh, j0 + step, Lmax, t, kv);
+        }
+        attn_lds_barrier();
+        if (wave == 0 && live) {
+            float sc = lane < nk
+                           ? (((sm->part[0][lane] + sm->part[1][lane]) + (sm->part[2][lane] + sm->part[3][lane])) * scale)
+                           : -INFINITY;
+            const float mx = fmaxf(mrun, lane63(wave_reduce63(sc, -INFINITY, [](float x, float y) { return fmaxf(x, y); })));
+            const float p = lane < nk ? expf(sc - mx) : 0.0f;
+            const float z = wave_reduce63(p, 0.0f, [](float x, float y) { return x + y; });
+            sm->pr[lane] = p;
+            if (r > 0) {  // (the first block's sums start from zero)
+                const float al = expf(mrun - mx);
+                if (lane == 63) run->alpha = al;
+                zrun = fmaf(zrun, al, z);
+            } else {
+                zrun = z;
+            }
+            mrun = mx;
+        }
+        attn_lds_barrier();
+        // unnormalised output: attn_tile's sums, scaled to the new maximum first
+        if (live) {
+            if (r > 0) {
+                const float al = run->alpha;
+                o0 *= al;
+                o1 *= al;
+            }
+            // the new key, the block's last, is added after the cached ones (the same order)
+            const int nc = holds_new ? lp : nk;
+#pragma unroll
+            for (int c0 = 0; c0 < VN; c0 += CH) {
+                const int first = g + c0 * G, last = g + (c0 + CH - 1) * G;
+                if (last < nc) {
+#pragma unroll
+                    for (int i = c0; i < c0 + CH; i += 2) {
+                        o0 = fmaf(sm->pr[g + i * G], kv.v[i], o0);
+                        o1 = fmaf(sm->pr[g + (i + 1) * G], kv.v[i + 1], o1);
+                    }
+                } else if (first < nc) {
+#pragma unroll
+                    for (int i = c0; i < c0 + CH; i += 2) {
+                        const int ja = g + i * G, jb = g + (i + 1) * G;
+                        const float sa = fmaf(sm->pr[ja], kv.v[i], o0), sb = fmaf(sm->pr[jb], kv.v[i + 1], o1);
+                        o0 = ja < nc ? sa : o0;
+                        o1 = jb < nc ? sb : o1;
+                    }
+                }
+            }
+            if (holds_new) {
+                // its slot among this thread's keys g, g + G, .. (g and lp uniform over the wave)
+                const int rel = __builtin_amdgcn_readfirstlane(lp - g);
+                if (rel >= 0 && rel % G == 0) {
+                    const float pn = sm->pr[lp], vn1 = sm->vs[d];
+                    if ((rel / G) & 1) o1 = fmaf(pn, vn1, o1);
+                    else o0 = fmaf(pn, vn1, o0);
+                }
+            }
+            if (more) attn_v_load<HD>(Vc, kh, j0 + step, Lmax, t, kv);
+        }
+    }
+    sm->ored[t] = o0 + o1;
+    if (wave == 0 && lane == 63) {
+        run->m = mrun;
+        run->z = zrun;
+    }
+    attn_lds_barrier();
+    if (tile == 0 && g == 0) {
+        float o = sm->ored[d];
+        for (int gg = 1; gg < G; ++gg) o += sm->ored[gg * HD + d];
+        // tile 0 holds the split's first block; tile 1 may hold none (m = -inf)
+        const float m0 = run->m, m1 = run1->m, m = fmaxf(m0, m1);
+        const float f0 = expf(m0 - m), f1 = m1 == -INFINITY ? 0.0f : expf(m1 - m);
+        float ob = sm1->ored[d];
+        for (int gg = 1; gg < G; ++gg) ob += sm1->ored[gg * HD + d];
+        wp[d] = fmaf(f1, ob, f0 * o);
+        if (d == 0) {
+            wp[HD] = m;
+            wp[HD + 1] = fmaf(f1, run1->z, f0 * run->z);
+        }
+    }
+    if (any_new && writer)
+        for (int e = t; e < HD; e += 256) {
+            Kc[((size_t)kh * HD + e) * Lmax + pos] = sm->ks[e];
+            Vc[((size_t)kh * Lmax + pos) * HD + e] = sm->vs[e];
+        }
+}
+
+// The partial of an empty split (no key at or before the position): m = -inf, z = 0; with
 // TAG every word of the tagged copy is written (the values as 0), so a reader can wait for
 // all of them.
 template <int HD, bool TAG = false>

@@ -329,7 +329,10 @@ constexpr int kAttnMaxThreads = 640;
 // same launch (qkv_attn_block): the GEMV's outputs are also stored as epoch-tagged
 // device-coherent words, which the attention workgroups poll.
 struct NoTail {};
-template <int HD>
+// the same tail with two tiles per query head (Lmax > 640), a kernel of its own: one kernel
+// holding both forms of the tile spills
+struct AttnTailLong : AttnTail {};
+template <int HD, int T>
 __device__ __forceinline__ void qkv_attn_block(const AttnTail& at, int total_rb);
 // The launch's epoch (AttnTail): *done / natt + 1, the same for every workgroup of a launch.
 __device__ __forceinline__ unsigned attn_epoch(const AttnTail& at) {
@@ -339,14 +342,14 @@ template <int MT, int PRO, bool PAIR = false, typename Tail = NoTail>
 __global__ void __launch_bounds__(PRO == 2 ? kAttnMaxThreads : 1024)
     gemv_ksplit_kernel(const float* pro_x, const float* pro_aux, const float* pro_aux2, int pro_K, int pro_mode,
                        float pro_eps, unsigned shape, unsigned nw_m, const v4u* w1, GemvArgs a, Tail at) {
-    constexpr bool SIG = std::is_same<Tail, AttnTail>::value;
+    constexpr bool SIG = std::is_base_of<AttnTail, Tail>::value;
     if constexpr (SIG) {
         // the GEMV's workgroup count rides in the shape word (a launch of inline problems
         // has no C1), so the GEMV workgroups start without a kernel-argument load
         static_assert(MT == 1 && !PAIR, "attention partials follow the one-token qkv GEMV");
         const int total_rb = (int)(shape >> 8);
         if ((int)blockIdx.x >= total_rb) {
-            qkv_attn_block<128>(at, total_rb);
+            qkv_attn_block<128, std::is_same<Tail, AttnTailLong>::value ? 2 : 1>(at, total_rb);
             return;
         }
     }
@@ -531,12 +534,12 @@ __global__ void __launch_bounds__(PRO == 2 ? kAttnMaxThreads : 1024)
 
 // Decode qkv GEMV (E-element RMSNorm prologue) with the attention partials of the token in
 // the same launch: workgroups [0, total_rb) are the GEMV's row blocks (q, k, v problems),
-// the following Hkv * P workgroups (P = S Gq / hpw) the attention of (KV head kh, key block
-// s, query heads hp hpw .. hp hpw + hpw - 1 of the group), kh slowest, then hp, each of hpw
-// 256-thread tiles (blockDim = 256 Gq: the waves past hpw tiles end at once).  Splitting a
+// the following Hkv * P workgroups (P = S Gq / hpw) the attention of (KV head kh, split
+// s, query heads hp hpw .. hp hpw + hpw - 1 of the group), kh slowest, then hp, each of hpw T
+// 256-thread tiles (blockDim = 256 Gq: the waves past them end at once).  Splitting a
 // group's heads over workgroups spreads the tiles' arithmetic over more CUs.  An attention
-// workgroup issues its key block's loads and reads the position and the epoch; when its
-// block holds a key, its first (hpw + 2) hd threads (one per q value of its heads and k, v
+// workgroup issues its first key blocks' loads and reads the position and the epoch; when its
+// split holds a key, its first (hpw + 2) hd threads (one per q value of its heads and k, v
 // value of its KV group) poll the GEMV's tagged outputs (bounded) until each carries the
 // epoch and leave the values in LDS, and the tiles of rt_attn_decode.h run on them.
 // Forward progress: the attention workgroups wait only for GEMV workgroups, which come
@@ -612,24 +615,33 @@ __device__ __forceinline__ void attn_peer_combine(const AttnTail& at, int kh, in
     if (act && (t & 31) == 31) at.ssq[k >> 5] = ss;
 }
 
-template <int HD>
+template <int HD, int T>
 __device__ __forceinline__ void qkv_attn_block(const AttnTail& at, int total_rb) {
     extern __shared__ __attribute__((aligned(16))) int red[];
-    // attention workgroup i: KV group kh, peer r = hp S + s in the group (key block s, query
-    // heads [hp hpw, hp hpw + hpw) of the group), one 256-thread tile per head; the waves past
-    // them end here, before any barrier
+    // attention workgroup i: KV group kh, peer r = hp S + s in the group (split s, query
+    // heads [hp hpw, hp hpw + hpw) of the group), T 256-thread tiles per head, all heads' tile 0
+    // first; the waves past them end here, before any barrier
     const int i = (int)blockIdx.x - total_rb, P = at.S * (at.Gq / at.hpw);
     const int kh = i / P, r = i - kh * P, hp = r / at.S, s = r - hp * at.S;
-    const int sub = (int)(threadIdx.x >> 8), t = (int)(threadIdx.x & 255);
-    if (sub >= at.hpw) return;
-    const int h0 = kh * at.Gq + hp * at.hpw, h = h0 + sub;
+    const int t = (int)(threadIdx.x & 255);
+    int sub = (int)(threadIdx.x >> 8);
+    if constexpr (T == 2) sub = __builtin_amdgcn_readfirstlane(sub);
+    if (sub >= at.hpw * T) return;
+    const int tile = T == 2 && sub >= at.hpw ? 1 : 0, hd_i = sub - tile * at.hpw;
+    const int h0 = kh * at.Gq + hp * at.hpw, h = h0 + hd_i;
     const AttnLdsPtr<HD> sm = (AttnLdsPtr<HD>)red;
     typedef __attribute__((address_space(3))) float lfl;
-    lfl* const qkv = (lfl*)(sm + at.hpw);  // the heads' q (hpw HD), the group's k (HD), v (HD)
+    lfl* const qkv = (lfl*)(sm + at.hpw * T);  // the heads' q (hpw HD), the group's k (HD), v (HD)
+    lds_run* const run = (lds_run*)(qkv + (at.hpw + 2) * HD);  // T = 2
     const int j0 = s * kAttnBlock;
     const int nin = (at.hpw + 2) * HD;
     AttnKV<HD> kv;
-    attn_kv_load<HD>(at.Kc, at.Vc, kh, j0, at.Lmax, t, kv);
+    if constexpr (T == 1) {
+        attn_kv_load<HD>(at.Kc, at.Vc, kh, j0, at.Lmax, t, kv);
+    } else {
+        attn_k_load<HD>(at.Kc, kh, j0 + tile * at.S * kAttnBlock, at.Lmax, t, kv);
+        attn_v_load<HD>(at.Vc, kh, j0 + tile * at.S * kAttnBlock, at.Lmax, t, kv);
+    }
     const unsigned ep = attn_epoch(at);
     const int pos = *at.pos;
     float* wp = at.work + ((size_t)h * at.S + s) * (HD + 2);
@@ -660,13 +672,18 @@ __device__ __forceinline__ void qkv_attn_block(const AttnTail& at, int total_rb)
         }
         __syncthreads();
         // one writer of the new key and value per KV group: the group's last head
-        attn_tile<HD, true, true>(qkv + sub * HD, qkv + at.hpw * HD, qkv + (at.hpw + 1) * HD, c, sn, at.Kc, at.Vc,
-                                  kh, h == kh * at.Gq + at.Gq - 1, at.Lmax, pos, j0, at.scale, wp, wt, tag, t,
-                                  sm + sub, kv);
-    } else {
+        const bool writer = h == kh * at.Gq + at.Gq - 1;
+        if constexpr (T == 1)
+            attn_tile<HD, true, true>(qkv + hd_i * HD, qkv + at.hpw * HD, qkv + (at.hpw + 1) * HD, c, sn, at.Kc, at.Vc,
+                                      kh, writer, at.Lmax, pos, j0, at.scale, wp, wt, tag, t, sm + hd_i, kv);
+        else  // (the combine in this launch is for one block per split, so no tagged copy here)
+            attn_tile2<HD, true>(qkv + hd_i * HD, qkv + at.hpw * HD, qkv + (at.hpw + 1) * HD, c, sn, at.Kc, at.Vc, kh,
+                                 writer, at.Lmax, pos, j0, at.S, tile, at.scale, wp, t, sm + sub, sm + at.hpw + hd_i,
+                                 run + sub, run + at.hpw + hd_i, kv);
+    } else if (tile == 0) {
         attn_tile_empty<HD, true>(wp, wt, tag, t);
     }
-    if (at.out) attn_peer_combine<HD>(at, kh, r, ep);
+    if (T == 1 && at.out) attn_peer_combine<HD>(at, kh, r, ep);
     // this workgroup is past its reads of the launch's tagged words: count it (the epoch of
     // the next launch follows from the count; no result to wait for)
     if (threadIdx.x == 0) (void)__builtin_amdgcn_atomic_inc32(at.done, at.wrap, __ATOMIC_RELAXED, "agent");
@@ -797,9 +814,13 @@ template <int PRO>
 static void launch_qkv_attn(dim3 grid, int nw, size_t lds, hipStream_t s, const GemvArgs& a, const AttnTail& at) {
     const QuantProb& P = a.pro;
     const unsigned shape = (unsigned)nw | ((unsigned)a.ninl << 5) | ((unsigned)a.total_rb << 8);
-    hipLaunchKernelGGL((gemv_ksplit_kernel<1, PRO, false, AttnTail>), grid, dim3((unsigned)(64 * nw)), lds, s, P.x,
-                       P.aux, P.aux2, P.K, P.mode, P.eps, shape, nw_reciprocal(nw), static_cast<const v4u*>(nullptr),
-                       a, at);
+    auto go = [&](auto tail) {
+        hipLaunchKernelGGL((gemv_ksplit_kernel<1, PRO, false, decltype(tail)>), grid, dim3((unsigned)(64 * nw)), lds, s,
+                           P.x, P.aux, P.aux2, P.K, P.mode, P.eps, shape, nw_reciprocal(nw),
+                           static_cast<const v4u*>(nullptr), a, tail);
+    };
+    if (at.T == 2) go(AttnTailLong{at});
+    else go(at);
 }
 
 hipError_t launch_gemv_attn(const GemvArgs& args, const AttnTail& at, int Hkv, int hd, GemvShape shape,
@@ -811,8 +832,8 @@ hipError_t launch_gemv_attn(const GemvArgs& args, const AttnTail& at, int Hkv, i
     const int nw = shape.nw;
     // the shapes the kernel assumes: three inline problems over one RMSNorm-quantised row,
     // one row block per workgroup, a 256-thread tile per query head of a KV group, groups of
-    // whole row blocks; an attention workgroup's live threads (256 hpw) hold its poll's
-    // (hpw + 2) hd values, so hpw >= 2 at hd = 128
+    // whole row blocks; an attention workgroup's live threads (256 hpw T) hold its poll's
+    // (hpw + 2) hd values and fit its 256 Gq
     const bool vec = P.K % 64 == 0 && aligned16(P.x) && aligned16(P.aux) && aligned16(P.aux2);
     const int E = vec ? vec_elements(P.K, 64 * nw) : 0;
     if (a.has_pro != 1 || a.M != 1 || a.out_i32 || a.pair_a || a.ninl != 3 || !shape.ksplit ||
@@ -820,11 +841,12 @@ hipError_t launch_gemv_attn(const GemvArgs& args, const AttnTail& at, int Hkv, i
         at.qrows != at.Gq * Hkv * hd || at.nkv != Hkv * hd || a.inl[0].N != at.qrows || a.inl[1].N != at.nkv ||
         a.inl[2].N != at.nkv || a.inl[1].wg_begin * kRowBlock != at.qrows ||
         a.inl[2].wg_begin * kRowBlock != at.qrows + at.nkv || at.S <= 0 || at.S != attn_splits(at.Lmax) ||
-        at.hpw < 2 || at.Gq % at.hpw || at.natt != (unsigned)(Hkv * at.S * (at.Gq / at.hpw)))
+        at.T != attn_tiles(at.Lmax) || at.hpw < 1 || at.Gq % at.hpw || at.hpw * at.T > at.Gq ||
+        (at.hpw + 2) * hd > 256 * at.hpw * at.T || at.natt != (unsigned)(Hkv * at.S * (at.Gq / at.hpw)))
         return hipErrorInvalidValue;
     const dim3 grid((unsigned)(a.total_rb + (int)at.natt), 1);
     const size_t lds = std::max((size_t)nw * kRowBlock * sizeof(int) + (size_t)P.Kp + sizeof(RowSmem),
-                                (size_t)at.Gq * sizeof(AttnTileLds<128>) + (size_t)(at.Gq + 2) * hd * sizeof(float));
+                                (size_t)at.Gq * (sizeof(AttnTileLds<128>) + sizeof(AttnRun)) + (size_t)(at.Gq + 2) * hd * sizeof(float));
     if (E == 4) launch_qkv_attn<3>(grid, nw, lds, s, a, at);
     else if (E == 8) launch_qkv_attn<4>(grid, nw, lds, s, a, at);
     else launch_qkv_attn<6>(grid, nw, lds, s, a, at);
@@ -836,7 +858,7 @@ hipError_t gemv_attn_capacity(int K, int Kp, int nw, int Gq, int* workgroups) {
     const int E = K % 64 == 0 ? vec_elements(K, 64 * nw) : 0;
     if (E == 0) return hipErrorInvalidValue;
     const size_t lds = std::max((size_t)nw * kRowBlock * sizeof(int) + (size_t)Kp + sizeof(RowSmem),
-                                (size_t)Gq * sizeof(AttnTileLds<128>) + (size_t)(Gq + 2) * 128 * sizeof(float));
+                                (size_t)Gq * (sizeof(AttnTileLds<128>) + sizeof(AttnRun)) + (size_t)(Gq + 2) * 128 * sizeof(float));
     const void* k = E == 4   ? reinterpret_cast<const void*>(&gemv_ksplit_kernel<1, 3, false, AttnTail>)
                     : E == 8 ? reinterpret_cast<const void*>(&gemv_ksplit_kernel<1, 4, false, AttnTail>)
                              : reinterpret_cast<const void*>(&gemv_ksplit_kernel<1, 6, false, AttnTail>);

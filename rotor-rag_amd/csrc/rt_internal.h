@@ -157,7 +157,7 @@ struct GemvArgs {
 // GEMV workgroups also store every output y of the q, k and v problems (concatenated, row
 // n of the launch at index n) as tagged[n] = epoch << 32 | bits(y), a 64-bit
 // device-coherent store; the natt = Hkv * S * Gq / hpw attention workgroups (hpw query heads
-// of a KV group and one key block each) poll their heads' q and the group's k and v words
+// of a KV group and one split of the keys each) poll their heads' q and the group's k and v words
 // until every one carries the epoch (bounded; err counts the waits that gave up,
 // never expected).  Each attention workgroup adds one to *done when it has finished, without
 // waiting for the result, and a launch's epoch is *done / natt + 1, read by every workgroup
@@ -181,10 +181,10 @@ struct AttnTail {
     const int* pos;
     float* work;                 // partials [H][S][hd + 2]
     int Gq, Lmax, S, nkv;        // nkv = Hkv hd: where k starts after q (H hd), v after k
-    int hpw;                     // query heads per attention workgroup (Gq / hpw of them per key block)
+    int hpw;                     // query heads per attention workgroup (Gq / hpw of them per split)
     int qrows;                   // H hd
     float scale;
-    // rt_plan_attention_combine (out != nullptr, S <= kAttnSMax): the attention workgroups
+    // rt_plan_attention_combine (out != nullptr, Lmax <= 64 kAttnSMax): the attention workgroups
     // also store their partials as tagged words ptag [H][S][hd + 2] (epoch << 32 | bits),
     // and the S Gq / hpw workgroups of KV group kh share its combine: each polls the partials
     // of its share of the group's outputs, combines them into out [H hd] and writes per 32 outputs
@@ -192,6 +192,7 @@ struct AttnTail {
     float* out;
     double* ssq;
     unsigned long long* ptag;
+    int T;  // tiles per query head (attn_tiles(Lmax))
 };
 
 struct GemvShape {
@@ -382,8 +383,14 @@ hipError_t launch_rope_append(float* q, float* k, const float* v, float* Kc, flo
                               int H, int Hkv, int hd, int Lmax, const int* pos, hipStream_t s);
 hipError_t launch_attention(const float* q, const float* Kc, const float* Vc, float* out, int M, int H, int Hkv,
                             int hd, int Lmax, const int* pos, float scale, hipStream_t s);
-// decode attention split over blocks of 64 keys: partials [H][S][hd + 2], S = attn_splits(Lmax)
-inline int attn_splits(int Lmax) { return (Lmax + 63) / 64; }
+// Decode attention: the keys go in blocks of 64, dealt to S = attn_splits(Lmax) splits per
+// query head (one block each up to Lmax 640, then every S-th block), partials [H][S][hd + 2].
+// Past one block per split, attn_tiles = 2 tiles share a split's blocks.  S stops at the
+// kAttnSMax partials that an o_proj prologue holds in registers (rt_attn_decode.h).
+constexpr int kAttnBlock = 64, kAttnSMax = 10;
+inline int attn_blocks(int Lmax) { return (Lmax + kAttnBlock - 1) / kAttnBlock; }
+inline int attn_splits(int Lmax) { return attn_blocks(Lmax) < kAttnSMax ? attn_blocks(Lmax) : kAttnSMax; }
+inline int attn_tiles(int Lmax) { return attn_blocks(Lmax) > kAttnSMax ? 2 : 1; }
 // rope != nullptr: q/knew/vnew are the raw projection outputs of the token at *pos; the
 // kernel applies RoPE, appends knew (rotated) and vnew to the caches and uses them for that
 // key.  rope == nullptr: q is rotated and the caches already hold the token.

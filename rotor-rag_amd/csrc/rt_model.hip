@@ -300,35 +300,48 @@ __global__ void __launch_bounds__(256) attn_prefill_mfma_kernel(const float* __r
     }
 }
 
-// Decode attention, split over the keys: workgroup (h, s) is the tile of query head h and
-// key block s (rt_attn_decode.h), writing its partial to work[h][s][0..HD+2).
-template <int HD, bool ROPE>
-__global__ void __launch_bounds__(256) attn_partial_kernel(const float* __restrict__ q, const float* __restrict__ knew,
+// Decode attention, split over the keys: workgroup (h, s) holds the T tiles of query head h
+// and split s (rt_attn_decode.h), writing the partial to work[h][s][0..HD+2).
+template <int HD, int T, bool ROPE>
+__global__ void __launch_bounds__(256 * T) attn_partial_kernel(const float* __restrict__ q, const float* __restrict__ knew,
                                                            const float* __restrict__ vnew, float* __restrict__ Kc,
                                                            float* __restrict__ Vc, const float* __restrict__ rope,
                                                            int H, int Hkv, int Lmax, const int* __restrict__ pos_p,
                                                            float scale, float* __restrict__ work) {
-    __shared__ AttnTileLds<HD> sm;
+    __shared__ AttnTileLds<HD> sm[T];
+    __shared__ AttnRun run[T];
     // Workgroup (h, s) from an XCD-ordered index whose fastest part is the query head within
     // its KV group: the G heads that read one key block run on one XCD and share its L2
     // (decode 1.235 -> 1.218 ms/token against one workgroup per (blockIdx.x, blockIdx.y))
     const int S = gridDim.y, Gq = H / Hkv;
     const int w = xcd_order((int)(blockIdx.x + gridDim.x * blockIdx.y), (int)(gridDim.x * gridDim.y));
-    const int kh = w / (Gq * S), s = (w / Gq) % S, h = kh * Gq + w % Gq, t = threadIdx.x;
-    const int j0 = s * kAttnBlock;
+    const int kh = w / (Gq * S), s = (w / Gq) % S, h = kh * Gq + w % Gq;
+    const int tile = T == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8)), t = threadIdx.x & 255;
+    const int js = s * kAttnBlock;
     AttnKV<HD> kv;
-    attn_kv_load<HD>(Kc, Vc, kh, j0, Lmax, t, kv);
+    if constexpr (T == 1) {
+        attn_kv_load<HD>(Kc, Vc, kh, js, Lmax, t, kv);
+    } else {
+        attn_k_load<HD>(Kc, kh, js + tile * S * kAttnBlock, Lmax, t, kv);
+        attn_v_load<HD>(Vc, kh, js + tile * S * kAttnBlock, Lmax, t, kv);
+    }
     const int pos = *pos_p;
     float* wp = work + ((size_t)h * S + s) * (HD + 2);
-    if (pos < j0) {
-        attn_tile_empty<HD>(wp, nullptr, 0ull, t);
+    if (pos < js) {
+        if (tile == 0) attn_tile_empty<HD>(wp, nullptr, 0ull, t);
         return;
     }
     float c = 0.0f, sn = 0.0f;
     if (ROPE) attn_rope_load<HD>(rope, pos, t, c, sn);
-    attn_tile<HD, ROPE>(q + (size_t)h * HD, ROPE ? knew + (size_t)kh * HD : nullptr,
-                        ROPE ? vnew + (size_t)kh * HD : nullptr, c, sn, Kc, Vc, kh, h % Gq == 0, Lmax, pos, j0, scale,
-                        wp, nullptr, 0ull, t, (AttnLdsPtr<HD>)&sm, kv);
+    const float *qh = q + (size_t)h * HD, *kn = ROPE ? knew + (size_t)kh * HD : nullptr,
+                *vn = ROPE ? vnew + (size_t)kh * HD : nullptr;
+    if constexpr (T == 1)
+        attn_tile<HD, ROPE>(qh, kn, vn, c, sn, Kc, Vc, kh, h % Gq == 0, Lmax, pos, js, scale, wp, nullptr, 0ull, t,
+                            (AttnLdsPtr<HD>)&sm[0], kv);
+    else
+        attn_tile2<HD, ROPE>(qh, kn, vn, c, sn, Kc, Vc, kh, h % Gq == 0, Lmax, pos, js, S, tile, scale, wp, t,
+                             (AttnLdsPtr<HD>)&sm[tile], (AttnLdsPtr<HD>)&sm[1], (lds_run*)&run[tile], (lds_run*)&run[1],
+                             kv);
 }
 
 // out[h*hd + d] from the S partials of head h (one thread per output element)
@@ -558,14 +571,21 @@ hipError_t launch_attention(const float* q, const float* Kc, const float* Vc, fl
 hipError_t launch_attn_partial(const float* q, const float* knew, const float* vnew, float* Kc, float* Vc,
                                const float* rope, int H, int Hkv, int hd, int Lmax, const int* pos, float scale,
                                float* work, hipStream_t s) {
-    const dim3 grid((unsigned)H, (unsigned)attn_splits(Lmax));
-    const bool r = rope != nullptr;
-    switch (hd * 2 + (r ? 1 : 0)) {
-        case 128: hipLaunchKernelGGL((attn_partial_kernel<64, false>), grid, dim3(256), 0, s, q, knew, vnew, Kc, Vc, rope, H, Hkv, Lmax, pos, scale, work); break;
-        case 129: hipLaunchKernelGGL((attn_partial_kernel<64, true>), grid, dim3(256), 0, s, q, knew, vnew, Kc, Vc, rope, H, Hkv, Lmax, pos, scale, work); break;
-        case 256: hipLaunchKernelGGL((attn_partial_kernel<128, false>), grid, dim3(256), 0, s, q, knew, vnew, Kc, Vc, rope, H, Hkv, Lmax, pos, scale, work); break;
-        case 257: hipLaunchKernelGGL((attn_partial_kernel<128, true>), grid, dim3(256), 0, s, q, knew, vnew, Kc, Vc, rope, H, Hkv, Lmax, pos, scale, work); break;
-        default: return hipErrorInvalidValue;
+    const int T = attn_tiles(Lmax);
+    const dim3 grid((unsigned)H, (unsigned)attn_splits(Lmax)), block(256u * (unsigned)T);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, block, 0, s, q, knew, vnew, Kc, Vc, rope, H, Hkv, Lmax, pos, scale, work);
+    };
+    if (hd != 64 && hd != 128) return hipErrorInvalidValue;
+    switch ((hd == 128 ? 4 : 0) + (T == 2 ? 2 : 0) + (rope ? 1 : 0)) {
+        case 0: go(attn_partial_kernel<64, 1, false>); break;
+        case 1: go(attn_partial_kernel<64, 1, true>); break;
+        case 2: go(attn_partial_kernel<64, 2, false>); break;
+        case 3: go(attn_partial_kernel<64, 2, true>); break;
+        case 4: go(attn_partial_kernel<128, 1, false>); break;
+        case 5: go(attn_partial_kernel<128, 1, true>); break;
+        case 6: go(attn_partial_kernel<128, 2, false>); break;
+        default: go(attn_partial_kernel<128, 2, true>); break;
     }
     return hipGetLastError();
 }

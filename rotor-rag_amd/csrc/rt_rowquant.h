@@ -468,7 +468,6 @@ __device__ __forceinline__ float row_finishE(const QuantProb& P, RowRegsE<E>& r,
 // 16-byte load of its four values and one 8-byte load of the block's (max, sum) -- and its
 // four norm weights; attn_finish1 combines them in the operation order of
 // attn_combine_element, then RMSNorm and quantisation as row_finish4.
-constexpr int kAttnSMax = 10;  // Lmax <= 640 (longer contexts take the general path)
 struct AttnRegs {
     float p[kAttnSMax][4], m[kAttnSMax], z[kAttnSMax], w[4];
     bool live;  // wave-uniform: some lane of this wave owns elements

@@ -397,6 +397,26 @@ def test_qkv_plan_with_attention_equals_separate_launches(hip, H, Hkv, pos0, Lma
     assert torch.equal(q, qr) and torch.equal(kcf, kc0) and not ws.any()
 
 
+# past 640 positions a split holds several blocks of 64 keys, dealt to two tiles per head: the
+# position in the first round's tile 0 and tile 1, at both ends of a block, in a later round, at
+# the end of Lmax; splits with an empty tile 1; H / Hkv = 4, 2, 3 and 1, head sizes 128 and 64
+LONG_SPLITS = [(639, 20, 5, 128, 704), (640, 20, 5, 128, 704), (703, 20, 5, 128, 704), (30, 20, 5, 128, 2048),
+               (1279, 20, 5, 128, 2048), (1280, 20, 5, 128, 2048), (1537, 20, 5, 128, 2048), (2047, 20, 5, 128, 2048),
+               (1000, 4, 4, 64, 1001), (3999, 8, 2, 64, 4100)]
+
+
+@pytest.mark.parametrize("pos0,H,Hkv,hd,Lmax", LONG_SPLITS)
+def test_attention_decode_split_long(hip, pos0, H, Hkv, hd, Lmax):
+    test_attention_decode_split(hip, pos0, H, Hkv, hd, Lmax)
+    test_rope_attention_decode_equals_separate_launches(hip, pos0, H, Hkv, hd, Lmax)
+
+
+@pytest.mark.parametrize("H,Hkv,pos0,Lmax", [(20, 5, 640, 704), (20, 5, 1279, 2048), (20, 5, 1300, 4096),
+                                             (64, 32, 1000, 1024), (54, 18, 1343, 1344)])
+def test_qkv_plan_with_attention_long(hip, H, Hkv, pos0, Lmax):
+    test_qkv_plan_with_attention_equals_separate_launches(hip, H, Hkv, pos0, Lmax)
+
+
 def test_attach_attention_rejects_other_plans(hip):
     """Plans the attention cannot join (one problem; 2 query heads per KV head) are refused
     with the library's message, and stay usable."""
