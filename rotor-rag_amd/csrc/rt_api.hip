@@ -147,7 +147,7 @@ struct rt_weights {
 
 struct rt_plan {
     int device = 0;
-    int G = 0, M = 0, Mpad = 0, mt = 1, total_rb = 0, U = 0;
+    int G = 0, M = 0, Mpad = 0, total_rb = 0, U = 0;
     GemvShape shape{};
     GemvProb* dev_probs = nullptr;   // [G]
     int* dev_rb2p = nullptr;         // [total_rb]
@@ -156,13 +156,15 @@ struct rt_plan {
     std::vector<GemvProb> probs;
     std::vector<QuantProb> quant;
     std::vector<GemmArgs> gemms;     // M > kGemvMaxM: one MFMA GEMM launch per problem
-    GemmArgs* dev_gemms = nullptr;   // M > 8: the problems of one grouped launch [G]
+    GemmArgs* dev_gemms = nullptr;   // M > 1: the problems of one grouped launch [G]
     int* dev_tile2p = nullptr;       // M > 64: problem of every tile of that launch
     int gemm_cfg = 0, gemm_tiles = 0;  // M > 64: tile shape, tiles over all problems
     bool pair_gemm = false;            // rt_plan_create_act_gate_up: tiles whose waves pair columns
-    int gemm_units = 0;              // 8 < M <= 64: workgroups of the split-K launch (parts x row blocks)
-    int* dev_unit2d = nullptr;       // 8 < M <= 64: descriptor of every unit
-    std::vector<int> gemm_bnd;       // M > 8: first unit (tile) of descriptors 1.. (launch arguments)
+    bool skinny = false;             // ... or, few tokens: of gemm_skinny_kernel, one unit per row block
+    int gemm_minC = 0, gemm_maxC = 0;  // its fewest and most chunks of a problem
+    int gemm_units = 0;              // 1 < M <= 64: workgroups of the split-K launch (parts x row blocks)
+    int* dev_unit2d = nullptr;       // 1 < M <= 64: descriptor of every unit
+    std::vector<int> gemm_bnd;       // M > 1: first unit (tile) of descriptors 1.. (launch arguments)
     int* gemm_cnt = nullptr;         // split problems: arrivals per row block (zero between launches)
     int* gemm_ws = nullptr;          // split problems: int32 partial tiles
     std::vector<const rt_act*> acts; // plans over caller-quantised activations
@@ -192,14 +194,13 @@ struct rt_act {
     int device = 0;
     int Mcap = 0, K = 0, Kp = 0, Mpad_cap = 0;
     int M = 0;      // tokens held (set by the last quantise call)
-    int Mpad = 0;   // rows valid for the GEMV/GEMM of M tokens (zero-filled past M)
     int8_t* qx = nullptr;
     float* sx = nullptr;
     void* mem = nullptr;
 };
 
-// Rows the matrix kernels read for M tokens: GEMV tokens per workgroup, or GEMM tile rows.
-static int act_rows(int M) { return M > kGemvMaxM ? round_up(M, gemm_bm(M)) : round_up(M, gemv_mt(M)); }
+// Rows the matrix kernels read for M tokens: one (GEMV), or GEMM tile rows.
+static int act_rows(int M) { return M > kGemvMaxM ? round_up(M, gemm_bm(M)) : M; }
 
 extern "C" {
 
@@ -373,7 +374,6 @@ static int stage_activations(rt_ctx* ctx, const float* x, const int8_t* q_in, in
     a.dev = nullptr;
     a.U = 1;
     a.M = M;
-    a.Mpad = Mpad;
     a.p = QuantProb{x, q_in, *qx, *sx, q_nat, K, Kp, q_in ? kPermute : kQuant, nullptr, 0.0f, nullptr, nullptr, 0, 0,
                     blocked};
     RT_HIP(launch_quant(a, ctx->stream, quant_rows_ok(a.p) ? K : 0));
@@ -426,7 +426,6 @@ static int launch_matrix(rt_ctx* ctx, const rt_weights* w, const int8_t* qx, con
         RT_HIP(launch_gemm(a, ctx->stream));
         return RT_OK;
     }
-    const int mt = gemv_mt(M);
     GemvArgs a{};
     a.dev = nullptr;
     a.rb2p = nullptr;
@@ -435,8 +434,8 @@ static int launch_matrix(rt_ctx* ctx, const rt_weights* w, const int8_t* qx, con
     a.out_i32 = out_i32 ? 1 : 0;
     a.total_rb = w->Np / kRowBlock;
     a.p = GemvProb{w->tiles, qx, sx, row_scale, out, w->scale, w->N, w->C, w->N, 0, res};
-    const GemvShape shape = gemv_shape(a.total_rb, (M + mt - 1) / mt, w->C);
-    RT_HIP(launch_gemv(a, mt, shape, ctx->stream));
+    const GemvShape shape = gemv_shape(a.total_rb, w->C);
+    RT_HIP(launch_gemv(a, shape, ctx->stream));
     return RT_OK;
 }
 
@@ -454,8 +453,8 @@ static int linear_m1_prologue(rt_ctx* ctx, const rt_weights* w, const float* x, 
     const int nb = a.total_rb;
     GemvShape shape;
     *launched = false;
-    if (!prologue_launch(gemv_shape(a.total_rb, 1, w->C), 1, &nb, 1, w->Kp, src, &a, &shape)) return RT_OK;
-    RT_HIP(launch_gemv(a, 1, shape, ctx->stream));
+    if (!prologue_launch(gemv_shape(a.total_rb, w->C), 1, &nb, 1, w->Kp, src, &a, &shape)) return RT_OK;
+    RT_HIP(launch_gemv(a, shape, ctx->stream));
     *launched = true;
     return RT_OK;
 }
@@ -505,8 +504,8 @@ int rt_linear_f32_noalloc(rt_ctx* ctx, const rt_weights* w, const float* x, int 
         if (rc || launched) return rc;
     }
     // the activations of the GEMV / GEMM tile rows: int8 [Mpad][Kp], then fp32 scales [Mpad];
-    // the quantiser writes every byte of both (padding rows as zeros), so what an earlier call
-    // left in the buffer is never read
+    // the quantiser writes every byte of the tokens' rows, and no output depends on the padding
+    // rows, so what an earlier call left in the buffer does not matter
     const int Mpad = act_rows(M);
     const size_t qbytes = (size_t)Mpad * w->Kp, need = qbytes + (size_t)Mpad * sizeof(float);
     if (need > RT_NOALLOC_SCRATCH_BYTES)
@@ -518,7 +517,6 @@ int rt_linear_f32_noalloc(rt_ctx* ctx, const rt_weights* w, const float* x, int 
     QuantArgs a{};
     a.U = 1;
     a.M = M;
-    a.Mpad = Mpad;
     a.p = QuantProb{x, nullptr, qx, sx, nullptr, w->K, w->Kp, kQuant, nullptr, 0.0f, nullptr, nullptr, 0, 0,
                     qx_blocked(M)};
     RT_HIP(launch_quant(a, ctx->stream, quant_rows_ok(a.p) ? w->K : 0));
@@ -551,8 +549,8 @@ int rt_plan_free(rt_plan* plan) {
     return RT_OK;
 }
 
-// M > 8: one launch serves all problems.  M <= 64: the split-K kernel, one unit per row
-// block and part (upload_splitk_group).  M > 64: the tile kernel, the tiles of problem g
+// M > 1: one launch serves all problems.  M <= 64: the split-K (or skinny) kernel, one unit per
+// row block and part (upload_splitk_group).  M > 64: the tile kernel, the tiles of problem g
 // after those of problems 0..g-1, with a tile -> problem table.
 // Split-K parts of a problem with C chunks when the group's shortest problem has Cmin: a
 // problem several times longer than the shortest is cut into about C / Cmin parts (at most
@@ -573,8 +571,19 @@ static hipError_t upload_splitk_group(rt_plan* p) {
     std::vector<int> unit2d;
     size_t cnt_n = 0, ws_n = 0;
     std::vector<std::pair<size_t, size_t>> offs(g.size());  // counter, workspace offsets of split problems
+    // few tokens: the skinny kernel where its rule allows, no problem cut into parts
+    bool split = false;
+    long long rbs = 0;
+    for (const GemmArgs& a : g) {
+        split = split || splitk_parts(a.C, Cmin) > 1;
+        rbs += a.Np / kRowBlock;
+        p->gemm_maxC = std::max(p->gemm_maxC, a.C);
+    }
+    p->gemm_minC = Cmin;
+    p->skinny = skinny_ok(p->M, (int)std::min(rbs, 1ll << 30), split);
+    auto parts_of = [&](int C) { return p->skinny ? 1 : splitk_parts(C, Cmin); };
     for (size_t i = 0; i < g.size(); ++i) {
-        const int parts = splitk_parts(g[i].C, Cmin), nrb = g[i].Np / kRowBlock;
+        const int parts = parts_of(g[i].C), nrb = g[i].Np / kRowBlock;
         offs[i] = {cnt_n, ws_n};
         if (parts > 1) {
             cnt_n += (size_t)nrb;
@@ -588,14 +597,14 @@ static hipError_t upload_splitk_group(rt_plan* p) {
         if (e == hipSuccess) e = hipMalloc(&p->gemm_ws, ws_n * sizeof(int));
         if (e != hipSuccess) return e;
     }
-    // the split problems' workgroups first in the grid: they walk their part of K and then
-    // hand over, so starting them first shortens the launch
+    // the split (or longest, skinny) problems' workgroups first in the grid: they walk their part
+    // of K and then hand over, so starting them first shortens the launch
     std::vector<size_t> order;
     for (int pass = 0; pass < 2; ++pass)
         for (size_t i = 0; i < g.size(); ++i)
             if ((splitk_parts(g[i].C, Cmin) > 1) == (pass == 0)) order.push_back(i);
     for (size_t i : order) {
-        const int parts = splitk_parts(g[i].C, Cmin), nrb = g[i].Np / kRowBlock;
+        const int parts = parts_of(g[i].C), nrb = g[i].Np / kRowBlock;
         for (int kp = 0; kp < parts; ++kp) {
             GemmArgs a = g[i];
             a.wg_begin = (int)unit2d.size();
@@ -622,7 +631,7 @@ static hipError_t upload_splitk_group(rt_plan* p) {
 
 static hipError_t upload_gemm_group(rt_plan* p) {
     if (p->gemms.empty()) return hipSuccess;
-    if (gemm_bm(p->M) == 64) return upload_splitk_group(p);
+    if (p->M <= 64) return upload_splitk_group(p);
     std::vector<GemmArgs> g = p->gemms;
     std::vector<int> tile2p;
     std::vector<int> Ns(g.size()), Cs(g.size());
@@ -672,8 +681,7 @@ int rt_plan_create(rt_ctx* ctx, int G, const rt_weights* const* w, const float* 
     p->device = ctx->device;
     p->G = G;
     p->M = M;
-    p->mt = gemv_mt(M);
-    p->Mpad = M > kGemvMaxM ? round_up(M, gemm_bm(M)) : round_up(M, p->mt);
+    p->Mpad = act_rows(M);
     // distinct inputs (same pointer => same quantisation; their K must agree)
     std::unordered_map<const float*, int> uid;
     std::vector<int> which(G);
@@ -736,7 +744,7 @@ int rt_plan_create(rt_ctx* ctx, int G, const rt_weights* const* w, const float* 
         if (w[g]->C < minC) minC = w[g]->C;
     }
     p->total_rb = wg;
-    p->shape = gemv_shape(wg, (M + p->mt - 1) / p->mt, minC);
+    p->shape = gemv_shape(wg, minC);
     if (M == 1) {
         std::vector<int> nb(G);
         int kp_max = 0;
@@ -786,7 +794,7 @@ int rt_plan_describe(const rt_plan* plan, int* kind, int* tile_m, int* tile_n, i
         u = plan->gemm_tiles;
     } else if (plan->dev_gemms) {
         k = RT_LAUNCH_SPLITK;
-        tm = 64;
+        tm = plan->skinny ? (plan->M <= 16 ? 16 : 32) : 64;
         tn = kRowBlock;
         u = plan->gemm_units;
     } else if (plan->fused || plan->run_pro) {
@@ -797,10 +805,9 @@ int rt_plan_describe(const rt_plan* plan, int* kind, int* tile_m, int* tile_n, i
         u = sh.ksplit ? plan->total_rb : plan->total_rb / sh.nw;
     } else {
         k = RT_LAUNCH_GEMV;
-        tm = plan->mt;
+        tm = 1;
         tn = plan->shape.ksplit ? kRowBlock : kRowBlock * plan->shape.nw;
-        u = (plan->shape.ksplit ? plan->total_rb : (plan->total_rb + plan->shape.nw - 1) / plan->shape.nw) *
-            ((plan->M + plan->mt - 1) / plan->mt);
+        u = plan->shape.ksplit ? plan->total_rb : (plan->total_rb + plan->shape.nw - 1) / plan->shape.nw;
     }
     if (kind) *kind = k;
     if (tile_m) *tile_m = tm;
@@ -825,7 +832,6 @@ int rt_plan_quantize(rt_ctx* ctx, const rt_plan* plan) {
     q.dev = plan->dev_quant;
     q.U = plan->U;
     q.M = plan->M;
-    q.Mpad = plan->Mpad;
     RT_HIP(launch_quant(q, ctx->stream, plan->quant_maxK));
     return RT_OK;
 }
@@ -843,7 +849,7 @@ int rt_plan_run(rt_ctx* ctx, const rt_plan* plan) {
         a.total_rb = plan->total_rb;
         a.has_pro = plan->run_pro;
         a.pro = plan->pro;
-        RT_HIP(launch_gemv(a, 1, plan->run_shape, ctx->stream));
+        RT_HIP(launch_gemv(a, plan->run_shape, ctx->stream));
         return RT_OK;
     }
     int rc = rt_plan_quantize(ctx, plan);
@@ -880,6 +886,12 @@ int rt_plan_gemv(rt_ctx* ctx, const rt_plan* plan) {
                                  plan->gemm_tiles, plan->gemm_cfg, ctx->stream));
         return RT_OK;
     }
+    if (plan->dev_gemms && plan->skinny) {
+        RT_HIP(launch_gemm_skinny(plan->dev_gemms, plan->dev_unit2d, plan->gemm_bnd.data(), group_bounds(plan), plan->M,
+                                  plan->gemm_units, plan->gemm_minC, plan->gemm_maxC,
+                                  ctx->stream));
+        return RT_OK;
+    }
     if (plan->dev_gemms) {
         RT_HIP(launch_gemm_group(plan->dev_gemms, plan->dev_unit2d, plan->gemm_bnd.data(), group_bounds(plan),
                                  plan->gemm_units, ctx->stream));
@@ -888,7 +900,7 @@ int rt_plan_gemv(rt_ctx* ctx, const rt_plan* plan) {
     if (plan->att_on)
         RT_HIP(launch_gemv_attn(a, plan->att, plan->att_Hkv, plan->att_hd, plan->shape, ctx->stream));
     else
-        RT_HIP(launch_gemv(a, plan->mt, plan->shape, ctx->stream));
+        RT_HIP(launch_gemv(a, plan->shape, ctx->stream));
     return RT_OK;
 }
 
@@ -937,12 +949,10 @@ static int act_fill(rt_ctx* ctx, rt_act* act, int M, int mode, const float* x, c
     q.dev = nullptr;
     q.U = 1;
     q.M = M;
-    q.Mpad = act_rows(M);
     q.p = QuantProb{x, nullptr, act->qx, act->sx, nullptr, act->K, act->Kp, mode, aux, eps, v_out, aux2, 0, 0,
                     qx_blocked(M)};
     RT_HIP(launch_quant(q, ctx->stream, quant_rows_ok(q.p) ? act->K : 0));
     act->M = M;
-    act->Mpad = q.Mpad;
     return RT_OK;
 }
 
@@ -1005,7 +1015,6 @@ int rt_plan_create_act(rt_ctx* ctx, int G, const rt_weights* const* w, const rt_
     p->device = ctx->device;
     p->G = G;
     p->M = M;
-    p->mt = gemv_mt(M);
     p->Mpad = act_rows(M);
     p->U = 0;  // inputs are quantised by the caller
     p->acts.assign(act, act + G);
@@ -1021,7 +1030,7 @@ int rt_plan_create_act(rt_ctx* ctx, int G, const rt_weights* const* w, const rt_
                                         w[g]->N, w[g]->Np, w[g]->C, w[g]->N, 0});
     }
     p->total_rb = wg;
-    p->shape = gemv_shape(wg, (M + p->mt - 1) / p->mt, minC);
+    p->shape = gemv_shape(wg, minC);
     std::vector<int> rb2p(wg);
     for (int g = 0; g < G; ++g)
         for (int r = 0; r < w[g]->Np / kRowBlock; ++r) rb2p[p->probs[g].wg_begin + r] = g;
@@ -1055,7 +1064,6 @@ int rt_plan_create_act_gate_up(rt_ctx* ctx, const rt_weights* w_gu, float s_gate
     p->device = ctx->device;
     p->G = 1;
     p->M = M;
-    p->mt = gemv_mt(M);
     p->Mpad = act_rows(M);
     p->U = 0;  // the input is quantised by the caller
     p->acts.assign(1, act);
@@ -1231,7 +1239,6 @@ int rt_plan_create_fused(rt_ctx* ctx, int G, const rt_weights* const* w, const r
     p->device = ctx->device;
     p->G = G;
     p->M = 1;
-    p->mt = 1;
     p->Mpad = 1;
     p->U = 0;
     p->fused = true;
@@ -1294,7 +1301,6 @@ int rt_plan_create_gate_up(rt_ctx* ctx, const rt_weights* w_gu, float s_gate, fl
     p->device = ctx->device;
     p->G = 1;
     p->M = 1;
-    p->mt = 1;
     p->Mpad = 1;
     p->U = 0;
     p->fused = true;

@@ -1,7 +1,7 @@
 // Prefill / batched ternary GEMM on the int8 matrix cores (gfx950 MFMA):
 // C[M,N] = A[M,K] x W[N,K]^T with A the per-token quantised activations (qx layout)
 // and W the rotor weight tiles, int32 accumulation, fp32 rescale epilogue.
-// Replaces, for M > 8 tokens, the reference's per-token loop
+// Replaces, for M > 1 tokens, the reference's per-token loop
 // (src/rotor/transformer.py:134-143) and its CPU sgemm (src/rotor/transformer.py:150).
 //
 // Workgroup: 4 waves (WAVES_M x WAVES_N), tile BM x BN, K step 64 (one weight chunk) =
@@ -193,7 +193,7 @@ __device__ __forceinline__ void store_tile_pair(const v16i (&acc)[FI][FJ], const
 }
 
 // One problem, or a group of them (dev != nullptr): unit b (a row block of the split-K
-// kernel, a tile of the tile kernel) serves problem rb2p[b], whose units start at its
+// and skinny kernels, a tile of the tile kernel) serves problem rb2p[b], whose units start at its
 // wg_begin.
 struct GemmGroupArgs {
     const GemmArgs* dev;
@@ -666,6 +666,131 @@ __global__ void __launch_bounds__(kRegThreads) gemm_region_kernel(GemmGroupArgs 
     else store(reinterpret_cast<const v4i(&)[HB][FJ]>(acc[0]));
 }
 
+// ---- a few tokens: weights straight into registers -------------------------------------
+// 16 MB rows (MB = 1: up to 16 tokens) by one 64-column row block per workgroup; its waves
+// split the K range in quads of 4 chunks and stream their weights and activations from
+// memory into registers, two quads ahead, with no LDS and no barrier before the final sum:
+// what bounds these launches is the latency from the start to the weights, then the weights.
+// With v_mfma_i32_16x16x64_i8 and K assigned to lanes so that every load is 16 bytes a lane:
+// lane l owns column l % 16 of each 16-column block and chunk 4 q + l / 16 of quad q, whose 16
+// bytes of code are the B operands of the quad's four MFMA steps (one dword each); the A
+// operand of step i is the 16-byte group i of the same chunk of row l % 16.  Both operands
+// use that assignment of k, so the int32 sums are exact.  B holds the device code g = w + 1
+// itself, four fields masked out of a dword (7 VALU operations; expanding to w takes 11), and
+// one more MFMA a step against ones gives sum x, subtracted at the end.  Chunks past C read as
+// zeros (both buffers end at chunk C): x = 0 there.
+// The nw partial tiles are summed in LDS (rows padded to 68 words: the four lane groups store
+// to different banks) and the workgroup applies the epilogue.
+// Measured (launch alone, 20 layers in rotation; before: the VALU GEMV, eight tokens a
+// workgroup, M <= 8, and the split-K kernel below): the seven projections of a 2560 / 6912
+// layer at M = 5 28.2 -> 9.9 us; q/k/v at M = 5 / 16 12.1 / 7.2 -> 4.4 / 4.8; down 17.1 / 12.5
+// -> 6.0 / 6.3; 64 matrices of 6912 x 2560 (283 MB) at M = 2 / 3 51.1 / 63.4 -> 48.3 / 49.4.
+constexpr int kSkinnyLd = 68;
+template <int MB, bool NT>
+__global__ void __launch_bounds__(1024 / MB) gemm_skinny_kernel(GemmGroupArgs ga, int xcd) {
+    extern __shared__ __attribute__((aligned(16))) v4u lds[];
+    const int t = threadIdx.x, lane = t & 63, c16 = lane & 15, h4 = lane >> 4;
+    const int nw = (int)(blockDim.x >> 6), wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int unit = xcd ? xcd_order((int)blockIdx.x, (int)gridDim.x) : (int)blockIdx.x;
+    const GemmArgs a = find_gemm(ga, unit);
+    const int C = a.C, rb = unit - a.wg_begin, n0 = rb * kRowBlock;
+    const int Q = (C + 3) >> 2;
+    const int q0 = __builtin_amdgcn_readfirstlane((wave * Q) / nw);
+    const int q1 = __builtin_amdgcn_readfirstlane(((wave + 1) * Q) / nw);
+    const __amdgpu_buffer_rsrc_t wr =
+        __builtin_amdgcn_make_buffer_rsrc((void*)(a.w + (size_t)rb * C * kRowBlock), 0, C * 1024, kBufDword3);
+    __amdgpu_buffer_rsrc_t ar[MB];
+#pragma unroll
+    for (int b = 0; b < MB; ++b)
+        ar[b] = __builtin_amdgcn_make_buffer_rsrc((void*)(a.qx + (size_t)b * C * 1024), 0, C * 1024, kBufDword3);
+    // rows past the tokens read as zeros too, from past the buffer: no traffic for them (for 2
+    // tokens, each XCD would otherwise read 14 rows of padding of every problem)
+    const int off = h4 * 1024 + c16 * 16;
+    int aoff[MB];
+#pragma unroll
+    for (int b = 0; b < MB; ++b) aoff[b] = 16 * b + c16 < a.M ? off : (int)0x80000000;
+    struct Quad {
+        v4u w[4];       // column block j
+        v4i x[MB][4];   // row block b, step i
+    };
+    auto load = [&](Quad& z, int q) {
+        const int o = off + q * 4096;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            z.w[j] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(wr, o + j * 256, 0, NT ? 2 : 0));
+#pragma unroll
+        for (int b = 0; b < MB; ++b)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                z.x[b][i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(ar[b], aoff[b] + q * 4096 + i * 256, 0, 0));
+    };
+    v4i acc[MB][4];
+#pragma unroll
+    for (int b = 0; b < MB; ++b)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[b][j] = v4i{};
+    v4i sum[MB];  // sum x over the wave's k, every column alike
+#pragma unroll
+    for (int b = 0; b < MB; ++b) sum[b] = v4i{};
+    const v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
+    auto math = [&](const Quad& z) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+#pragma unroll
+            for (int b = 0; b < MB; ++b)
+                sum[b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(z.x[b][i], ones, sum[b], 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                constexpr unsigned kM = 0x03030303u;
+                const unsigned u = z.w[j][i];
+                const v4i g = {(int)(u & kM), (int)((u >> 2) & kM), (int)((u >> 4) & kM), (int)((u >> 6) & kM)};
+#pragma unroll
+                for (int b = 0; b < MB; ++b)
+                    acc[b][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(z.x[b][i], g, acc[b][j], 0, 0, 0);
+            }
+        }
+    };
+    Quad z0, z1;
+    if (q0 < q1) load(z0, q0);
+    if (q0 + 1 < q1) load(z1, q0 + 1);
+    for (int q = q0; q < q1; q += 2) {
+        math(z0);
+        if (q + 2 < q1) load(z0, q + 2);
+        if (q + 1 < q1) math(z1);
+        if (q + 3 < q1) load(z1, q + 3);
+    }
+    int* const part = reinterpret_cast<int*>(lds) + wave * (16 * MB) * kSkinnyLd;
+#pragma unroll
+    for (int b = 0; b < MB; ++b)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) part[(16 * b + 4 * h4 + r) * kSkinnyLd + 16 * j + c16] = acc[b][j][r] - sum[b][r];
+    __syncthreads();
+    // wave w: rows w, w + nw, .. of column n0 + lane, each row of the output (and residual) a raw
+    // buffer of its own: columns past N fall outside, and M N may exceed 32-bit offsets
+    const int n = n0 + lane;
+    const float sw = a.out_i32 ? 0.0f : a.rs ? a.rs[min(n, a.N - 1)] : a.s_w;
+    for (int m = wave; m < a.M; m += nw) {
+        int v = 0;
+        for (int w = 0; w < nw; ++w) v += reinterpret_cast<const int*>(lds)[(w * 16 * MB + m) * kSkinnyLd + lane];
+        const size_t row = (size_t)m * a.ldo;
+        const __amdgpu_buffer_rsrc_t out =
+            __builtin_amdgcn_make_buffer_rsrc(static_cast<int*>(a.out) + row, 0, a.N * 4, kBufDword3);
+        unsigned bits = (unsigned)v;
+        if (!a.out_i32) {
+            float y = ((float)v * a.sx[m]) * sw;
+            if (a.res) {
+                const __amdgpu_buffer_rsrc_t res =
+                    __builtin_amdgcn_make_buffer_rsrc((void*)(a.res + row), 0, a.N * 4, kBufDword3);
+                y = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(res, n * 4, 0, 0)) + y;
+            }
+            bits = __builtin_bit_cast(unsigned, y);
+        }
+        __builtin_amdgcn_raw_buffer_store_b32(bits, out, n * 4, 0, 0);
+    }
+}
+
 // ---- M <= 64: K split over the waves ------------------------------------------------
 // One workgroup per 64-column tile of the output and all (<= 64) rows, over the unit's
 // chunks (a part of a long-K problem, GemmArgs::parts, or all C); compute wave w of NW
@@ -887,6 +1012,44 @@ static GemmGroupArgs group_args(const GemmArgs* dev, const int* u2p, const int* 
     return ga;
 }
 
+// Waves per workgroup.  With at most a workgroup per CU, a wave per quad of the longest problem
+// (up to 16): the launch is the latency of a wave's quads (6912 x 2560 at M = 3: 4 / 8 / 10
+// waves 5.8 / 5.3 / 4.9 us).  Up to two a CU, 8, so that both fit (a layer's 356 row blocks:
+// 4 / 8 / 10 / 16 waves 10.9 / 9.8 / 11.1 / 11.3 us).  Past that the chip is full anyway and
+// a wave's fixed cost counts (6912 row blocks: 2 / 4 / 8 waves 51.7 / 57.4 / 77.0 us).
+static int skinny_waves(int units, int maxC, int mb) {
+    const int quads = (maxC + 3) / 4;
+    const int nw = units <= kSkinnyOneRound ? 16 : units <= 2 * kSkinnyOneRound ? 8 : units <= 4 * kSkinnyOneRound ? 4 : 2;
+    return std::max(1, std::min(std::min(nw, 16 / mb), quads));
+}
+
+template <int MB>
+static hipError_t launch_skinny(const GemmGroupArgs& ga, int units, int minC, int maxC, hipStream_t s) {
+    const int nw = skinny_waves(units, maxC, MB);
+    const size_t lds = (size_t)nw * 16 * MB * kSkinnyLd * sizeof(int);
+    // weights beyond the L2s' 32 MB together are streamed past them (61 -> 52 us for 283 MB);
+    // smaller ones may stay for the next launch (q/k/v, down of one layer 3 and 12 % faster)
+    const bool nt = (long long)units * maxC * 1024 > (32ll << 20);
+    // many row blocks of equal length: contiguous ranges per XCD, so that a problem's
+    // activations come into one L2 (128 problems of 2 tokens: 100 -> 94 us).  Else round robin:
+    // the long problems lead the grid, and one XCD would get them all (a layer 11.4 -> 13.6).
+    const int xcd = minC == maxC && units > 4 * kSkinnyOneRound;
+    const dim3 grid((unsigned)units), block((unsigned)(64 * nw));
+    if (nt) hipLaunchKernelGGL((gemm_skinny_kernel<MB, true>), grid, block, lds, s, ga, xcd);
+    else hipLaunchKernelGGL((gemm_skinny_kernel<MB, false>), grid, block, lds, s, ga, xcd);
+    return hipGetLastError();
+}
+
+static hipError_t launch_skinny_m(const GemmGroupArgs& ga, int M, int units, int minC, int maxC, hipStream_t s) {
+    if (units <= 0) return hipSuccess;
+    return M <= 16 ? launch_skinny<1>(ga, units, minC, maxC, s) : launch_skinny<2>(ga, units, minC, maxC, s);
+}
+
+hipError_t launch_gemm_skinny(const GemmArgs* dev, const int* rb2p, const int* bnd, int nb, int M, int units, int minC,
+                              int maxC, hipStream_t s) {
+    return launch_skinny_m(group_args(dev, rb2p, bnd, nb), M, units, minC, maxC, s);
+}
+
 hipError_t launch_gemm_group(const GemmArgs* dev, const int* rb2p, const int* bnd, int nb, int total_rb,
                              hipStream_t s) {
     if (total_rb <= 0) return hipSuccess;
@@ -981,14 +1144,19 @@ hipError_t launch_gemm_tiles(const GemmArgs* dev, const int* tile2p, const int* 
 
 hipError_t launch_gemm(const GemmArgs& a, hipStream_t s) {
     if (a.M <= 0 || a.N <= 0) return hipSuccess;
+    const int units = a.Np / kRowBlock;
+    if (skinny_ok(a.M, units, false)) {
+        GemmArgs one = a;
+        one.wg_begin = 0;
+        return launch_skinny_m(GemmGroupArgs{nullptr, nullptr, one, -1, {}}, a.M, units, a.C, a.C, s);
+    }
     // byte offsets inside one tile's rows are 32-bit
     if (!gemm_ldo_ok(a.M, a.ldo)) return hipErrorInvalidValue;
     // gemm_bm(M) sized the activation padding; the row tile divides it or clamps its loads
-    const int bm = gemm_bm(a.M);
-    if (bm == 64) {
+    if (a.M <= 64) {
         GemmArgs one = a;
         one.wg_begin = 0;
-        return launch_splitk<kSplitkWaves, 4>(GemmGroupArgs{nullptr, nullptr, one, -1, {}}, a.Np / kRowBlock, s);
+        return launch_splitk<kSplitkWaves, 4>(GemmGroupArgs{nullptr, nullptr, one, -1, {}}, units, s);
     }
     const int cfg = gemm_tile_cfg(a.M, &a.N, &a.C, 1);
     GemmArgs one = a;

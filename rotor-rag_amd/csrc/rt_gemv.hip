@@ -1,5 +1,4 @@
-// Decode GEMV / skinny GEMM for the ternary linear, M = 1..8 tokens per workgroup,
-// no MFMA.  Replaces the reference's thread-per-row OpenCL kernel
+// Decode GEMV for the ternary linear, one token, no MFMA.  Replaces the reference's thread-per-row OpenCL kernel
 // (src/rotor/gpu_ternary.py:12-45, launched per token at src/rotor/transformer.py:134-143)
 // and its CPU twin np.dot(x, W_i8.T) * scale (src/rotor/transformer.py:150).
 //
@@ -698,16 +697,16 @@ GemvShape gemv_shape_fused(int total_rb, int min_C) {
     return GemvShape{true, nw};
 }
 
-GemvShape gemv_shape(int total_rb, int m_blocks, int min_C) {
+GemvShape gemv_shape(int total_rb, int min_C) {
     // Enough waves to fill 256 CUs x 8 waves; split K only when rows alone cannot.
-    const long long waves_rows = (long long)total_rb * m_blocks;
+    const int waves_rows = total_rb;
     GemvShape s;
     if (waves_rows >= 1024 || min_C < 4) {
         s.ksplit = false;
         s.nw = 4;
         return s;
     }
-    int nw = (int)((2048 + waves_rows - 1) / waves_rows);
+    int nw = (2048 + waves_rows - 1) / waves_rows;
     if (nw > 16) nw = 16;
     if (nw > min_C / 2) nw = min_C / 2;
     s.ksplit = nw > 1;
@@ -741,8 +740,9 @@ static void launch_ksplit(dim3 grid, int nw, size_t lds, hipStream_t s, const Ge
                        P.K, P.mode, P.eps, shape, nw_reciprocal(nw), one ? a.inl[0].w : nullptr, a, NoTail{});
 }
 
-hipError_t launch_gemv(const GemvArgs& args, int mt, GemvShape shape, hipStream_t s) {
+hipError_t launch_gemv(const GemvArgs& args, GemvShape shape, hipStream_t s) {
     if (args.total_rb <= 0 || args.M <= 0) return hipSuccess;
+    if (args.M != 1) return hipErrorInvalidValue;
     // the leading weight-stream table: the inline problems, or the one problem of a
     // single-problem launch as an inline problem
     GemvArgs a = args;
@@ -752,17 +752,16 @@ hipError_t launch_gemv(const GemvArgs& args, int mt, GemvShape shape, hipStream_
     }
     for (int j = 0; j < kInlineProbs; ++j)
         a.inw[j] = j < a.ninl ? GemvWeights{a.inl[j].w, a.inl[j].C, a.inl[j].wg_begin} : GemvWeights{nullptr, 0, 0};
-    const unsigned mblocks = (unsigned)((a.M + mt - 1) / mt);
     const dim3 block((unsigned)(64 * shape.nw));
     if (a.has_pro == 2) {  // single token, each problem's own row quantised in the prologue: ROWS
-        if (mt != 1 || a.M != 1 || shape.ksplit || a.total_rb % shape.nw) return hipErrorInvalidValue;
+        if (shape.ksplit || a.total_rb % shape.nw) return hipErrorInvalidValue;
         const dim3 grid((unsigned)(a.total_rb / shape.nw), 1);
         const size_t lds = (size_t)a.pro.Kp + sizeof(RowSmem);  // pro.Kp: the largest Kp of the problems
         hipLaunchKernelGGL((gemv_rows_kernel<1, 1>), grid, block, lds, s, a);
     } else if (a.has_pro && a.pair_a) {  // gate/up pair: an E-element prologue
         const QuantProb& P = a.pro;
         const int E = vec_elements(P.K, 64 * shape.nw);
-        if (mt != 1 || a.M != 1 || !shape.ksplit || P.K % 64 || !aligned16(P.x) || !aligned16(P.aux) ||
+        if (!shape.ksplit || P.K % 64 || !aligned16(P.x) || !aligned16(P.aux) ||
             !aligned16(P.aux2) || E == 0)
             return hipErrorInvalidValue;
         const dim3 grid((unsigned)a.total_rb, 1);
@@ -771,7 +770,7 @@ hipError_t launch_gemv(const GemvArgs& args, int mt, GemvShape shape, hipStream_
         else if (E == 8) launch_ksplit<1, 4, true>(grid, shape.nw, lds, s, a);
         else launch_ksplit<1, 6, true>(grid, shape.nw, lds, s, a);
     } else if (a.has_pro) {  // single token, prologue-quantised input: KSPLIT shape only
-        if (mt != 1 || a.M != 1 || !shape.ksplit) return hipErrorInvalidValue;
+        if (!shape.ksplit) return hipErrorInvalidValue;
         const dim3 grid((unsigned)a.total_rb, 1);
         const QuantProb& P = a.pro;
         const int nw = a.pro.mode == kAttnNorm ? std::min(shape.nw, kAttnMaxThreads / 64) : shape.nw;
@@ -788,24 +787,10 @@ hipError_t launch_gemv(const GemvArgs& args, int mt, GemvShape shape, hipStream_
             launch_ksplit<1, 1>(grid, nw, lds, s, a);
         }
     } else if (shape.ksplit) {
-        const dim3 grid((unsigned)a.total_rb, mblocks);
-        const size_t lds = (size_t)shape.nw * mt * kRowBlock * sizeof(int);
-        switch (mt) {
-            case 1: launch_ksplit<1, 0>(grid, shape.nw, lds, s, a); break;
-            case 2: launch_ksplit<2, 0>(grid, shape.nw, lds, s, a); break;
-            case 4: launch_ksplit<4, 0>(grid, shape.nw, lds, s, a); break;
-            case 8: launch_ksplit<8, 0>(grid, shape.nw, lds, s, a); break;
-            default: return hipErrorInvalidValue;
-        }
+        launch_ksplit<1, 0>(dim3((unsigned)a.total_rb), shape.nw, (size_t)shape.nw * kRowBlock * sizeof(int), s, a);
     } else {
-        const dim3 grid((unsigned)((a.total_rb + shape.nw - 1) / shape.nw), mblocks);
-        switch (mt) {
-            case 1: hipLaunchKernelGGL((gemv_rows_kernel<1, 0>), grid, block, 0, s, a); break;
-            case 2: hipLaunchKernelGGL((gemv_rows_kernel<2, 0>), grid, block, 0, s, a); break;
-            case 4: hipLaunchKernelGGL((gemv_rows_kernel<4, 0>), grid, block, 0, s, a); break;
-            case 8: hipLaunchKernelGGL((gemv_rows_kernel<8, 0>), grid, block, 0, s, a); break;
-            default: return hipErrorInvalidValue;
-        }
+        const dim3 grid((unsigned)((a.total_rb + shape.nw - 1) / shape.nw));
+        hipLaunchKernelGGL((gemv_rows_kernel<1, 0>), grid, block, 0, s, a);
     }
     return hipGetLastError();
 }

@@ -21,7 +21,8 @@
 //    so that dword i of a group holds element i of each of the 4 weight bytes of the
 //    matching weight dword: the decoded weight dword for field position i of a weight
 //    dword pairs with activation dword i in one v_dot4_i32_i8.  Padding is 0.
-//    Rows are padded with zeros to a multiple of the GEMV's tokens per workgroup.
+//    Rows are padded to the matrix kernels' row tiles; what the padding rows hold is not
+//    defined, and no output depends on it.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -202,7 +203,7 @@ struct GemvShape {
 
 struct QuantArgs {
     const QuantProb* dev;  // device descriptor array [U] or nullptr -> p
-    int U, M, Mpad;
+    int U, M;
     QuantProb p;
 };
 
@@ -303,7 +304,16 @@ __device__ __forceinline__ T lane63(T v) {
 __device__ __forceinline__ int wave_sum(int v) {
     return lane63(wave_reduce63(v, 0, [](int a, int b) { return a + b; }));
 }
-constexpr int kGemvMaxM = 8;  // up to this many tokens: VALU GEMV; beyond: MFMA GEMM
+constexpr int kGemvMaxM = 1;  // one token: VALU GEMV; beyond: MFMA GEMM
+// gemm_skinny_kernel's launches.  Up to 8 tokens always.  Up to 16 unless a long problem of the
+// group is to be cut into split-K parts (what rt_plan_describe reports of such a plan is kept).
+// Up to 32 with at most one workgroup per CU (two 16-row blocks a workgroup; launch alone, 20
+// layers in rotation, split-K / this: q/k/v 7.2 / 6.3, down 12.6 / 8.7 us, but a layer's 356
+// row blocks 12.6 / 15.8).
+constexpr int kSkinnyRows = 8, kSkinnyOneRound = 256;
+inline bool skinny_ok(int M, int units, bool split) {
+    return M <= kSkinnyRows || (!split && (M <= 16 || (M <= 32 && units <= kSkinnyOneRound)));
+}
 // qx layout.  Rows (M <= kGemvMaxM, read by the GEMV): row m at m * Kp.  Blocked
 // (M > kGemvMaxM, read by the MFMA GEMM): 16-row x 64-k blocks of 1 KiB, block
 // (m / 16, c) at (m / 16 * C + c) * 1024, where the 16-byte group q (k = 16 q .. 16 q + 15
@@ -312,10 +322,13 @@ constexpr int kGemvMaxM = 8;  // up to this many tokens: VALU GEMV; beyond: MFMA
 inline bool qx_blocked(int M) { return M > kGemvMaxM; }
 
 // rows of the GEMM workgroup tile for M tokens (the activations are zero-padded to it)
-inline int gemm_bm(int M) { return M <= 64 ? 64 : M <= 128 ? 128 : 256; }
+inline int gemm_bm(int M) { return M <= kSkinnyRows ? 16 : M <= 64 ? 64 : M <= 128 ? 128 : 256; }
 // The GEMM epilogues address one row tile of the output (and residual) with 32-bit byte
 // offsets and buffer ranges: a tile of gemm_bm(M) rows of ldo floats must span < 2^31 bytes.
-inline bool gemm_ldo_ok(int M, int ldo) { return (long long)gemm_bm(M) * ldo * 4 < (1ll << 31); }
+// (The skinny kernel addresses its outputs row by row.)
+inline bool gemm_ldo_ok(int M, int ldo) {
+    return M <= kSkinnyRows || (long long)gemm_bm(M) * ldo * 4 < (1ll << 31);
+}
 
 // Launchers (return hipSuccess or the launch error).
 hipError_t launch_relayout(const uint8_t* src, int N, int K, v4u* tiles, hipStream_t s);
@@ -326,8 +339,8 @@ hipError_t launch_quant(const QuantArgs& a, hipStream_t s, int maxK = 0);
 bool quant_rows_ok(const QuantProb& P);
 // qx rows [M][Kp] (permuted) -> natural-order int8 [M][K]
 hipError_t launch_unpermute(const int8_t* qx, int M, int K, int Kp, bool blocked, int8_t* q, hipStream_t s);
-// mt = tokens per workgroup (1, 2, 4 or 8).
-hipError_t launch_gemv(const GemvArgs& a, int mt, GemvShape shape, hipStream_t s);
+// One token (M = 1).
+hipError_t launch_gemv(const GemvArgs& a, GemvShape shape, hipStream_t s);
 hipError_t launch_gemm(const GemmArgs& a, hipStream_t s);
 // Tile shapes of the MFMA GEMM for M > 64 (rows x columns per workgroup).  A launch over
 // one or several problems (same M) takes 256 x 256 when that yields kGemmFillTiles tiles,
@@ -370,6 +383,9 @@ hipError_t launch_gemv_attn(const GemvArgs& args, const AttnTail& at, int Hkv, i
 // Workgroups of that launch (source row of K elements, nw waves, Gq query heads per KV head)
 // that the current device holds at once.
 hipError_t gemv_attn_capacity(int K, int Kp, int nw, int Gq, int* workgroups);
+// The same for gemm_skinny_kernel (skinny_ok; minC, maxC: the fewest and most chunks of a problem).
+hipError_t launch_gemm_skinny(const GemmArgs* dev, const int* rb2p, const int* bnd, int nb, int M, int units, int minC,
+                              int maxC, hipStream_t s);
 hipError_t launch_gemm_group(const GemmArgs* dev, const int* rb2p, const int* bnd, int nb, int total_rb,
                              hipStream_t s);
 // Once per device (current) before any launch: the function attributes the GEMM kernels
@@ -402,10 +418,8 @@ hipError_t launch_lm_head(const uint16_t* E, const float* x, const float* norm_w
                           float* logits, unsigned long long* best, int* token, int* pos, int advance,
                           int* next_ids, int* out_tokens, int pos_base, int out_cap, float* next_h, hipStream_t s);
 
-// Host policy: tokens per workgroup for M tokens.
-inline int gemv_mt(int M) { return M <= 1 ? 1 : M <= 2 ? 2 : M <= 4 ? 4 : 8; }
 // Host policy: launch shape so that small launches still fill the chip.
-GemvShape gemv_shape(int total_rb, int m_blocks, int min_C);
+GemvShape gemv_shape(int total_rb, int min_C);
 // Launch shape of a plan whose GEMV quantises its input in the prologue (M = 1).
 GemvShape gemv_shape_fused(int total_rb, int min_C);
 // Elements per thread (4, 8 or 16) of the vectorised decode prologue for a row of K

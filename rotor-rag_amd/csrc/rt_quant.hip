@@ -3,7 +3,10 @@
 // the FFN sub-norm), and the int8 permute used by the int32 parity entry point.
 // The row arithmetic lives in rt_rowquant.h (shared with the decode GEMV prologue).
 //
-// One 256-thread workgroup per token row; rows in [M, Mpad) are zero-filled.
+// One workgroup per token row.  The rows that pad the tokens to the matrix kernels' row tiles are
+// left as they are: a padding row's bytes reach only that row's accumulators, which no kernel
+// stores.  (Zeroing them took more of the launch than the tokens' rows for few tokens: 128
+// inputs of 2 tokens in 16-row tiles, 118 -> 99 us for the plan.)
 #include <algorithm>
 
 #include "rt_rowquant.h"
@@ -23,12 +26,6 @@ __global__ void __launch_bounds__(256) quant_kernel(QuantArgs a) {
     v4u* const qx = reinterpret_cast<v4u*>(P.qx);
     const QxRow qrow = P.blocked ? QxRow{qx + (size_t)(m >> 4) * (Kp >> 6) * 64 + (m & 15), 64, 16}
                                  : QxRow{qx + (size_t)m * (Kp >> 4), 4, 1};
-    if (m >= a.M) {  // padding token rows
-        const v4u z = {0u, 0u, 0u, 0u};
-        for (int g = threadIdx.x; g < groups; g += blockDim.x) qrow[g] = z;
-        if (threadIdx.x == 0 && P.sx) P.sx[m] = 0.0f;
-        return;
-    }
     if (P.mode == kPermute) {  // int8 in natural order -> qx
         const int8_t* qr = P.q_in + (size_t)m * K;
         for (int g = threadIdx.x; g < groups; g += blockDim.x) {
@@ -62,12 +59,6 @@ __global__ void __launch_bounds__(1024) quant_rows_kernel(QuantArgs a) {
     v4u* const qx = reinterpret_cast<v4u*>(P.qx);
     const QxRow qrow = P.blocked ? QxRow{qx + (size_t)(m >> 4) * (Kp >> 6) * 64 + (m & 15), 64, 16}
                                  : QxRow{qx + (size_t)m * (Kp >> 4), 4, 1};
-    if (m >= a.M) {  // padding token rows
-        const v4u z = {0u, 0u, 0u, 0u};
-        for (int g = threadIdx.x; g < groups; g += blockDim.x) qrow[g] = z;
-        if (threadIdx.x == 0 && P.sx) P.sx[m] = 0.0f;
-        return;
-    }
     QuantProb R = P;  // row m of the sources
     R.x = P.x + (size_t)m * P.K;
     if (has_relu2(P)) R.aux = P.aux + (size_t)m * P.K;
@@ -107,9 +98,9 @@ bool quant_rows_ok(const QuantProb& P) {
 }
 
 hipError_t launch_quant(const QuantArgs& a, hipStream_t s, int maxK) {
-    if (a.U <= 0 || a.Mpad <= 0) return hipSuccess;
+    if (a.U <= 0 || a.M <= 0) return hipSuccess;
     if (maxK > 0) {  // every problem passed quant_rows_ok; maxK: the largest K
-        const dim3 grid((unsigned)a.Mpad, (unsigned)a.U);
+        const dim3 grid((unsigned)a.M, (unsigned)a.U);
         const size_t lds = 8192 + sizeof(RowSmem);
         // whole waves (the workgroup reductions take one slot per wave); 8 or 16 elements per
         // thread: fewer waves in the row's two reductions (512-token prefill 4.70 -> 4.59 ms
@@ -121,7 +112,7 @@ hipError_t launch_quant(const QuantArgs& a, hipStream_t s, int maxK) {
         }
         return hipGetLastError();
     }
-    hipLaunchKernelGGL(quant_kernel, dim3((unsigned)a.Mpad, (unsigned)a.U), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(quant_kernel, dim3((unsigned)a.M, (unsigned)a.U), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

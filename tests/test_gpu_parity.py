@@ -290,6 +290,61 @@ def test_splitk_parts_vs_oracle(hip, K_long, parts):
             assert np.array_equal(y.cpu().numpy(), y_exact), f"run {rep}: {y.shape[1]}x{x.shape[1]}"
 
 
+# gemm_skinny_kernel: both row-block counts and their edges, K of one chunk, a ragged quad of
+# chunks, fewer quads than waves and more; N of part of a row block, one, one and a bit, many
+@pytest.mark.parametrize("M", [2, 7, 8, 9, 16, 17, 31, 32])
+@pytest.mark.parametrize("N,K", [(1, 64), (64, 60), (65, 320), (1111, 2050), (200, 6912), (16500, 256)])
+def test_skinny_vs_oracle(hip, M, N, K):
+    """int32 accumulators over the full int8 range, the fp32 epilogue with per-row scales and
+    with a residual, bit-exact."""
+    import torch
+
+    rng = np.random.default_rng(M + N + K)
+    W, scale = O.make_ternary(rng, N, K)
+    w = hip.upload(O.pack_rotor(W), K, scale)
+    q = rng.integers(-128, 128, size=(M, K), dtype=np.int8)
+    acc = hip.linear_i32(w, torch.from_numpy(q)).cpu().numpy()
+    assert np.array_equal(acc.astype(np.int64), O.linear_i64_fast(q, W))
+    x = rng.standard_normal((M, K), dtype=np.float32)
+    rs = rng.uniform(0.01, 0.05, N).astype(np.float32)
+    r = rng.standard_normal((M, N), dtype=np.float32)
+    _, q, s, acc = O.ternary_linear(x, W, scale)
+    y = hip.linear_device(w, torch.from_numpy(x), row_scale=torch.from_numpy(rs)).cpu().numpy()
+    assert np.array_equal(y, (acc.astype(np.float32) * s[:, None]) * rs)
+    act = hip.activations(40, K)
+    hip.act_quantize(torch.from_numpy(x).cuda(), act)
+    y = hip.linear_act(w, act, residual=torch.from_numpy(r).cuda()).cpu().numpy()
+    assert np.array_equal(y, r + (acc.astype(np.float32) * s[:, None]) * np.float32(scale))
+
+
+# plans on it: two problems of unequal K, more than a workgroup per CU, more than 16 problems
+# (descriptors from the table), weights past the L2s (streamed)
+@pytest.mark.parametrize("M,shapes", [(5, [(100, 640), (200, 7040)]), (16, [(17000, 300), (640, 300)]),
+                                      (3, [(1000, 128)] * 20), (2, [(35000, 256), (70, 320)]),
+                                      (8, [(40000, 3500)]), (32, [(2560, 640), (100, 640)])])
+def test_skinny_plans_equal_oracle(hip, M, shapes):
+    import torch
+
+    from rotor import _hip as H_
+
+    rng = np.random.default_rng(M + len(shapes))
+    ws, xs, ys, cases = [], [], [], []
+    for N, K in shapes:
+        W, scale = O.make_ternary(rng, N, K)
+        cases.append((rng.standard_normal((M, K), dtype=np.float32), W, scale))
+        ws.append(hip.upload(O.pack_rotor(W), K, scale))
+        xs.append(torch.from_numpy(cases[-1][0]).cuda())
+        ys.append(torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda"))
+    plan = hip.plan(ws, xs, ys)
+    assert plan.describe() == (H_.LAUNCH_SPLITK, 16 if M <= 16 else 32, 64, sum((N + 63) // 64 for N, _ in shapes))
+    for _ in range(2):
+        plan.run()
+        torch.cuda.synchronize()
+        for (x, W, scale), y in zip(cases, ys):
+            _, q, s, acc = O.ternary_linear(x, W, scale)
+            assert np.array_equal(y.cpu().numpy(), (acc.astype(np.float32) * s[:, None]) * np.float32(scale))
+
+
 @pytest.mark.parametrize("G", [3, 16, 17, 20])
 @pytest.mark.parametrize("M", [20, 100])
 def test_grouped_gemm_descriptor_lookup(hip, G, M):
