@@ -791,8 +791,8 @@ __global__ void __launch_bounds__(1024 / MB) gemm_skinny_kernel(GemmGroupArgs ga
     }
 }
 
-// ---- M <= 64: K split over the waves ------------------------------------------------
-// One workgroup per 64-column tile of the output and all (<= 64) rows, over the unit's
+// ---- M <= 64, and single problems of few tiles: K split over the waves -----------------
+// One workgroup per 64-column tile of the output and up to 64 rows, over the unit's
 // chunks (a part of a long-K problem, GemmArgs::parts, or all C); compute wave w of NW
 // covers an NW-th of them (a wave tile of 64 x 64 = 2 x 2 blocks of 32 x 32, fragment
 // reads, weight expansion and result layout those of gemm_kernel) from a private LDS ring
@@ -815,7 +815,15 @@ __global__ void __launch_bounds__(2 * NW * 64, 4) gemm_splitk_kernel(GemmGroupAr
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const bool loader = wave >= NW;
     const int cw = loader ? wave - NW : wave;  // the compute wave this wave is or feeds
-    const GemmArgs a = find_gemm(ga, blockIdx.x);
+    GemmArgs a = find_gemm(ga, blockIdx.x);
+    if (gridDim.y > 1) {  // 64-row tile blockIdx.y of a longer single problem
+        const int m0 = (int)blockIdx.y * 64;
+        a.qx += (size_t)(m0 >> 4) * a.C * 1024;
+        a.sx += m0;
+        a.out = static_cast<char*>(a.out) + (size_t)m0 * a.ldo * 4;
+        if (a.res) a.res += (size_t)m0 * a.ldo;
+        a.M = min(a.M - m0, 64);
+    }
     const int C = a.C, rb = (int)blockIdx.x - a.wg_begin, n0 = rb * kRowBlock;
     // the epilogue's scales (thread t: column n0 + t % 64, rows t / 64 + 2 NW j), requested now
     // so that the epilogue does not wait for them (a load wave's ring waits count them too:
@@ -991,17 +999,17 @@ template <int NW, int S>
 constexpr int splitk_lds() { return NW * S * (5 * 1024); }
 
 template <int NW, int S>
-static hipError_t launch_splitk(const GemmGroupArgs& ga, int blocks, hipStream_t s) {
+static hipError_t launch_splitk(const GemmGroupArgs& ga, int blocks, hipStream_t s, int mtiles = 1) {
     constexpr int LDS = splitk_lds<NW, S>();
     static_assert(S * 5 * 1024 >= 64 * 64 * 4 + 4, "a wave's ring must hold its partial tile (and wave 0's the arrival flag)");
-    hipLaunchKernelGGL((gemm_splitk_kernel<NW, S>), dim3((unsigned)blocks), dim3(2 * NW * 64), LDS, s, ga);
+    hipLaunchKernelGGL((gemm_splitk_kernel<NW, S>), dim3((unsigned)blocks, (unsigned)mtiles), dim3(2 * NW * 64), LDS, s, ga);
     return hipGetLastError();
 }
 
 // Four waves per workgroup: 80 KiB of LDS, so two workgroups share a CU and the 356 row
 // blocks of a BitNet-2B layer's seven projections are all resident at once (21.2 -> 19.8 us
 // against eight waves, 160 KiB, one workgroup per CU and 1.4 rounds).
-constexpr int kSplitkWaves = 4;
+constexpr int kSplitkWaves = 4, kSplitkOneRound = 512;
 
 static GemmGroupArgs group_args(const GemmArgs* dev, const int* u2p, const int* bnd, int nb) {
     GemmGroupArgs ga{dev, u2p, GemmArgs{}, -1, {}};
@@ -1153,10 +1161,17 @@ hipError_t launch_gemm(const GemmArgs& a, hipStream_t s) {
     // byte offsets inside one tile's rows are 32-bit
     if (!gemm_ldo_ok(a.M, a.ldo)) return hipErrorInvalidValue;
     // gemm_bm(M) sized the activation padding; the row tile divides it or clamps its loads
-    if (a.M <= 64) {
+    // 64-row tiles with K split over the waves while they fill the chip no more than once (two a
+    // CU): the larger tiles leave most CUs idle there, each walking all of K.  Launch alone,
+    // tiles / this: 2560 x 2560 at 128 / 300 / 512 tokens 13.7 / 11.5 / 12.1 -> 7.4 / 8.1 / 11.4 us,
+    // 2560 x 6912 at 201 / 512 22.2 / 23.9 -> 13.9 / 20.9, 640 x 2560 at 1024 11.2 -> 8.1; past the
+    // line they lose (6912 x 2560 at 512, 864 tiles: 18.2 -> 21.0), and for long prompts of
+    // narrow matrices the line is one a CU (1111 x 2050 at 1024, 288 tiles: 10.6 -> 10.8).
+    const long long tiles64 = (long long)units * ((a.M + 63) / 64);
+    if (a.M <= 64 || tiles64 <= kSplitkOneRound / 2 || (tiles64 <= kSplitkOneRound && a.M <= 768)) {
         GemmArgs one = a;
         one.wg_begin = 0;
-        return launch_splitk<kSplitkWaves, 4>(GemmGroupArgs{nullptr, nullptr, one, -1, {}}, units, s);
+        return launch_splitk<kSplitkWaves, 4>(GemmGroupArgs{nullptr, nullptr, one, -1, {}}, units, s, (a.M + 63) / 64);
     }
     const int cfg = gemm_tile_cfg(a.M, &a.N, &a.C, 1);
     GemmArgs one = a;

@@ -317,7 +317,32 @@ def test_skinny_vs_oracle(hip, M, N, K):
     assert np.array_equal(y, r + (acc.astype(np.float32) * s[:, None]) * np.float32(scale))
 
 
-# plans on it: two problems of unequal K, more than a workgroup per CU, more than 16 problems
+# single problems of more than 64 tokens as 64-row tiles with K split over the waves: the edges of
+# a row tile and of the 128- and 256-row padding, fewer chunks than waves, ragged N and K, both
+# sides of the line to the larger tiles (256 tiles at M > 768, 512 below)
+@pytest.mark.parametrize("M,N,K", [(65, 64, 64), (128, 70, 130), (129, 1111, 2050), (192, 300, 448), (257, 130, 6912),
+                                   (704, 2944, 320), (705, 2944, 320), (1024, 1024, 576), (1025, 1024, 576),
+                                   (2000, 60, 200)])
+def test_splitk_row_tiles_vs_oracle(hip, M, N, K):
+    import torch
+
+    rng = np.random.default_rng(M + N + K)
+    W, scale = O.make_ternary(rng, N, K)
+    w = hip.upload(O.pack_rotor(W), K, scale)
+    q = rng.integers(-128, 128, size=(M, K), dtype=np.int8)
+    assert np.array_equal(hip.linear_i32(w, torch.from_numpy(q)).cpu().numpy().astype(np.int64), O.linear_i64_fast(q, W))
+    x = rng.standard_normal((M, K), dtype=np.float32)
+    r = rng.standard_normal((M, N), dtype=np.float32)
+    _, q, s, acc = O.ternary_linear(x, W, scale)
+    act = hip.activations(M, K)
+    hip.act_quantize(torch.from_numpy(x).cuda(), act)
+    y = torch.full((M + 1, N), 7.0, device="cuda")
+    hip.linear_act(w, act, out=y, residual=torch.from_numpy(r).cuda())
+    assert np.array_equal(y[:M].cpu().numpy(), r + (acc.astype(np.float32) * s[:, None]) * np.float32(scale))
+    assert (y[M] == 7.0).all()  # nothing past the tokens' rows
+
+
+# plans on gemm_skinny_kernel: two problems of unequal K, more than a workgroup per CU, more than 16 problems
 # (descriptors from the table), weights past the L2s (streamed)
 @pytest.mark.parametrize("M,shapes", [(5, [(100, 640), (200, 7040)]), (16, [(17000, 300), (640, 300)]),
                                       (3, [(1000, 128)] * 20), (2, [(35000, 256), (70, 320)]),
