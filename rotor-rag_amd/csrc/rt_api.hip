@@ -640,10 +640,9 @@ static hipError_t upload_gemm_group(rt_plan* p) {
         Cs[i] = g[i].C;
     }
     p->gemm_cfg = gemm_tile_cfg(p->M, Ns.data(), Cs.data(), (int)g.size());
-    // the pair epilogue runs in tiles whose waves hold one 64-column group: not the 64-row
-    // tile's 32 columns, the 256-column tile's 128 or the region kernel (its own epilogue)
+    // the pair epilogue runs in tiles whose waves hold whole 64-column groups: not the 64-row
+    // tile's 32 columns or the region kernel (its own epilogue)
     if (p->pair_gemm && (p->gemm_cfg == kTile64x128 || p->gemm_cfg == kRegion128x160)) p->gemm_cfg = kTile128x128;
-    if (p->pair_gemm && p->gemm_cfg == kTile256x256) p->gemm_cfg = kTile256x128;
     long long total = 0;
     for (size_t i = 0; i < g.size(); ++i) {
         g[i].wg_begin = (int)total;

@@ -222,7 +222,7 @@ __device__ __forceinline__ GemmArgs find_gemm(const GemmGroupArgs& ga, int b) {
     const cgemm* q = (cgemm*)ga.dev + j;
     return GemmArgs{q->w,  q->qx,       q->sx, q->rs, q->out, q->s_w, q->M,     q->N,   q->Np,
                     q->C,  q->ldo,      q->out_i32, q->res, q->wg_begin, q->c0, q->c1, q->kp, q->parts,
-                    q->cnt, q->part_ws, q->pair_a, q->pair_sg, q->pair_su};
+                    q->cnt, q->part_ws, nullptr, 0.0f, 0.0f, j};
 }
 
 template <int BM, int BN, int WAVES_M, int STAGES>
@@ -381,12 +381,25 @@ __global__ void __launch_bounds__(256) gemm_kernel(GemmGroupArgs ga) {
     // epilogue (this barrier publishes the row scales)
     wait_barrier<0>();
     const int rows = min(BM, a.M - m0);
+    if constexpr (FJ % 2 == 0) {
+        // the gate/up pair's fields are read from the descriptor here (the empty asm keeps the
+        // loads behind the main loop): held through it, they made the 256-column tile spill
+        if (ga.dev) {
+            const cgemm* q = (cgemm*)ga.dev;
+            asm volatile("" : "+s"(q));
+            q += a.idx;
+            GemmArgs pr = a;
+            pr.pair_a = q->pair_a;
+            if (pr.pair_a) {
+                pr.pair_sg = q->pair_sg;
+                pr.pair_su = q->pair_su;
+                store_tile_pair<FI, FJ>(acc, pr, m0, rows, mrow, nb, sx_lds);
+                return;
+            }
+        }
+    }
     if (a.out_i32) {
         store_tile<FI, FJ, 0>(acc, a, m0, rows, mrow, nb, sx_lds, swv);
-    } else if (FJ == 2 && a.pair_a) {
-        // the host pairs only tiles whose waves hold one 64-column group (in the 256-column
-        // tile, even holding pair_a through the main loop made it spill)
-        if constexpr (FJ == 2) store_tile_pair<FI, FJ>(acc, a, m0, rows, mrow, nb, sx_lds);
     } else if (a.res) {
         store_tile<FI, FJ, 2>(acc, a, m0, rows, mrow, nb, sx_lds, swv);
     } else {

@@ -232,6 +232,7 @@ struct GemmArgs {
     // g = ((float)acc * sx) * pair_sg and u likewise with pair_su
     float* pair_a;
     float pair_sg, pair_su;
+    int idx;  // in a kernel: the descriptor's index in the launch
 };
 
 constexpr int kBufDword3 = 0x00020000;  // buffer resource word 3 for gfx9 raw buffers

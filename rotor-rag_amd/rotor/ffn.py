@@ -16,7 +16,9 @@ Otherwise, and for several tokens, four:
   2. gate and up in one GEMV/GEMM launch on the shared int8 x (rt_plan_create_act)
   3. relu^2(gate) * up fused with the quantiser               (rt_act_relu2_mul_quantize)
   4. down on the int8 activations                             (rt_linear_act_f32)
-Both give the same bits.  No call allocates device memory after the first forward at a
+where, past 64 tokens and at those widths, 2 runs on the interleaved copy and writes
+relu^2(gate) * up itself (rt_plan_create_act_gate_up), half the bytes 3 then reads and
+quantises.  All give the same bits.  No call allocates device memory after the first forward at a
 given token count (and, for one token, input buffer), so a forward can be captured in a
 HIP graph.
 """
@@ -37,10 +39,10 @@ class TernaryFFNBlock:
         self.up_proj = TernaryLinear(d_model, d_ff, use_gpu)
         self.down_proj = TernaryLinear(d_ff, d_model, use_gpu)
         self.gpu = self.gate_proj.gpu
-        self._state = {}   # token count -> (plan, g, u, y)
+        self._state = {}   # token count -> (plan, g, u, y); u None: g is relu^2(gate) * up
         self._acts = None
         self._norm_w_dev = None
-        self._gu = None      # interleaved gate/up copy for the one-token path
+        self._gu = None      # interleaved gate/up copy for one token and for more than 64
         self._pair = None    # (input pointer, gate/up plan, down plan, y)
         self._xin = None     # forward()'s device copy of its input
         self.pair_ok = d_model % 64 == 0 and d_ff % 64 == 0 and d_ff <= 8192
@@ -60,6 +62,18 @@ class TernaryFFNBlock:
             self._acts = (self.gpu.activations(self.max_tokens, self.d_model),
                           self.gpu.activations(self.max_tokens, self.d_ff))
 
+    def _gate_up(self):
+        """The interleaved gate/up matrix (HIPTernaryOps.interleave_gate_up's layout) and its
+        scales, laid out on the device from the rotor bytes the layers were loaded with."""
+        if self._gu is None:
+            import torch
+
+            dev, D, F = self.gpu.device, self.d_model, self.d_ff
+            g, u = (torch.from_numpy(p._packed).to(dev).view(F // 32, 32, -1) for p in (self.gate_proj, self.up_proj))
+            self._gu = (self.gpu.upload_device(torch.stack([g, u], dim=1).view(2 * F, -1), D, 1.0),
+                        (self.gate_proj.scale, self.up_proj.scale))
+        return self._gu
+
     def _buffers(self, M):
         st = self._state.get(M)
         if st is None:
@@ -67,11 +81,16 @@ class TernaryFFNBlock:
 
             dev = self.gpu.device
             g = torch.empty((M, self.d_ff), dtype=torch.float32, device=dev)
-            u = torch.empty((M, self.d_ff), dtype=torch.float32, device=dev)
             y = torch.empty((M, self.d_model), dtype=torch.float32, device=dev)
             act_h = self._acts[0]
-            plan = self.gpu.plan_act([self.gate_proj.gpu_packed_weights, self.up_proj.gpu_packed_weights],
-                                     [act_h, act_h], M, [g, u])
+            u = None
+            if M > 64 and self.pair_ok:
+                w_gu, scales = self._gate_up()
+                plan = self.gpu.plan_act_gate_up(w_gu, scales, act_h, M, g)
+            else:
+                u = torch.empty((M, self.d_ff), dtype=torch.float32, device=dev)
+                plan = self.gpu.plan_act([self.gate_proj.gpu_packed_weights, self.up_proj.gpu_packed_weights],
+                                         [act_h, act_h], M, [g, u])
             st = self._state[M] = (plan, g, u, y)
         return st
 
@@ -84,9 +103,7 @@ class TernaryFFNBlock:
             from . import _hip
 
             hip, dev = self.gpu, self.gpu.device
-            if self._gu is None:
-                self._gu = hip.interleave_gate_up(self.gate_proj.gpu_packed_weights, self.up_proj.gpu_packed_weights)
-            w_gu, scales = self._gu
+            w_gu, scales = self._gate_up()
             a = torch.empty(self.d_ff, dtype=torch.float32, device=dev)
             ssq = torch.empty(self.d_ff // 32, dtype=torch.float64, device=dev)
             y = torch.empty((1, self.d_model), dtype=torch.float32, device=dev)
@@ -118,7 +135,10 @@ class TernaryFFNBlock:
         hip.act_rmsnorm_quantize(x, self._norm_w_dev, act_h, self.eps)
         act_h.tokens = M
         plan.gemv()
-        hip.act_relu2_mul_quantize(g, u, act_a)
+        if u is None:
+            hip.act_quantize(g, act_a)
+        else:
+            hip.act_relu2_mul_quantize(g, u, act_a)
         hip.linear_act(self.down_proj.gpu_packed_weights, act_a, out=y)
         return y
 
