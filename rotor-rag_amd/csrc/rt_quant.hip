@@ -46,28 +46,108 @@ __global__ void __launch_bounds__(256) quant_kernel(QuantArgs a) {
     if (threadIdx.x == 0 && P.sx) P.sx[m] = s;
 }
 
-// Rows with K % 64 == 0 and no natural-order / value outputs: K / E threads per row, E
-// (4 or 8) consecutive elements each (the decode prologue's row path), the int8 row
-// assembled in LDS and copied out 16 bytes per thread.
-template <int E>
-__global__ void __launch_bounds__(1024) quant_rows_kernel(QuantArgs a) {
-    extern __shared__ __attribute__((aligned(16))) v4u qrow_lds[];
-    RowSmem* sm = reinterpret_cast<RowSmem*>(qrow_lds + 512);  // rows of up to 8192 bytes
+// Rows with K % 64 == 0 and no natural-order / value outputs.  Thread t of T reads float4
+// i T + t, i < NV, so a wave's load is one contiguous KiB.  The four lanes of a quad hold the 16
+// elements of one group; a 4 x 4 byte transpose within the quad (two DPP exchanges) gives each
+// lane one dword of the permuted group, stored directly.  The rows go to the XCDs in
+// contiguous ranges: the 16 rows of a block share its lines 16 bytes at a time, and dealt out
+// row by row every XCD's L2 wrote back its own part of each.
+// Bound by the latency of its two reductions for few rows, by memory and the f64 quotients for
+// many.  Measured (launch alone, 10 inputs in rotation; before: 8 or 16 consecutive elements
+// per thread, the row assembled in LDS, rows round robin): 2560 wide, plain 5 / 512 / 2048 rows
+// 3.6 / 5.6 / 10.5 -> 3.3 / 4.5 / 8.0 us, RMSNorm 4.4 / 6.8 / 13.8 -> 4.4 / 5.8 / 10.6; 6912 wide,
+// plain 4.0 / 8.3 / 25.9 -> 3.8 / 6.6 / 19.1, RMSNorm 5.7 / 11.0 / 33.1 -> 5.3 / 9.1 / 25.3.
+template <int CTRL>
+__device__ __forceinline__ unsigned quad_perm(unsigned v) {
+    return (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, 0xf, 0xf, true);
+}
+template <int NV>
+__global__ void __launch_bounds__(NV == 4 ? 512 : 256) quant_wide_kernel(QuantArgs a) {
+    __shared__ RowSmem sm;
     const QuantProb P = select_quant(a, blockIdx.y);
-    const int m = blockIdx.x;
-    const int Kp = P.Kp, groups = Kp >> 4;
-    v4u* const qx = reinterpret_cast<v4u*>(P.qx);
-    const QxRow qrow = P.blocked ? QxRow{qx + (size_t)(m >> 4) * (Kp >> 6) * 64 + (m & 15), 64, 16}
-                                 : QxRow{qx + (size_t)m * (Kp >> 4), 4, 1};
-    QuantProb R = P;  // row m of the sources
-    R.x = P.x + (size_t)m * P.K;
-    if (has_relu2(P)) R.aux = P.aux + (size_t)m * P.K;
-    RowRegsE<E> rr;
-    row_loadE<E>(R, rr);
-    const float s = row_finishE<E>(R, rr, qrow_lds, sm);
+    const int m = xcd_order((int)blockIdx.x, (int)gridDim.x), t = threadIdx.x, T = (int)blockDim.x, K = P.K, F4 = K >> 2;
+    const int nw = T >> 6, wave = t >> 6, lane = t & 63;
+    const bool relu2 = has_relu2(P), norm = has_norm(P);
+    const float4* x = reinterpret_cast<const float4*>(P.x + (size_t)m * K);
+    const float4* up = reinterpret_cast<const float4*>(P.aux + (relu2 ? (size_t)m * K : 0));
+    const float4* nwt = reinterpret_cast<const float4*>(norm_weight(P));
+    float v[NV][4];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int f = i * T + t;
+        const float4 z = f < F4 ? x[f] : float4{0.0f, 0.0f, 0.0f, 0.0f};
+        v[i][0] = z.x;
+        v[i][1] = z.y;
+        v[i][2] = z.z;
+        v[i][3] = z.w;
+    }
+    if (relu2) {
+        float4 u[NV];
+#pragma unroll
+        for (int i = 0; i < NV; ++i) u[i] = i * T + t < F4 ? up[i * T + t] : float4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const float uu[4] = {u[i].x, u[i].y, u[i].z, u[i].w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[i][j] = v[i][j] > 0.0f ? (v[i][j] * v[i][j]) * uu[j] : 0.0f;
+        }
+    }
+    if (norm) {
+        float4 w[NV];  // requested before the reduction
+#pragma unroll
+        for (int i = 0; i < NV; ++i) w[i] = i * T + t < F4 ? nwt[i * T + t] : float4{0.0f, 0.0f, 0.0f, 0.0f};
+        double ss = 0.0;
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) ss += (double)v[i][j] * (double)v[i][j];
+        ss = wave_reduce63(ss, 0.0, [](double p, double q) { return p + q; });
+        if (lane == 63) sm.d[wave] = ss;
+        __syncthreads();
+        ss = sm.d[0];
+        for (int k = 1; k < nw; ++k) ss += sm.d[k];
+        const float nrm = sqrtf((float)(ss / (double)K) + P.eps);
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            divide_all<4>(v[i], nrm);
+            const float ww[4] = {w[i].x, w[i].y, w[i].z, w[i].w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[i][j] = i * T + t < F4 ? v[i][j] * ww[j] : 0.0f;
+        }
+    }
+    float amax = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) amax = fmaxf(amax, fabsf(v[i][j]));
+    amax = wave_reduce63(amax, 0.0f, [](float p, float q) { return fmaxf(p, q); });
+    if (lane == 63) sm.f[wave] = amax;
     __syncthreads();
-    for (int g = threadIdx.x; g < groups; g += blockDim.x) qrow[g] = qrow_lds[g];
-    if (threadIdx.x == 0 && P.sx) P.sx[m] = s;
+    amax = sm.f[0];
+    for (int k = 1; k < nw; ++k) amax = fmaxf(amax, sm.f[k]);
+    const float sc = amax > 0.0f ? amax / 127.0f : 1.0f;
+    if (t == 0 && P.sx) P.sx[m] = sc;
+    const double rs = 1.0 / (double)sc;  // as scatter_q
+    v4u* const qx = reinterpret_cast<v4u*>(P.qx);
+    const QxRow qrow = P.blocked ? QxRow{qx + (size_t)(m >> 4) * (P.Kp >> 6) * 64 + (m & 15), 64, 16}
+                                 : QxRow{qx + (size_t)m * (P.Kp >> 4), 4, 1};
+    const bool odd = t & 1, high = t & 2;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        unsigned d = 0u;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float f = rintf((float)((double)v[i][j] * rs));
+            d |= ((unsigned)(int)fminf(fmaxf(f, -128.0f), 127.0f) & 0xffu) << (8 * j);
+        }
+        // byte j of lane b to byte b of lane j
+        const unsigned e = quad_perm<0xB1>(d);  // lane ^ 1
+        const unsigned p = __builtin_amdgcn_perm(d, e, odd ? 0x07030501u : 0x02060004u);
+        const unsigned r = quad_perm<0x4E>(p);  // lane ^ 2
+        const unsigned o = high ? (p & 0xFFFF0000u) | (r >> 16) : (p & 0xFFFFu) | (r << 16);
+        const int f4 = i * T + t;
+        if (f4 < F4) reinterpret_cast<unsigned*>(&qrow[f4 >> 2])[t & 3] = o;
+    }
 }
 
 __global__ void __launch_bounds__(256) unpermute_kernel(const int8_t* __restrict__ qx, int K, int Kp, int blocked,
@@ -100,15 +180,19 @@ bool quant_rows_ok(const QuantProb& P) {
 hipError_t launch_quant(const QuantArgs& a, hipStream_t s, int maxK) {
     if (a.U <= 0 || a.M <= 0) return hipSuccess;
     if (maxK > 0) {  // every problem passed quant_rows_ok; maxK: the largest K
-        const dim3 grid((unsigned)a.M, (unsigned)a.U);
-        const size_t lds = 8192 + sizeof(RowSmem);
-        // whole waves (the workgroup reductions take one slot per wave); 8 or 16 elements per
-        // thread: fewer waves in the row's two reductions (512-token prefill 4.70 -> 4.59 ms
-        // against 4 and 8)
-        if (maxK <= 4096) {
-            hipLaunchKernelGGL((quant_rows_kernel<8>), grid, dim3((unsigned)((maxK / 8 + 63) / 64 * 64)), lds, s, a);
-        } else {
-            hipLaunchKernelGGL((quant_rows_kernel<16>), grid, dim3((unsigned)((maxK / 16 + 63) / 64 * 64)), lds, s, a);
+        // float4s per thread: few rows want their reductions over little work per thread (2560
+        // wide, RMSNorm, 5 rows: 4 / 8 / 10 a thread 4.4 / 5.4 / 6.1 us; 1024 wide 2 a thread, whose
+        // two waves measured 3 % under 4's four); many rows fewer waves each (2560 wide, 2048
+        // rows: 11.9 / 13.7 / 10.6, one wave a row with 10; 6912 wide 30.8 / 25.3 / 30.6)
+        const bool many = (long long)a.M * a.U > 1024;
+        const int NV = many && maxK > 2560 ? 8 : many && maxK > 1536 ? 10 : maxK > 1024 ? 4 : 2;
+        const unsigned threads = (unsigned)round_up((maxK / 4 + NV - 1) / NV, 64);
+        const dim3 grid((unsigned)a.M, (unsigned)a.U), block(threads);
+        switch (NV) {
+            case 2: hipLaunchKernelGGL((quant_wide_kernel<2>), grid, block, 0, s, a); break;
+            case 4: hipLaunchKernelGGL((quant_wide_kernel<4>), grid, block, 0, s, a); break;
+            case 8: hipLaunchKernelGGL((quant_wide_kernel<8>), grid, block, 0, s, a); break;
+            default: hipLaunchKernelGGL((quant_wide_kernel<10>), grid, block, 0, s, a); break;
         }
         return hipGetLastError();
     }

@@ -70,6 +70,15 @@ def test_act_quantize_without_value_outputs(hip, M, K):
     assert np.array_equal(_np(s), so) and np.array_equal(_np(q), qo)
 
 
+# the vectorised rows: each number of float4s per thread and the widths where it changes (1024,
+# 1536, 2560; few rows and more than 1024), part of a wave, part of the last float4 round, the
+# widest row, a block of 16 rows cut by M
+@pytest.mark.parametrize("M,K", [(3, 64), (17, 1024), (5, 1088), (9, 1536), (1030, 1536), (1030, 1600), (1025, 2560),
+                                 (1030, 2624), (1025, 6912), (33, 8192), (1040, 8192)])
+def test_act_quantize_widths(hip, M, K):
+    test_act_quantize_without_value_outputs(hip, M, K)
+
+
 @pytest.mark.parametrize("M,K", [(1, 6912), (4, 6912), (64, 6912), (2, 33)])
 def test_act_relu2_mul_quantize_bit_exact(hip, M, K):
     import torch
