@@ -553,6 +553,11 @@ __global__ void __launch_bounds__(PRO == 2 ? kAttnMaxThreads : 1024)
 // its 32 outputs (for an RMSNORM_SSQ prologue).  A workgroup waits only for its peers'
 // partials, which every peer stores before any wait of its own; the host allows the combine
 // only when the device holds the whole grid at once.
+// A wait that gave up: counted, and flagged in the host's memory.
+__device__ __forceinline__ void attn_gave_up(const AttnTail& at) {
+    __hip_atomic_fetch_add(at.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(at.err_host, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 template <int HD>
 __device__ __forceinline__ void attn_peer_combine(const AttnTail& at, int kh, int r, unsigned ep) {
     const int S = at.S, NC = at.Gq * HD / 32, P = S * (at.Gq / at.hpw);  // P: workgroups of a KV group
@@ -580,7 +585,7 @@ __device__ __forceinline__ void attn_peer_combine(const AttnTail& at, int kh, in
         }
         if (__all(ok)) break;
         if (it >= kAttnSpinLimit) {  // never expected: counted, and the launch goes on
-            if (t == 0) __hip_atomic_fetch_add(at.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (t == 0) attn_gave_up(at);
             break;
         }
         __builtin_amdgcn_s_sleep(1);
@@ -662,7 +667,7 @@ __device__ __forceinline__ void qkv_attn_block(const AttnTail& at, int total_rb)
                 w = __hip_atomic_load(at.tagged + g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 if (__all((unsigned)(w >> 32) == ep)) break;
                 if (++it > kAttnSpinLimit) {  // never expected: counted, and the launch goes on
-                    if ((threadIdx.x & 63) == 0) __hip_atomic_fetch_add(at.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if ((threadIdx.x & 63) == 0) attn_gave_up(at);
                     break;
                 }
                 __builtin_amdgcn_s_sleep(1);

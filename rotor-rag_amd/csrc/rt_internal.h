@@ -194,6 +194,7 @@ struct AttnTail {
     double* ssq;
     unsigned long long* ptag;
     int T;  // tiles per query head (attn_tiles(Lmax))
+    int* err_host;  // pinned host word, non-zero once err is: the check after a launch copies nothing
 };
 
 struct GemvShape {

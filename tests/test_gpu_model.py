@@ -749,6 +749,38 @@ def test_decode_attention_in_qkv_launch_bit_exact(hip):
     assert list(runs[0][1]) == list(runs[1][1])
 
 
+@pytest.mark.parametrize("Lmax", [96, 704])
+def test_forward_step_graph_equals_eager(hip, Lmax):
+    """The captured one-token step of BitNetModel.forward gives the eager step's logits (the
+    traced forward launches them one by one) and cache bit for bit: over several tokens, when
+    rewound, on another stream, and captured again after a switch of the launches changed."""
+    import torch
+
+    params = O.make_bitnet_params(23, WIDE16, Lmax)
+    model = _device_model(hip, params, WIDE16, Lmax)
+    dev = model._dev
+    _, c0 = model.forward(np.arange(3, 40, dtype=np.int32), return_logits=False, use_cache=True)
+
+    def steps(eager):
+        out, c = [], c0
+        for tok in (7, 11, 400):
+            dev.trace = {} if eager else None
+            lg, c = model.forward(np.array([tok], np.int32), past_kv_cache=c, use_cache=True)
+            out.append(lg)
+        dev.trace = None
+        return np.concatenate(out), c[1]["k"], c[1]["v"]
+
+    ref = steps(True)
+    same = lambda got: all(np.array_equal(a, b) for a, b in zip(ref, got))
+    assert same(steps(False)) and same(steps(False))
+    first = dev._step[1]
+    with torch.cuda.stream(torch.cuda.Stream()):
+        assert same(steps(False))
+    assert dev._step[1] is first
+    dev.attn_in_qkv = False  # a key of the capture (the plans of st[1] stay as built)
+    assert same(steps(False)) and dev._step[1] is not first
+
+
 def _embed32(params):
     E = params.get("_embed_f32")
     if E is None:
