@@ -37,6 +37,9 @@ from . import _hip
 TERNARY = ("q_proj", "k_proj", "v_proj", "o_proj", "gate_proj", "up_proj", "down_proj")
 
 
+_STAGE_BYTES = 8 << 20  # one of a model's two pinned staging buffers
+
+
 def rope_table(max_len: int, head_dim: int, theta: float) -> np.ndarray:
     """(cos, sin) of pos * theta^(-2i/head_dim), [max_len, head_dim/2, 2] fp32 (computed in f64)."""
     i = np.arange(head_dim // 2, dtype=np.float64)
@@ -214,6 +217,7 @@ class _DeviceModel:
         self.trace = None
         self._tbuf = None  # the trace's device buffers (allocated before any graph capture)
         self._step = None  # (switches, graph) of forward's one-token step
+        self._stage = None  # the pinned buffers of _to_host, freed with the model
         hip = self.hip = model.gpu
         dev = self.device = hip.device
         D, F, H, Hkv, hd = model.d_model, model.d_ff, model.n_heads, model.n_kv_heads, model.head_dim
@@ -562,7 +566,38 @@ class _DeviceModel:
         else:
             hn = self._final_norm(h)
             out = self._lm_head_all(hn) if return_logits else hn
-        return out.cpu().numpy()
+        return self._to_host(out)
+
+    def _to_host(self, t):
+        """t (device fp32) as a new host array.  Large results (every position's logits) go
+        through two pinned buffers of this model, each chunk copied on by the host's threads
+        while the next one arrives: a direct copy into fresh pageable memory faults its pages
+        in one by one (131 MB: 32 ms against 7)."""
+        import torch
+
+        step = _STAGE_BYTES // 4
+        if t.numel() <= step:
+            return t.cpu().numpy()
+        if self._stage is None:
+            self._stage = [torch.empty(step, dtype=torch.float32, pin_memory=True) for _ in range(2)]
+        src = t.contiguous().view(-1)
+        out = torch.empty(t.shape, dtype=torch.float32)
+        dst = out.view(-1)
+        parts = list(zip(src.split(step), dst.split(step)))
+        stream = torch.cuda.current_stream(self.device)
+        done = [torch.cuda.Event(), torch.cuda.Event()]
+
+        def fetch(i):
+            self._stage[i & 1][:parts[i][0].numel()].copy_(parts[i][0], non_blocking=True)
+            done[i & 1].record(stream)
+
+        fetch(0)
+        for i, (_, d) in enumerate(parts):
+            if i + 1 < len(parts):
+                fetch(i + 1)  # its buffer's previous chunk was copied on below
+            done[i & 1].synchronize()
+            d.copy_(self._stage[i & 1][:d.numel()])
+        return out.numpy()
 
     def _final_norm(self, h):
         import torch

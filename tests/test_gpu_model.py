@@ -781,6 +781,18 @@ def test_forward_step_graph_equals_eager(hip, Lmax):
     assert same(steps(False)) and dev._step[1] is not first
 
 
+@pytest.mark.parametrize("shape", [(1, 5), (2048, 1024), (2048, 1025), (5, 1 << 20), (3, 1999999)])
+def test_to_host_stages_large_results(small_model, shape):
+    """The staged copy to the host (8 MB chunks through two buffers): one chunk or less, one
+    element more, several, a short last one; a new array each time."""
+    import torch
+
+    dev = small_model[0]._dev
+    t = torch.randn(shape, device="cuda")
+    a, b = dev._to_host(t), dev._to_host(t * 2)
+    assert a.shape == shape and np.array_equal(a, t.cpu().numpy()) and np.array_equal(b, (t * 2).cpu().numpy())
+
+
 def _embed32(params):
     E = params.get("_embed_f32")
     if E is None:
