@@ -122,30 +122,38 @@ __global__ void __launch_bounds__(256) attention_kernel(const float* __restrict_
 // rate).  Workgroup (kv head kh, query block) owns 32 rows r = i G + g (query i of the
 // block, q-head g of the G = H / Hkv heads sharing kh); lane l of every wave works on row
 // l % 32.  Its 4 waves take the visible keys in blocks of 32, wave w blocks w, w + 4, ..,
-// each block staged in the wave's own LDS slice (K dimension-major as in the cache, V
-// key-major), with an online softmax per wave:
-//   S^T = K Q^T   (A = K[key][d] from LDS, B = Q^T from registers; the 128 dims are
-//                  taken in 64 steps pairing d = s and d = 64 + s over the lane halves)
+// with an online softmax per wave:
+//   S^T = K Q^T   (A = K[key][d], B = Q^T, both in registers; the 128 dims are taken in 64
+//                  steps pairing d = s and d = 64 + s over the lane halves)
 //   P^T = e^(S^T scale - m) per row, rows are lanes, so max and sum need one
 //                  lane-half exchange
-//   O^T += V^T P^T (A = V^T from LDS, B = P^T straight from the S^T registers: the
-//                  MFMA output layout puts keys 8 (r / 4) + 4 (l / 32) + r % 4 of the
-//                  lane's row in register r, and step r pairs exactly those keys)
+//   O^T += V^T P^T (A = V^T, B = P^T straight from the S^T registers: the MFMA output
+//                  layout puts keys 8 (r / 4) + 4 (l / 32) + r % 4 of the lane's row in
+//                  register r, and step r pairs exactly those keys)
 // The 4 waves' (m, l, O) are merged through LDS at the end.  fp32 products, fp32 sums in
 // the matrix cores' order.
+// K and V go from memory to registers 16 at a time, so a wave needs no LDS slice and 210
+// registers: two workgroups share a CU and one's softmax, waits and merge run under the
+// other's MFMAs (with K and V in LDS, 32 KiB a wave, each SIMD had one wave).  Before / now, 20
+// heads of 128 over 5: 1024 tokens after 1024 228 -> 199 us (matrix cores busy 74 % of the CUs'
+// cycles), 512 / 256 / 64 tokens from an empty cache 32.5 / 19.7 / 11.7 -> 30.2 / 15.1 / 9.0, 2
+// tokens after 1400 70 -> 56; V by one 16-byte load for the four blocks of O^T instead of four
+// 4-byte ones 207 -> 199.
+typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(3))) void lds_void;
 
 template <int HD>
-__global__ void __launch_bounds__(256) attn_prefill_mfma_kernel(const float* __restrict__ q,
+__global__ void __launch_bounds__(256, 2) attn_prefill_mfma_kernel(const float* __restrict__ q,
                                                                 const float* __restrict__ Kc,
                                                                 const float* __restrict__ Vc, float* __restrict__ out,
                                                                 int M, int H, int Hkv, int Lmax,
                                                                 const int* __restrict__ pos_p, float scale) {
     static_assert(HD == 128, "two 64-dim halves per lane");
-    constexpr int BK = 32, SLICE = HD * BK * 2;  // floats per wave: K [HD][BK], V [BK][HD]
+    constexpr int BK = 32, OLD = HD + 1, SLICE = OLD * 32;  // merge: [32 rows][HD] per wave, rows padded by a word
     extern __shared__ __attribute__((aligned(16))) float lds_pf[];
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, row = lane & 31, hl = lane >> 5;
+    const int t = threadIdx.x, lane = t & 63, row = lane & 31, hl = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int G = H / Hkv, BQ = 32 / G;
     // the last query blocks see the most keys: they go out first, so that the short ones
     // fill in behind them when the grid takes more than one round of workgroups
@@ -155,8 +163,6 @@ __global__ void __launch_bounds__(256) attn_prefill_mfma_kernel(const float* __r
     const int lastpos = m < M ? pos0 + m : -1;     // keys <= lastpos visible to this row
     const int kend = pos0 + min(i0 + BQ, M);       // keys [0, kend) visible to some row
     const int nblk = (kend + BK - 1) / BK;
-    float* Ks = lds_pf + wave * SLICE;
-    float* Vs = Ks + HD * BK;
     // this lane's half of its row of Q: dims 64 hl .. 64 hl + 63
     float qr[64];
     {
@@ -174,54 +180,47 @@ __global__ void __launch_bounds__(256) attn_prefill_mfma_kernel(const float* __r
 #pragma unroll
     for (int nb = 0; nb < HD / 32; ++nb) o[nb] = v16f{};
     float mrow = -INFINITY, lrow = 0.0f;
-    const float* K = Kc + (size_t)kh * HD * Lmax;
-    const float* V = Vc + (size_t)kh * Lmax * HD;
-    // K and V blocks go global -> LDS directly (buffer loads with an LDS destination, range
-    // checked per head: keys past Lmax read as zeros).  A block's K loads are issued as
-    // soon as the previous block's K operands have been read out of the slice, its V loads
-    // as soon as the previous V operands have: each has a whole block of MFMAs to land.
-    // Keys past kend are masked below.
-    const __amdgpu_buffer_rsrc_t krs =
-        __builtin_amdgcn_make_buffer_rsrc((void*)K, 0, (unsigned)(HD * Lmax * 4), kBufDword3);
-    const __amdgpu_buffer_rsrc_t vrs =
-        __builtin_amdgcn_make_buffer_rsrc((void*)V, 0, (unsigned)(HD * Lmax * 4), kBufDword3);
-    constexpr int kBlkLoads = HD * BK / 4 / 64;  // 16-byte loads per lane per block (16)
-    auto load_k = [&](int key0) {  // Ks[d][j] = K[d][key0 + j], 8 dims per load
+    // The MFMA operands come straight from memory, 16 registers a chunk: the block's K as four
+    // chunks of 16 dims a lane half, its V as four chunks of 4 keys a lane half, each requested
+    // while the chunk before it is multiplied (two register sets).  K: dim 64 hl + st of key
+    // key0 + row; keys past Lmax re-read its last one (masked below).  V: dims 4 row .. 4 row + 3
+    // of a key in one load, one for each block of O^T (block nb: dims 4 d + nb); keys past kend
+    // lie outside the buffer and read as zeros.
+    const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(Kc + (size_t)kh * HD * Lmax), 0, (unsigned)(HD * Lmax * 4), kBufDword3);
+    const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(Vc + (size_t)kh * Lmax * HD), 0, (unsigned)(min(kend, Lmax) * HD * 4), kBufDword3);
+    const int Lrow = Lmax * 4;
+    float buf[2][16];
+    auto load_k = [&](float (&x)[16], int key0, int c) {
+        const int off = 64 * hl * Lrow + 4 * min(key0 + row, Lmax - 1);
 #pragma unroll
-        for (int it = 0; it < kBlkLoads; ++it) {
-            const int d = 8 * it + (lane >> 3), j = 4 * (lane & 7);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(krs, (lds_void*)(Ks + 256 * it), 16, (d * Lmax + key0 + j) * 4, 0,
-                                                     0, 0);
+        for (int i = 0; i < 16; ++i)
+            x[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(krs, off, (16 * c + i) * Lrow, 0));
+    };
+    auto load_v = [&](float (&x)[16], int key0, int c) {
+        const int off = ((key0 + 8 * c + 4 * hl) * HD + 4 * row) * 4;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const v4f z = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(vrs, off + i * HD * 4, 0, 0));
+#pragma unroll
+            for (int j = 0; j < 4; ++j) x[4 * i + j] = z[j];
         }
     };
-    auto load_v = [&](int key0) {  // Vs[j][d] = V[key0 + j][d], 2 keys per load
-#pragma unroll
-        for (int it = 0; it < kBlkLoads; ++it) {
-            const int j = 2 * it + (lane >> 5), dq = 4 * (lane & 31);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(vrs, (lds_void*)(Vs + 256 * it), 16, ((key0 + j) * HD + dq) * 4, 0,
-                                                     0, 0);
-        }
-    };
-    if (wave < nblk) {
-        load_k(wave * BK);
-        load_v(wave * BK);
-    }
+    if (wave < nblk) load_k(buf[0], wave * BK, 0);
     for (int b = wave; b < nblk; b += 4) {
         const int key0 = b * BK;
-        const bool more = b + 4 < nblk;
-        // this block's K has landed (its V may still be in flight)
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kBlkLoads) : "memory");
-        // S^T[key][row]; the 64 A operands are read from LDS ahead of the MFMA chain (read
-        // one by one in front of each MFMA, every pair of MFMAs would wait for the LDS)
-        float ka[64];
-#pragma unroll
-        for (int st = 0; st < 64; ++st) ka[st] = Ks[(64 * hl + st) * BK + row];
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // K slice read out: refill it
-        if (more) load_k((b + 4) * BK);
-        __builtin_amdgcn_sched_barrier(0);  // keep the reads and loads ahead of the chain
         v16f sacc = v16f{};
 #pragma unroll
-        for (int st = 0; st < 64; ++st) sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(ka[st], qr[st], sacc, 0, 0, 0);
+        for (int c = 0; c < 4; ++c) {
+            if (c < 3) load_k(buf[(c + 1) & 1], key0, c + 1);
+            else load_v(buf[0], key0, 0);
+            __builtin_amdgcn_sched_barrier(0);  // the requests ahead of the chain
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(buf[c & 1][i], qr[16 * c + i], sacc, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         float pr[16];
         float mx = -INFINITY;
 #pragma unroll
@@ -242,34 +241,29 @@ __global__ void __launch_bounds__(256) attn_prefill_mfma_kernel(const float* __r
         ls += __shfl_xor(ls, 32, 64);
         lrow = lrow * alpha + ls;
         mrow = mnew;
-        // this block's V has landed (the next block's K may still be in flight)
-        if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kBlkLoads) : "memory");
-        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        // O^T[dim][row] = alpha O^T + V^T P^T (A operands read ahead, as above)
-        float va[HD / 32][16];
+        // O^T[dim][row] = alpha O^T + V^T P^T
 #pragma unroll
-        for (int nb = 0; nb < HD / 32; ++nb)
+        for (int nb = 0; nb < HD / 32; ++nb) o[nb] *= alpha;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) va[nb][r] = Vs[(8 * (r >> 2) + 4 * hl + (r & 3)) * HD + 32 * nb + row];
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // V slice read out: refill it
-        if (more) load_v((b + 4) * BK);
-        __builtin_amdgcn_sched_barrier(0);
+        for (int c = 0; c < 4; ++c) {
+            if (c < 3) load_v(buf[(c + 1) & 1], key0, c + 1);
+            else if (b + 4 < nblk) load_k(buf[0], key0 + 4 * BK, 0);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int nb = 0; nb < HD / 32; ++nb) {
-            v16f acc = o[nb] * alpha;
+            for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(va[nb][r], pr[r], acc, 0, 0, 0);
-            o[nb] = acc;
+                for (int nb = 0; nb < HD / 32; ++nb)
+                    o[nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(buf[c & 1][4 * i + nb], pr[4 * c + i], o[nb], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
-    // merge the waves: slice w becomes [32 rows][HD] of O^T, then (m, l) per row
-    __syncthreads();
+    // merge the waves: slice w holds [32 rows][HD] of O^T, then (m, l) per row
     float* Om = lds_pf + wave * SLICE;
     float* ml = lds_pf + 4 * SLICE;  // [4 waves][32 rows][2]
 #pragma unroll
     for (int nb = 0; nb < HD / 32; ++nb)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) Om[row * HD + 32 * nb + 8 * (r >> 2) + 4 * hl + (r & 3)] = o[nb][r];
+        for (int r = 0; r < 16; ++r) Om[row * OLD + 4 * (8 * (r >> 2) + 4 * hl + (r & 3)) + nb] = o[nb][r];
     if (hl == 0) {
         ml[(wave * 32 + row) * 2] = mrow;
         ml[(wave * 32 + row) * 2 + 1] = lrow;
@@ -295,7 +289,7 @@ __global__ void __launch_bounds__(256) attn_prefill_mfma_kernel(const float* __r
     for (int e = 0; e < HD / 8; ++e) {
         float num = 0.0f;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) num += fw[w] * lds_pf[w * SLICE + orow * HD + d0 + e];
+        for (int w = 0; w < 4; ++w) num += fw[w] * lds_pf[w * SLICE + orow * OLD + d0 + e];
         dst[e] = num / den;
     }
 }
@@ -467,7 +461,6 @@ __global__ void __launch_bounds__(256) lm_head_kernel(const uint16_t* __restrict
     }
 }
 
-typedef float v4f __attribute__((ext_vector_type(4)));
 
 // token = argmax; optionally also written to next_ids[0] (the next step's input) and,
 // with p = *pos_p + advance, to out_tokens[p - 1 - pos_base]; then *pos_p = p.  With
@@ -545,7 +538,7 @@ hipError_t launch_rope_append(float* q, float* k, const float* v, float* Kc, flo
 
 // the matrix-core prefill attention's LDS (above 64 KiB: allowed once per device, at
 // context creation, so that no launch makes a function-attribute call)
-constexpr size_t kAttnPrefillLds = (size_t)(4 * 128 * 32 * 2 + 4 * 32 * 2) * sizeof(float);
+constexpr size_t kAttnPrefillLds = (size_t)(4 * 129 * 32 + 4 * 32 * 2) * sizeof(float);
 
 hipError_t model_prepare_device() {
     return hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_prefill_mfma_kernel<128>),
