@@ -74,7 +74,10 @@ def test_act_quantize_without_value_outputs(hip, M, K):
 # 1536, 2560; few rows and more than 1024), part of a wave, part of the last float4 round, the
 # widest row, a block of 16 rows cut by M
 @pytest.mark.parametrize("M,K", [(3, 64), (17, 1024), (5, 1088), (9, 1536), (1030, 1536), (1030, 1600), (1025, 2560),
-                                 (1030, 2624), (1025, 6912), (33, 8192), (1040, 8192)])
+                                 (1030, 2624), (1025, 6912), (33, 8192), (1040, 8192),
+                                 # no multiple of 64: element by element (or whole float4s of a ragged row)
+                                 (3, 1), (5, 63), (20, 1023), (100, 2050), (7, 2564), (1030, 2561), (1025, 6911),
+                                 (3, 8191)])
 def test_act_quantize_widths(hip, M, K):
     test_act_quantize_without_value_outputs(hip, M, K)
 
