@@ -50,11 +50,14 @@ class TernaryFFNBlock:
     def load(self, norm_weight, gate, up, down):
         """gate/up/down: (rotor bytes [out, ceil(in/4)], scale) each."""
         self.norm.weight = np.asarray(norm_weight, dtype=np.float32)
-        self.gate_proj.load_from_bitnet(*gate)
-        self.up_proj.load_from_bitnet(*up)
-        self.down_proj.load_from_bitnet(*down)
         self._state.clear()
         self._gu = self._pair = None
+        if self.use_gpu and self.pair_ok:
+            self._load_pair(gate, up)
+        else:
+            self.gate_proj.load_from_bitnet(*gate)
+            self.up_proj.load_from_bitnet(*up)
+        self.down_proj.load_from_bitnet(*down)
         if self.use_gpu:
             import torch
 
@@ -62,17 +65,19 @@ class TernaryFFNBlock:
             self._acts = (self.gpu.activations(self.max_tokens, self.d_model),
                           self.gpu.activations(self.max_tokens, self.d_ff))
 
-    def _gate_up(self):
-        """The interleaved gate/up matrix (HIPTernaryOps.interleave_gate_up's layout) and its
-        scales, laid out on the device from the rotor bytes the layers were loaded with."""
-        if self._gu is None:
-            import torch
+    def _load_pair(self, gate, up):
+        """Gate and up from one copy of their bytes on the device: the two matrices and the
+        interleaved one (HIPTernaryOps.interleave_gate_up's layout)."""
+        import torch
 
-            dev, D, F = self.gpu.device, self.d_model, self.d_ff
-            g, u = (torch.from_numpy(p._packed).to(dev).view(F // 32, 32, -1) for p in (self.gate_proj, self.up_proj))
-            self._gu = (self.gpu.upload_device(torch.stack([g, u], dim=1).view(2 * F, -1), D, 1.0),
-                        (self.gate_proj.scale, self.up_proj.scale))
-        return self._gu
+        dev, D, F = self.gpu.device, self.d_model, self.d_ff
+        halves = []
+        for proj, (packed, scale) in ((self.gate_proj, gate), (self.up_proj, up)):
+            proj._set_packed(packed, scale)
+            halves.append(torch.from_numpy(proj._packed).to(dev))
+            proj._set_device(self.gpu.upload_device(halves[-1], D, proj.scale))
+        gu = torch.stack([h.view(F // 32, 32, -1) for h in halves], dim=1).view(2 * F, -1)
+        self._gu = (self.gpu.upload_device(gu, D, 1.0), (self.gate_proj.scale, self.up_proj.scale))
 
     def _buffers(self, M):
         st = self._state.get(M)
@@ -85,7 +90,7 @@ class TernaryFFNBlock:
             act_h = self._acts[0]
             u = None
             if M > 64 and self.pair_ok:
-                w_gu, scales = self._gate_up()
+                w_gu, scales = self._gu
                 plan = self.gpu.plan_act_gate_up(w_gu, scales, act_h, M, g)
             else:
                 u = torch.empty((M, self.d_ff), dtype=torch.float32, device=dev)
@@ -103,7 +108,7 @@ class TernaryFFNBlock:
             from . import _hip
 
             hip, dev = self.gpu, self.gpu.device
-            w_gu, scales = self._gate_up()
+            w_gu, scales = self._gu
             a = torch.empty(self.d_ff, dtype=torch.float32, device=dev)
             ssq = torch.empty(self.d_ff // 32, dtype=torch.float64, device=dev)
             y = torch.empty((1, self.d_model), dtype=torch.float32, device=dev)

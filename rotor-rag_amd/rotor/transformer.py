@@ -87,6 +87,11 @@ class TernaryLinear:
     def load_from_bitnet(self, packed_weights: np.ndarray, scale: float = 1.0):
         """Load rotor/BitNet bytes [out_features, ceil(in_features/4)] (uint8) and a
         per-tensor scale (src/rotor/transformer.py:77-109)."""
+        self._set_packed(packed_weights, scale)
+        if self.gpu is not None and self.use_gpu:
+            self._set_device(self.gpu.upload(self._packed, self.in_features, self.scale))
+
+    def _set_packed(self, packed_weights: np.ndarray, scale: float):
         p = np.ascontiguousarray(packed_weights, dtype=np.uint8)
         if p.ndim != 2 or p.shape[0] != self.out_features or p.shape[1] * 4 < self.in_features:
             raise ValueError(f"packed weights of shape {p.shape} do not fit "
@@ -96,9 +101,10 @@ class TernaryLinear:
         self._packed = p
         self._planes = None
         self._weights_cache = None
-        if self.gpu is not None and self.use_gpu:
-            self.gpu_packed_weights = self.gpu.upload(p, self.in_features, self.scale)
-            self.gpu_scales = np.full(self.out_features, self.scale, dtype=np.float32)
+
+    def _set_device(self, weights):
+        self.gpu_packed_weights = weights
+        self.gpu_scales = np.full(self.out_features, self.scale, dtype=np.float32)
 
     def forward(self, x):
         """y = x @ W.T * scale for x [batch, seq, in] or [seq, in] (src/rotor/transformer.py:111-155).
