@@ -200,8 +200,10 @@ struct rt_act {
     void* mem = nullptr;
 };
 
-// Rows the matrix kernels read for M tokens: one (GEMV), or GEMM tile rows.
-static int act_rows(int M) { return M > kGemvMaxM ? round_up(M, gemm_bm(M)) : M; }
+// Rows the matrix kernels read for M tokens: one (GEMV), a small block, or GEMM tile rows.
+static int act_rows(int M) {
+    return M <= kGemvMaxM ? M : M <= kSkinnyRows ? qx_block_rows(M) : round_up(M, gemm_bm(M));
+}
 
 extern "C" {
 
@@ -364,7 +366,7 @@ static int check_act(const rt_ctx* ctx, int M, int K, const char* who) {
 }
 
 // Quantise (x != NULL) or permute (q_in != NULL) M rows of K into the context scratch.
-static int stage_activations(rt_ctx* ctx, const float* x, const int8_t* q_in, int M, int K, int Mpad, bool blocked,
+static int stage_activations(rt_ctx* ctx, const float* x, const int8_t* q_in, int M, int K, int Mpad, int blocked,
                              int8_t* q_nat, float* s_out, int8_t** qx, float** sx) {
     const int Kp = round_up(K, kChunk);
     const size_t qbytes = (size_t)Mpad * Kp;

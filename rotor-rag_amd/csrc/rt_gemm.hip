@@ -687,7 +687,9 @@ __global__ void __launch_bounds__(kRegThreads) gemm_region_kernel(GemmGroupArgs 
 // With v_mfma_i32_16x16x64_i8 and K assigned to lanes so that every load is 16 bytes a lane:
 // lane l owns column l % 16 of each 16-column block and chunk 4 q + l / 16 of quad q, whose 16
 // bytes of code are the B operands of the quad's four MFMA steps (one dword each); the A
-// operand of step i is the 16-byte group i of the same chunk of row l % 16.  Both operands
+// operand of step i is the 16-byte group i of the same chunk of row l % 16 (in blocks of
+// qx_block_rows rows; the step's part of the address is the unchecked scalar offset, which
+// never leaves a chunk in range).  Both operands
 // use that assignment of k, so the int32 sums are exact.  B holds the device code g = w + 1
 // itself, four fields masked out of a dword (7 VALU operations; expanding to w takes 11), and
 // one more MFMA a step against ones gives sum x, subtracted at the end.  Chunks past C read as
@@ -698,7 +700,7 @@ __global__ void __launch_bounds__(kRegThreads) gemm_region_kernel(GemmGroupArgs 
 // workgroup, M <= 8, and the split-K kernel below): the seven projections of a 2560 / 6912
 // layer at M = 5 28.2 -> 9.9 us; q/k/v at M = 5 / 16 12.1 / 7.2 -> 4.4 / 4.8; down 17.1 / 12.5
 // -> 6.0 / 6.3; 64 matrices of 6912 x 2560 (283 MB) at M = 2 / 3 51.1 / 63.4 -> 48.3 / 49.4.
-constexpr int kSkinnyLd = 68;
+constexpr int kSkinnyLd = 68, kSkinnyLds = 16 * 16 * kSkinnyLd * 4;  // (at most 16 / MB waves)
 template <int MB, bool NT>
 __global__ void __launch_bounds__(1024 / MB) gemm_skinny_kernel(GemmGroupArgs ga, int xcd) {
     extern __shared__ __attribute__((aligned(16))) v4u lds[];
@@ -712,16 +714,17 @@ __global__ void __launch_bounds__(1024 / MB) gemm_skinny_kernel(GemmGroupArgs ga
     const int q1 = __builtin_amdgcn_readfirstlane(((wave + 1) * Q) / nw);
     const __amdgpu_buffer_rsrc_t wr =
         __builtin_amdgcn_make_buffer_rsrc((void*)(a.w + (size_t)rb * C * kRowBlock), 0, C * 1024, kBufDword3);
+    const int B = MB == 1 ? qx_block_rows(a.M) : 16;  // rows of an activation block
     __amdgpu_buffer_rsrc_t ar[MB];
 #pragma unroll
     for (int b = 0; b < MB; ++b)
-        ar[b] = __builtin_amdgcn_make_buffer_rsrc((void*)(a.qx + (size_t)b * C * 1024), 0, C * 1024, kBufDword3);
+        ar[b] = __builtin_amdgcn_make_buffer_rsrc((void*)(a.qx + (size_t)b * C * 1024), 0, C * 64 * B, kBufDword3);
     // rows past the tokens read as zeros too, from past the buffer: no traffic for them (for 2
     // tokens, each XCD would otherwise read 14 rows of padding of every problem)
     const int off = h4 * 1024 + c16 * 16;
     int aoff[MB];
 #pragma unroll
-    for (int b = 0; b < MB; ++b) aoff[b] = 16 * b + c16 < a.M ? off : (int)0x80000000;
+    for (int b = 0; b < MB; ++b) aoff[b] = 16 * b + c16 < a.M ? h4 * 64 * B + c16 * 16 : (int)0x80000000;
     struct Quad {
         v4u w[4];       // column block j
         v4i x[MB][4];   // row block b, step i
@@ -735,7 +738,7 @@ __global__ void __launch_bounds__(1024 / MB) gemm_skinny_kernel(GemmGroupArgs ga
         for (int b = 0; b < MB; ++b)
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                z.x[b][i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(ar[b], aoff[b] + q * 4096 + i * 256, 0, 0));
+                z.x[b][i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(ar[b], aoff[b] + q * 256 * B, i * 16 * B, 0));
     };
     v4i acc[MB][4];
 #pragma unroll
@@ -1100,6 +1103,10 @@ static hipError_t allow_tile_lds() {
 
 hipError_t gemm_prepare_device() {
     hipError_t e = allow_lds(&gemm_splitk_kernel<kSplitkWaves, 4>, splitk_lds<kSplitkWaves, 4>());
+    if (e == hipSuccess) e = allow_lds(&gemm_skinny_kernel<1, false>, kSkinnyLds);
+    if (e == hipSuccess) e = allow_lds(&gemm_skinny_kernel<1, true>, kSkinnyLds);
+    if (e == hipSuccess) e = allow_lds(&gemm_skinny_kernel<2, false>, kSkinnyLds);
+    if (e == hipSuccess) e = allow_lds(&gemm_skinny_kernel<2, true>, kSkinnyLds);
     if (e == hipSuccess) e = allow_lds(&gemm_region_kernel<kRegS>, 2 * kRegS * kRegStage);
     if (e == hipSuccess) e = allow_tile_lds<128, 128, 2, 4>();
     if (e == hipSuccess) e = allow_tile_lds<256, 128, 2, 4>();

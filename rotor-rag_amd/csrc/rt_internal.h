@@ -96,7 +96,7 @@ struct QuantProb {
     float* v_out;        // optional fp32 [M][K]: the values that were quantised
     const float* aux2;   // norm_w [K] (kRelu2MulNorm)
     int attn_S, attn_hd; // kAttnNorm: partial blocks per head, head dimension
-    int blocked;         // qx layout: 0 rows, 1 blocked (see qx_blocked)
+    int blocked;         // qx layout: 0 rows, else the rows of a block (see qx_blocked)
 };
 
 // ---- one GEMV problem (a ternary matrix applied to M tokens) -------------------
@@ -316,14 +316,16 @@ constexpr int kSkinnyRows = 8, kSkinnyOneRound = 256;
 inline bool skinny_ok(int M, int units, bool split) {
     return M <= kSkinnyRows || (!split && (M <= 16 || (M <= 32 && units <= kSkinnyOneRound)));
 }
-// qx layout.  Rows (M <= kGemvMaxM, read by the GEMV): row m at m * Kp.  Blocked
-// (M > kGemvMaxM, read by the MFMA GEMM): 16-row x 64-k blocks of 1 KiB, block
-// (m / 16, c) at (m / 16 * C + c) * 1024, where the 16-byte group q (k = 16 q .. 16 q + 15
-// of chunk c) of row m sits at ((m % 16) + 16 q) * 16: the block is laid out as the
-// matrix-core operand fragments, so the GEMM copies it to LDS with contiguous loads.
-inline bool qx_blocked(int M) { return M > kGemvMaxM; }
+// qx layout.  Rows (M <= kGemvMaxM, read by the GEMV): row m at m * Kp.  Blocked (beyond, read by
+// the MFMA GEMMs): blocks of B = qx_block_rows(M) rows x 64 k, block (m / B, c) at
+// (m / B * C + c) * 64 B, where the 16-byte group q (k = 16 q .. 16 q + 15 of chunk c) of row m
+// sits at ((m % B) + B q) * 16.  With B = 16 a 1 KiB block is laid out as the matrix-core operand
+// fragments, so the GEMM copies it to LDS with contiguous loads; up to 8 tokens take 2, 4 or 8
+// rows (gemm_skinny_kernel), so that a static buffer holds rows of millions.
+inline __host__ __device__ int qx_block_rows(int M) { return M <= 2 ? 2 : M <= 4 ? 4 : M <= kSkinnyRows ? 8 : 16; }
+inline int qx_blocked(int M) { return M > kGemvMaxM ? qx_block_rows(M) : 0; }
 
-// rows of the GEMM workgroup tile for M tokens (the activations are zero-padded to it)
+// rows of the GEMM workgroup tile for M tokens (the activations are padded to it past 8 tokens)
 inline int gemm_bm(int M) { return M <= kSkinnyRows ? 16 : M <= 64 ? 64 : M <= 128 ? 128 : 256; }
 // The GEMM epilogues address one row tile of the output (and residual) with 32-bit byte
 // offsets and buffer ranges: a tile of gemm_bm(M) rows of ldo floats must span < 2^31 bytes.
@@ -340,7 +342,7 @@ hipError_t launch_unrelayout(const v4u* tiles, int N, int K, uint8_t* dst, hipSt
 hipError_t launch_quant(const QuantArgs& a, hipStream_t s, int maxK = 0);
 bool quant_rows_ok(const QuantProb& P);
 // qx rows [M][Kp] (permuted) -> natural-order int8 [M][K]
-hipError_t launch_unpermute(const int8_t* qx, int M, int K, int Kp, bool blocked, int8_t* q, hipStream_t s);
+hipError_t launch_unpermute(const int8_t* qx, int M, int K, int Kp, int blocked, int8_t* q, hipStream_t s);
 // One token (M = 1).
 hipError_t launch_gemv(const GemvArgs& a, GemvShape shape, hipStream_t s);
 hipError_t launch_gemm(const GemmArgs& a, hipStream_t s);

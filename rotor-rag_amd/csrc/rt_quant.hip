@@ -18,14 +18,20 @@ namespace rt {
 
 __device__ __forceinline__ QuantProb select_quant(const QuantArgs& a, int i) { return a.dev ? a.dev[i] : a.p; }
 
+// row m of problem P's activations in their layout (qx_blocked)
+__device__ __forceinline__ QxRow qx_row(const QuantProb& P, v4u* qx, int m) {
+    const int B = P.blocked;
+    if (B == 0) return QxRow{qx + (size_t)m * (P.Kp >> 4), 4, 1};
+    return QxRow{qx + (size_t)(m / B) * (P.Kp >> 6) * (4 * B) + m % B, 4 * B, B};
+}
+
 __global__ void __launch_bounds__(256) quant_kernel(QuantArgs a) {
     __shared__ RowSmem sm;
     const QuantProb P = select_quant(a, blockIdx.y);
     const int m = blockIdx.x;
     const int K = P.K, Kp = P.Kp, groups = Kp >> 4;
     v4u* const qx = reinterpret_cast<v4u*>(P.qx);
-    const QxRow qrow = P.blocked ? QxRow{qx + (size_t)(m >> 4) * (Kp >> 6) * 64 + (m & 15), 64, 16}
-                                 : QxRow{qx + (size_t)m * (Kp >> 4), 4, 1};
+    const QxRow qrow = qx_row(P, qx, m);
     if (P.mode == kPermute) {  // int8 in natural order -> qx
         const int8_t* qr = P.q_in + (size_t)m * K;
         for (int g = threadIdx.x; g < groups; g += blockDim.x) {
@@ -140,8 +146,7 @@ __global__ void __launch_bounds__(NV == 4 ? 512 : 256) quant_wide_kernel(QuantAr
     if (t == 0 && P.sx) P.sx[m] = sc;
     const double rs = 1.0 / (double)sc;  // as scatter_q
     v4u* const qx = reinterpret_cast<v4u*>(P.qx);
-    const QxRow qrow = P.blocked ? QxRow{qx + (size_t)(m >> 4) * (P.Kp >> 6) * 64 + (m & 15), 64, 16}
-                                 : QxRow{qx + (size_t)m * (P.Kp >> 4), 4, 1};
+    const QxRow qrow = qx_row(P, qx, m);
     const bool odd = t & 1, high = t & 2;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
@@ -167,14 +172,15 @@ __global__ void __launch_bounds__(256) unpermute_kernel(const int8_t* __restrict
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= K) return;
     const int g = k >> 4, e = k & 15;  // element e of group g sits at byte 4*(e%4) + e/4
-    const size_t group = blocked ? ((size_t)(m >> 4) * (Kp >> 6) + (g >> 2)) * 1024 + ((m & 15) + 16 * (g & 3)) * 16
-                                 : (size_t)m * Kp + g * 16;
+    const int B = blocked;
+    const size_t group = B ? ((size_t)(m / B) * (Kp >> 6) + (g >> 2)) * (64 * B) + (m % B + B * (g & 3)) * 16
+                           : (size_t)m * Kp + g * 16;
     q[(size_t)m * K + k] = qx[group + 4 * (e & 3) + (e >> 2)];
 }
 
-hipError_t launch_unpermute(const int8_t* qx, int M, int K, int Kp, bool blocked, int8_t* q, hipStream_t s) {
+hipError_t launch_unpermute(const int8_t* qx, int M, int K, int Kp, int blocked, int8_t* q, hipStream_t s) {
     hipLaunchKernelGGL(unpermute_kernel, dim3((unsigned)((K + 255) / 256), (unsigned)M), dim3(256), 0, s, qx, K, Kp,
-                       (int)blocked, q);
+                       blocked, q);
     return hipGetLastError();
 }
 

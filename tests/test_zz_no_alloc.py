@@ -74,6 +74,28 @@ def test_noalloc_rejects_inputs_beyond_the_buffer(hip):
     assert lib.rt_linear_f32_noalloc(hip.ctx, w.handle, None, 1, None) == RT_EINVAL
 
 
+@pytest.mark.parametrize("M,K", [(2, 1 << 22), (8, 2000000), (3, 2000000), (4, 4000000)])
+def test_noalloc_few_tokens_of_long_rows(hip, M, K):
+    """Up to 8 tokens take 2, 4 or 8 rows of the static buffer, so rows of millions fit; exact
+    against the int64 sums."""
+    import torch
+
+    from rotor import _hip
+
+    lib = _hip.load()
+    rng = np.random.default_rng(M)
+    N = 3
+    W = rng.choice(np.array([-1, 0, 1], np.int8), size=(N, K))
+    w = hip.upload(O.pack_rotor(W), K, 0.5)
+    x = rng.standard_normal((M, K), dtype=np.float32)
+    hip._bind_stream()
+    rc, y = _run(lib, hip.ctx, lib.rt_linear_f32_noalloc, w, torch.from_numpy(x).cuda(), N)
+    assert rc == RT_OK, _hip.last_error()
+    q, s = O.quant_rows(x)
+    acc = q.astype(np.int64) @ W.astype(np.int64).T
+    assert np.array_equal(y.cpu().numpy(), (acc.astype(np.float32) * s[:, None]) * np.float32(0.5))
+
+
 # The allocation-free call captured in a HIP graph: every replay, each on a new input written
 # in place between replays (with the process's own eager launches and synchronisations in
 # between), equals the eager rt_linear_f32 bit for bit.  The child process captures each
