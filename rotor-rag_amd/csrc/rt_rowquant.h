@@ -195,8 +195,8 @@ __device__ __forceinline__ void rmsnorm_group(const QuantProb& P, float norm, in
 }
 
 // Destination of one row's permuted 16-byte groups: group g at
-// base[(g / 4) * chunk + (g % 4) * sub] (v4u units); rows: chunk 4, sub 1; blocked qx:
-// chunk 64, sub 16.
+// base[(g / 4) * chunk + (g % 4) * sub] (v4u units); rows: chunk 4, sub 1; blocks
+// of B rows: chunk 4 B, sub B.
 struct QxRow {
     v4u* base;
     int chunk, sub;
