@@ -136,6 +136,34 @@ def test_rope_append_and_attention(hip, M, pos0, H, Hkv, hd, Lmax):
     assert torch.equal(out, out2)
 
 
+# A workgroup takes 1024 pairs: exactly one for q, one and a pair, several with a ragged end,
+# and more than one pass over k; tokens that do and do not divide over the XCDs
+@pytest.mark.parametrize("M,pos0,H,Hkv,hd", [(1, 3, 16, 4, 128), (9, 0, 1025, 1, 2), (8, 5, 36, 36, 64),
+                                             (17, 2, 20, 20, 256), (3, 60, 1, 1, 2)])
+def test_rope_append_parts(hip, M, pos0, H, Hkv, hd):
+    import torch
+
+    lib, chk = _lib()
+    rng = np.random.default_rng(M)
+    Lmax = 64
+    table = O.rope_table(Lmax, hd, 500000.0)
+    q, k, v = (rng.standard_normal((M, n * hd)).astype(np.float32) for n in (H, Hkv, Hkv))
+    qd, kd, vd, td = (torch.from_numpy(a).cuda() for a in (q, k, v, np.ascontiguousarray(table)))
+    kc = torch.full((Hkv, hd, Lmax), 7.0, device="cuda")
+    vc = torch.full((Hkv, Lmax, hd), 7.0, device="cuda")
+    pos = torch.tensor([pos0], dtype=torch.int32, device="cuda")
+    hip._bind_stream()
+    chk(lib.rt_rope_kv_append(hip.ctx, qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), kc.data_ptr(), vc.data_ptr(),
+                              td.data_ptr(), M, H, Hkv, hd, Lmax, pos.data_ptr()))
+    kr = O.apply_rope(k.reshape(M, Hkv, hd), table, pos0)
+    assert np.array_equal(qd.cpu().numpy().reshape(M, H, hd), O.apply_rope(q.reshape(M, H, hd), table, pos0))
+    assert np.array_equal(kd.cpu().numpy().reshape(M, Hkv, hd), kr)
+    K, V = np.full((Hkv, hd, Lmax), 7.0, np.float32), np.full((Hkv, Lmax, hd), 7.0, np.float32)
+    K[:, :, pos0:pos0 + M] = kr.transpose(1, 2, 0)
+    V[:, pos0:pos0 + M] = v.reshape(M, Hkv, hd).transpose(1, 0, 2)
+    assert np.array_equal(kc.cpu().numpy(), K) and np.array_equal(vc.cpu().numpy(), V)
+
+
 # The last block's key count nk = pos0 % 64 + 1 walks the value sums' runs of 8 key pairs:
 # hd 128 (2 key groups): runs of 16 keys, so nk 16 ends a run, 17 opens one, 25 and 31 end
 # inside one; hd 64 (4 groups): runs of 32 keys.
