@@ -199,9 +199,14 @@ hipError_t launch_quant(const QuantArgs& a, hipStream_t s, int maxK) {
         // float4s per thread: few rows want their reductions over little work per thread (2560
         // wide, RMSNorm, 5 rows: 4 / 8 / 10 a thread 4.4 / 5.4 / 6.1 us; 1024 wide 2 a thread, whose
         // two waves measured 3 % under 4's four); many rows fewer waves each (2560 wide, 2048
-        // rows: 11.9 / 13.7 / 10.6, one wave a row with 10; 6912 wide 30.8 / 25.3 / 30.6)
-        const bool many = (long long)a.M * a.U > 1024;
-        const int NV = many && maxK > 2560 ? 8 : many && maxK > 1536 ? 10 : maxK > 1024 ? 4 : 2;
+        // rows: 11.9 / 13.7 / 10.6, one wave a row with 10; 6912 wide 30.8 / 25.3 / 30.6), the long
+        // rows from one a CU on (RMSNorm with 4 / 8, 6912 wide 128 / 300 / 768 rows 6.4 / 8.9 / 13.4
+        // against 6.6 / 8.6 / 11.9; 5120 wide 300 / 768 rows 7.7 / 11.6 against 8.0 / 10.8; 4096
+        // wide 6.4 / 8.4 against 8.0 / 9.4)
+        const long long rows = (long long)a.M * a.U;
+        const bool many = rows > 1024;
+        const bool eight = (many && maxK > 2560) || (rows > 256 && maxK > 5120);
+        const int NV = eight ? 8 : many && maxK > 1536 ? 10 : maxK > 1024 ? 4 : 2;
         const unsigned threads = (unsigned)round_up((round_up(maxK, kChunk) / 4 + NV - 1) / NV, 64);
         const dim3 grid((unsigned)a.M, (unsigned)a.U), block(threads);
         switch (NV) {

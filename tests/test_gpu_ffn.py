@@ -77,7 +77,9 @@ def test_act_quantize_without_value_outputs(hip, M, K):
                                  (1030, 2624), (1025, 6912), (33, 8192), (1040, 8192),
                                  # no multiple of 64: element by element (or whole float4s of a ragged row)
                                  (3, 1), (5, 63), (20, 1023), (100, 2050), (7, 2564), (1030, 2561), (1025, 6911),
-                                 (3, 8191)])
+                                 (3, 8191),
+                                 # from more than 256 rows on, wider than 5120
+                                 (257, 5120), (257, 5121), (256, 5184), (257, 6911), (300, 8192)])
 def test_act_quantize_widths(hip, M, K):
     test_act_quantize_without_value_outputs(hip, M, K)
 
