@@ -48,36 +48,46 @@ class TernaryFFNBlock:
         self.pair_ok = d_model % 64 == 0 and d_ff % 64 == 0 and d_ff <= 8192
 
     def load(self, norm_weight, gate, up, down):
-        """gate/up/down: (rotor bytes [out, ceil(in/4)], scale) each."""
-        self.norm.weight = np.asarray(norm_weight, dtype=np.float32)
-        self._state.clear()
-        self._gu = self._pair = None
-        if self.use_gpu and self.pair_ok:
-            self._load_pair(gate, up)
-        else:
-            self.gate_proj.load_from_bitnet(*gate)
-            self.up_proj.load_from_bitnet(*up)
-        self.down_proj.load_from_bitnet(*down)
+        """gate/up/down: (rotor bytes [out, ceil(in/4)], scale) each.  A load that is refused, or
+        for which the device has no room, leaves the block as it was.  At the widths of the
+        interleaved copy it is laid out here (4.4 MB a matrix of 6912 x 2560), whatever token
+        counts follow, so that no forward waits for it."""
+        norm = np.asarray(norm_weight, dtype=np.float32)
+        projs = (self.gate_proj, self.up_proj, self.down_proj)
+        packed = [p._checked(*w) for p, w in zip(projs, (gate, up, down))]
+        weights, gu = (None, None, None), None
         if self.use_gpu:
             import torch
 
-            self._norm_w_dev = torch.from_numpy(self.norm.weight.copy()).to(self.gpu.device)
-            self._acts = (self.gpu.activations(self.max_tokens, self.d_model),
-                          self.gpu.activations(self.max_tokens, self.d_ff))
+            if self.pair_ok:
+                gate_up, gu = self._upload_pair(packed)
+            else:
+                gate_up = [self.gpu.upload(b, self.d_model, s) for b, s in packed[:2]]
+            weights = (*gate_up, self.gpu.upload(packed[2][0], self.d_ff, packed[2][1]))
+            norm_dev = torch.from_numpy(norm.copy()).to(self.gpu.device)
+            acts = (self.gpu.activations(self.max_tokens, self.d_model),
+                    self.gpu.activations(self.max_tokens, self.d_ff))
+        # all of it is accepted
+        self.norm.weight = norm
+        for p, (b, s), w in zip(projs, packed, weights):
+            p._set(b, s, w)
+        self._state.clear()
+        self._pair = None
+        if self.use_gpu:
+            self._gu = gu
+            self._norm_w_dev, self._acts = norm_dev, acts
 
-    def _load_pair(self, gate, up):
-        """Gate and up from one copy of their bytes on the device: the two matrices and the
-        interleaved one (HIPTernaryOps.interleave_gate_up's layout)."""
+    def _upload_pair(self, packed):
+        """Gate's and up's weights, and (interleaved matrix, scales) as
+        HIPTernaryOps.interleave_gate_up returns them, from one device copy of the bytes."""
         import torch
 
-        dev, D, F = self.gpu.device, self.d_model, self.d_ff
-        halves = []
-        for proj, (packed, scale) in ((self.gate_proj, gate), (self.up_proj, up)):
-            proj._set_packed(packed, scale)
-            halves.append(torch.from_numpy(proj._packed).to(dev))
-            proj._set_device(self.gpu.upload_device(halves[-1], D, proj.scale))
+        D, F = self.d_model, self.d_ff
+        halves = [torch.from_numpy(b).to(self.gpu.device) for b, _ in packed[:2]]
+        scales = tuple(s for _, s in packed[:2])
+        weights = [self.gpu.upload_device(h, D, s) for h, s in zip(halves, scales)]
         gu = torch.stack([h.view(F // 32, 32, -1) for h in halves], dim=1).view(2 * F, -1)
-        self._gu = (self.gpu.upload_device(gu, D, 1.0), (self.gate_proj.scale, self.up_proj.scale))
+        return weights, (self.gpu.upload_device(gu, D, 1.0), scales)
 
     def _buffers(self, M):
         st = self._state.get(M)

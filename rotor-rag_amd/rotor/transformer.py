@@ -87,24 +87,28 @@ class TernaryLinear:
     def load_from_bitnet(self, packed_weights: np.ndarray, scale: float = 1.0):
         """Load rotor/BitNet bytes [out_features, ceil(in_features/4)] (uint8) and a
         per-tensor scale (src/rotor/transformer.py:77-109)."""
-        self._set_packed(packed_weights, scale)
-        if self.gpu is not None and self.use_gpu:
-            self._set_device(self.gpu.upload(self._packed, self.in_features, self.scale))
+        packed, scale = self._checked(packed_weights, scale)
+        on_gpu = self.gpu is not None and self.use_gpu
+        self._set(packed, scale, self.gpu.upload(packed, self.in_features, scale) if on_gpu else None)
 
-    def _set_packed(self, packed_weights: np.ndarray, scale: float):
+    def _checked(self, packed_weights: np.ndarray, scale: float = 1.0):
+        """(rotor bytes [out, ceil(in/4)], scale) as load_from_bitnet keeps them, or ValueError;
+        changes nothing of the layer."""
         p = np.ascontiguousarray(packed_weights, dtype=np.uint8)
         if p.ndim != 2 or p.shape[0] != self.out_features or p.shape[1] * 4 < self.in_features:
             raise ValueError(f"packed weights of shape {p.shape} do not fit "
                              f"[{self.out_features}, {(self.in_features + 3) // 4}]")
-        p = np.ascontiguousarray(p[:, : (self.in_features + 3) // 4])
-        self.scale = float(scale)
-        self._packed = p
+        return np.ascontiguousarray(p[:, : (self.in_features + 3) // 4]), float(scale)
+
+    def _set(self, packed, scale, weights):
+        """Take over checked bytes, their scale and (on the GPU) the device weights."""
+        self.scale = scale
+        self._packed = packed
         self._planes = None
         self._weights_cache = None
-
-    def _set_device(self, weights):
-        self.gpu_packed_weights = weights
-        self.gpu_scales = np.full(self.out_features, self.scale, dtype=np.float32)
+        if weights is not None:
+            self.gpu_packed_weights = weights
+            self.gpu_scales = np.full(self.out_features, scale, dtype=np.float32)
 
     def forward(self, x):
         """y = x @ W.T * scale for x [batch, seq, in] or [seq, in] (src/rotor/transformer.py:111-155).

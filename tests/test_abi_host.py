@@ -119,6 +119,24 @@ def test_ternary_linear_cpu_mode_is_reference_formula():
     assert np.array_equal(layer.bit0, b0.reshape(-1)) and np.array_equal(layer.bit1, b1.reshape(-1))
 
 
+@pytest.mark.parametrize("which", [0, 1, 2])
+def test_ffn_block_refused_load_changes_nothing_on_cpu(which):
+    from rotor.ffn import TernaryFFNBlock
+
+    rng = np.random.default_rng(which)
+    D, F = 24, 40
+    proj = lambda n, k: (O.pack_rotor(O.make_ternary(rng, n, k)[0]), 0.5)
+    blk = TernaryFFNBlock(D, F, use_gpu=False)
+    blk.load(np.ones(D), proj(F, D), proj(F, D), proj(D, F))
+    x = rng.standard_normal((3, D)).astype(np.float32)
+    ref = blk.forward(x)
+    new = [proj(F, D), proj(F, D), proj(D, F)]
+    new[which] = (new[which][0][:-1], 0.5)
+    with pytest.raises(ValueError, match="do not fit"):
+        blk.load(np.full(D, 2.0), *new)
+    assert np.array_equal(blk.forward(x), ref)
+
+
 def test_use_gpu_without_backend_raises_and_latches(monkeypatch, tmp_path):
     from rotor import _hip, gpu_layers
     from rotor.transformer import TernaryLinear

@@ -179,6 +179,49 @@ def test_ffn_block_graph_replay(hip):
         gpu_layers._gpu_instance = None
 
 
+@pytest.fixture
+def ffn_block(hip):
+    """(block of 256 / 512 with its first weights loaded, a maker of (bytes, scale), norm weight)."""
+    from rotor import gpu_layers
+    from rotor.ffn import TernaryFFNBlock
+
+    D, F = 256, 512
+    rng = np.random.default_rng(17)
+
+    def proj(n, k):
+        W, s = O.make_ternary(rng, n, k)
+        return O.pack_rotor(W), s
+
+    nw = rng.uniform(0.5, 1.5, D).astype(np.float32)
+    gpu_layers._gpu_instance = hip
+    try:
+        blk = TernaryFFNBlock(D, F, use_gpu=True, max_tokens=100)
+        blk.load(nw, proj(F, D), proj(F, D), proj(D, F))
+        yield blk, proj, nw
+    finally:
+        gpu_layers._gpu_instance = None
+
+
+@pytest.mark.parametrize("which", [0, 1, 2])
+@pytest.mark.parametrize("M", [1, 8, 100])
+def test_ffn_block_refused_load_changes_nothing(ffn_block, M, which):
+    """Bytes that one projection refuses: the block goes on with its old weights and norm, at
+    each of its three routes, for token counts it has and has not run before."""
+    blk, proj, nw = ffn_block
+    D, F = blk.d_model, blk.d_ff
+    x = np.random.default_rng(M).standard_normal((100, D)).astype(np.float32)
+    ref = blk.forward(x[:M])
+    new = [proj(F, D), proj(F, D), proj(D, F)]
+    new[which] = (new[which][0][:-1], new[which][1])  # a row short
+    with pytest.raises(ValueError, match="do not fit"):
+        blk.load(nw * 2, *new)
+    assert np.array_equal(blk.forward(x[:M]), ref)
+    blk._state.clear()  # plans and buffers built anew: the same weights
+    blk._pair = None
+    assert np.array_equal(blk.forward(x[:M]), ref)
+    assert np.array_equal(blk.norm.weight, nw)
+
+
 @pytest.mark.parametrize("mode,K,N", [(0, 2560, 640), (2, 2560, 2560), (3, 6912, 2560), (4, 6912, 2560), (2, 100, 77),
                                       (4, 20000, 128)])  # more groups than threads: general prologue path
 def test_fused_plan_equals_act_path(hip, mode, K, N):
