@@ -42,7 +42,7 @@ class TernaryFFNBlock:
         self._state = {}   # token count -> (plan, g, u, y); u None: g is relu^2(gate) * up
         self._acts = None
         self._norm_w_dev = None
-        self._gu = None      # interleaved gate/up copy for one token and for more than 64
+        self._gu = None      # (gate, up, their interleaved copy for one token and past 64, scales)
         self._pair = None    # (input pointer, gate/up plan, down plan, y)
         self._xin = None     # forward()'s device copy of its input
         self.pair_ok = d_model % 64 == 0 and d_ff % 64 == 0 and d_ff <= 8192
@@ -74,7 +74,7 @@ class TernaryFFNBlock:
         self._state.clear()
         self._pair = None
         if self.use_gpu:
-            self._gu = gu
+            self._gu = (*gate_up, *gu) if gu is not None else None
             self._norm_w_dev, self._acts = norm_dev, acts
 
     def _upload_pair(self, packed):
@@ -89,6 +89,14 @@ class TernaryFFNBlock:
         gu = torch.stack([h.view(F // 32, 32, -1) for h in halves], dim=1).view(2 * F, -1)
         return weights, (self.gpu.upload_device(gu, D, 1.0), scales)
 
+    def _gate_up(self):
+        """(interleaved matrix, scales) of gate's and up's present weights: load's, or a new one
+        where either projection has been loaded on its own since."""
+        gate, up = self.gate_proj.gpu_packed_weights, self.up_proj.gpu_packed_weights
+        if self._gu is None or self._gu[0] is not gate or self._gu[1] is not up:
+            self._gu = (gate, up, *self.gpu.interleave_gate_up(gate, up))
+        return self._gu[2:]
+
     def _buffers(self, M):
         st = self._state.get(M)
         if st is None:
@@ -100,7 +108,7 @@ class TernaryFFNBlock:
             act_h = self._acts[0]
             u = None
             if M > 64 and self.pair_ok:
-                w_gu, scales = self._gu
+                w_gu, scales = self._gate_up()
                 plan = self.gpu.plan_act_gate_up(w_gu, scales, act_h, M, g)
             else:
                 u = torch.empty((M, self.d_ff), dtype=torch.float32, device=dev)
@@ -118,7 +126,7 @@ class TernaryFFNBlock:
             from . import _hip
 
             hip, dev = self.gpu, self.gpu.device
-            w_gu, scales = self._gu
+            w_gu, scales = self._gate_up()
             a = torch.empty(self.d_ff, dtype=torch.float32, device=dev)
             ssq = torch.empty(self.d_ff // 32, dtype=torch.float64, device=dev)
             y = torch.empty((1, self.d_model), dtype=torch.float32, device=dev)

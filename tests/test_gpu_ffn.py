@@ -222,6 +222,21 @@ def test_ffn_block_refused_load_changes_nothing(ffn_block, M, which):
     assert np.array_equal(blk.norm.weight, nw)
 
 
+@pytest.mark.parametrize("M", [1, 8, 100])
+def test_ffn_block_projection_loaded_on_its_own(ffn_block, M):
+    """A projection loaded after the block, before its first forward at a token count, is the one
+    that the forward uses."""
+    blk, proj, nw = ffn_block
+    D, F = blk.d_model, blk.d_ff
+    rng = np.random.default_rng(M)
+    x = rng.standard_normal((M, D)).astype(np.float32)
+    Ws = [O.make_ternary(rng, n, k) for n, k in ((F, D), (F, D), (D, F))]
+    blk.load(nw, *[(O.pack_rotor(W), s) for W, s in Ws])
+    blk.gate_proj.load_from_bitnet(O.pack_rotor(Ws[1][0]), 0.25)
+    yo, _ = O.ffn_block_w2a8(x, nw, Ws[1][0], 0.25, *Ws[1], *Ws[2])
+    assert np.array_equal(blk.forward(x), yo)
+
+
 @pytest.mark.parametrize("mode,K,N", [(0, 2560, 640), (2, 2560, 2560), (3, 6912, 2560), (4, 6912, 2560), (2, 100, 77),
                                       (4, 20000, 128)])  # more groups than threads: general prologue path
 def test_fused_plan_equals_act_path(hip, mode, K, N):
