@@ -83,7 +83,7 @@ class TernaryFFNBlock:
         import torch
 
         D, F = self.d_model, self.d_ff
-        halves = [torch.from_numpy(b).to(self.gpu.device) for b, _ in packed[:2]]
+        halves = [torch.from_numpy(np.require(b, requirements="W")).to(self.gpu.device) for b, _ in packed[:2]]
         scales = tuple(s for _, s in packed[:2])
         weights = [self.gpu.upload_device(h, D, s) for h, s in zip(halves, scales)]
         gu = torch.stack([h.view(F // 32, 32, -1) for h in halves], dim=1).view(2 * F, -1)

@@ -237,6 +237,23 @@ def test_ffn_block_projection_loaded_on_its_own(ffn_block, M):
     assert np.array_equal(blk.forward(x), yo)
 
 
+@pytest.mark.filterwarnings("error")
+@pytest.mark.parametrize("M", [1, 8, 100])
+def test_ffn_block_load_takes_what_a_projection_takes(ffn_block, M):
+    """Bytes without a scale (1.0), and read-only arrays without a warning."""
+    blk, _, nw = ffn_block
+    D, F = blk.d_model, blk.d_ff
+    rng = np.random.default_rng(M)
+    x = rng.standard_normal((M, D)).astype(np.float32)
+    Ws = [O.make_ternary(rng, n, k)[0] for n, k in ((F, D), (F, D), (D, F))]
+    packed = [O.pack_rotor(W) for W in Ws]
+    for p in packed:
+        p.setflags(write=False)
+    blk.load(nw, *[(p,) for p in packed])
+    yo, _ = O.ffn_block_w2a8(x, nw, Ws[0], 1.0, Ws[1], 1.0, Ws[2], 1.0)
+    assert np.array_equal(blk.forward(x), yo)
+
+
 @pytest.mark.parametrize("mode,K,N", [(0, 2560, 640), (2, 2560, 2560), (3, 6912, 2560), (4, 6912, 2560), (2, 100, 77),
                                       (4, 20000, 128)])  # more groups than threads: general prologue path
 def test_fused_plan_equals_act_path(hip, mode, K, N):
