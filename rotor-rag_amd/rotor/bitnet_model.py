@@ -526,7 +526,8 @@ class _DeviceModel:
         """forward's one-token step (ids[0] at *pos), captured once: the host's 120 launches of a
         30-layer step took longer than the step (1.86 ms a forward against 1.2).  Captured
         again where a switch that shapes the launches has changed.  The capture runs on a
-        stream of its own and concerns this thread only."""
+        stream of its own, to which the backend's context, one for all its users, is bound
+        meanwhile: the caller binds its own again."""
         import torch
 
         key = (self.attn_in_prologue, self.ffn_pair, self.attn_in_qkv, self.attn_combine_in_qkv, self.ssq_chain)
@@ -553,7 +554,11 @@ class _DeviceModel:
         self.pos.fill_(start)
         if M == 1 and self.trace is None:
             st = self._state(1)
-            self._step_graph().replay()
+            try:
+                step = self._step_graph()
+            finally:  # not the capture's stream, nor an earlier caller's: as after an eager forward
+                self.hip._bind_stream()
+            step.replay()
         else:
             st = self._enqueue(M, pos_base=1 << 30, out_cap=0)
         if M == 1:

@@ -809,6 +809,49 @@ def test_forward_step_graph_equals_eager(hip, Lmax):
     assert same(steps(False)) and dev._step[1] is not first
 
 
+@pytest.mark.filterwarnings("ignore:The CUDA Graph is empty")
+def test_forward_step_leaves_the_callers_stream_bound(hip, monkeypatch):
+    """After a one-token forward the backend's context is on the stream the caller runs on: after
+    the capture, after a replay from another stream, and after a capture that raised."""
+    import torch
+
+    params = O.make_bitnet_params(23, WIDE16, 96)
+    model = _device_model(hip, params, WIDE16, 96)
+    dev, gpu = model._dev, model.gpu
+    _, c = model.forward(np.arange(3, 10, dtype=np.int32), return_logits=False, use_cache=True)
+    bound = []
+
+    class Lib:
+        def __getattr__(self, name):
+            return getattr(real, name)
+
+        def rt_ctx_set_stream(self, ctx, s):
+            bound.append(s.value or 0)
+            return real.rt_ctx_set_stream(ctx, s)
+
+    real = gpu.lib
+    monkeypatch.setattr(gpu, "lib", Lib())
+
+    def step():
+        _, cc = model.forward(np.array([7], np.int32), past_kv_cache=c, use_cache=True)
+        assert bound[-1] == torch.cuda.current_stream().cuda_stream
+
+    def failing(*a, **k):
+        gpu._bind_stream()
+        raise RuntimeError("refused")
+
+    with monkeypatch.context() as m, torch.cuda.stream(torch.cuda.Stream()):
+        m.setattr(dev, "_enqueue", failing)
+        with pytest.raises(RuntimeError, match="refused"):
+            step()
+        assert bound[-1] == torch.cuda.current_stream().cuda_stream
+    step()  # captures
+    side = torch.cuda.Stream()
+    for s in (side, torch.cuda.default_stream(), side):
+        with torch.cuda.stream(s):
+            step()
+
+
 @pytest.mark.parametrize("shape", [(1, 5), (2048, 1024), (2048, 1025), (5, 1 << 20), (3, 1999999)])
 def test_to_host_stages_large_results(small_model, shape):
     """The staged copy to the host (8 MB chunks through two buffers): one chunk or less, one
