@@ -37,6 +37,8 @@ from . import _hip
 TERNARY = ("q_proj", "k_proj", "v_proj", "o_proj", "gate_proj", "up_proj", "down_proj")
 
 
+# _DeviceModel's switches that shape a state's plans and launches
+_SWITCHES = ("attn_in_prologue", "ffn_pair", "attn_in_qkv", "attn_combine_in_qkv", "ssq_chain")
 _STAGE_BYTES = 8 << 20  # one of a model's two pinned staging buffers
 
 
@@ -216,7 +218,6 @@ class _DeviceModel:
         # the o_proj prologue combines them), "h": [D], "logits": [V]} to trace["steps"]
         self.trace = None
         self._tbuf = None  # the trace's device buffers (allocated before any graph capture)
-        self._step = None  # (switches, graph) of forward's one-token step
         self._stage = None  # the pinned buffers of _to_host, freed with the model
         hip = self.hip = model.gpu
         dev = self.device = hip.device
@@ -287,14 +288,20 @@ class _DeviceModel:
         self.ssq_chain = True
 
     def _state(self, M):
+        """Buffers and plans of a forward over M tokens, built once and again after a switch has
+        changed; for M = 1 also forward's captured step ("step"), which lives and goes with them."""
+        switches = tuple(getattr(self, name) for name in _SWITCHES)
         st = self.state.get(M)
         if st is not None:
-            return st
+            if st["switches"] == switches:
+                return st
+            del self.state[M], st  # the old plans go before the new ones are built
         import torch
 
         dev, D, F, H, Hkv, hd = self.device, self.D, self.F, self.H, self.Hkv, self.hd
         e = lambda *s: torch.empty(s, dtype=torch.float32, device=dev)
-        st = {"h": e(M, D), "q": e(M, H * hd), "k": e(M, Hkv * hd), "v": e(M, Hkv * hd), "o": e(M, H * hd),
+        st = {"switches": switches, "step": None,
+              "h": e(M, D), "q": e(M, H * hd), "k": e(M, Hkv * hd), "v": e(M, Hkv * hd), "o": e(M, H * hd),
               "g": e(M, F), "u": e(M, F), "a": e(F),
               "ssq": torch.empty(F // 32, dtype=torch.float64, device=dev),
               "hssq": torch.empty((D + 31) // 32, dtype=torch.float64, device=dev)}
@@ -522,17 +529,14 @@ class _DeviceModel:
         if ids.min() < 0 or ids.max() >= self.m.vocab_size:
             raise ValueError("token id out of range")
 
-    def _step_graph(self):
-        """forward's one-token step (ids[0] at *pos), captured once: the host's 120 launches of a
-        30-layer step took longer than the step (1.86 ms a forward against 1.2).  Captured
-        again where a switch that shapes the launches has changed.  The capture runs on a
-        stream of its own, to which the backend's context, one for all its users, is bound
-        meanwhile: the caller binds its own again."""
+    def _step_graph(self, st):
+        """forward's one-token step (ids[0] at *pos), captured once per state: the host's 120
+        launches of a 30-layer step took longer than the step (1.86 ms a forward against 1.2).
+        The capture runs on a stream of its own, to which the backend's context, one for all its
+        users, is bound meanwhile: the caller binds its own again."""
         import torch
 
-        key = (self.attn_in_prologue, self.ffn_pair, self.attn_in_qkv, self.attn_combine_in_qkv, self.ssq_chain)
-        if self._step is None or self._step[0] != key:
-            self._state(1)  # plans and buffers, outside the capture
+        if st["step"] is None:
             side = torch.cuda.Stream(self.device)
             side.wait_stream(torch.cuda.current_stream(self.device))
             g = torch.cuda.CUDAGraph()
@@ -542,8 +546,8 @@ class _DeviceModel:
                     self._enqueue(1, pos_base=1 << 30, out_cap=0)
                 finally:
                     g.capture_end()
-            self._step = (key, g)
-        return self._step[1]
+            st["step"] = g
+        return st["step"]
 
     def forward(self, ids, start, return_logits):
         import torch
@@ -555,7 +559,7 @@ class _DeviceModel:
         if M == 1 and self.trace is None:
             st = self._state(1)
             try:
-                step = self._step_graph()
+                step = self._step_graph(st)
             finally:  # not the capture's stream, nor an earlier caller's: as after an eager forward
                 self.hip._bind_stream()
             step.replay()
@@ -639,6 +643,7 @@ class _DeviceModel:
         emb1 = not self.embed_in_argmax
         g = None
         if n > 1 and graph:  # capture the decode step first (capture does not execute it)
+            self._state(1)  # plans and buffers, outside the capture
             torch.cuda.synchronize()
             g = torch.cuda.CUDAGraph()
             with torch.cuda.graph(g):

@@ -781,7 +781,8 @@ def test_decode_attention_in_qkv_launch_bit_exact(hip):
 def test_forward_step_graph_equals_eager(hip, Lmax):
     """The captured one-token step of BitNetModel.forward gives the eager step's logits (the
     traced forward launches them one by one) and cache bit for bit: over several tokens, when
-    rewound, on another stream, and captured again after a switch of the launches changed."""
+    rewound, on another stream, and captured again over new plans: where the state was dropped
+    and where a switch of the launches changed."""
     import torch
 
     params = O.make_bitnet_params(23, WIDE16, Lmax)
@@ -801,12 +802,25 @@ def test_forward_step_graph_equals_eager(hip, Lmax):
     ref = steps(True)
     same = lambda got: all(np.array_equal(a, b) for a, b in zip(ref, got))
     assert same(steps(False)) and same(steps(False))
-    first = dev._step[1]
+    first = dev.state[1]["step"]
     with torch.cuda.stream(torch.cuda.Stream()):
         assert same(steps(False))
-    assert dev._step[1] is first
-    dev.attn_in_qkv = False  # a key of the capture (the plans of st[1] stay as built)
-    assert same(steps(False)) and dev._step[1] is not first
+    assert dev.state[1]["step"] is first
+    dev.state.clear()  # plans and buffers go, and the step captured over them
+    assert same(steps(False)) and dev.state[1]["step"] is not first
+    # each switch builds other plans: the replayed step gives the eager step's bits with them (the
+    # forms agree bit for bit but for the f64 sums of squares, taken in another order)
+    for name, made in (("attn_in_qkv", lambda st: not any(st["attn_fused"])),
+                       ("ssq_chain", lambda st: True), ("ffn_pair", lambda st: True),
+                       ("attn_in_prologue", lambda st: True), ("attn_combine_in_qkv", lambda st: True)):
+        before = dev.state[1]
+        setattr(dev, name, False)
+        ref = steps(True)
+        assert dev.state[1] is not before and made(dev.state[1]), name
+        assert dev.state[1]["step"] is None  # (the traced steps capture nothing)
+        assert same(steps(False)) and same(steps(False)), name
+        now = dev.state[1]["step"]
+        assert same(steps(False)) and dev.state[1]["step"] is now, name
 
 
 @pytest.mark.filterwarnings("ignore:The CUDA Graph is empty")
