@@ -26,6 +26,7 @@ GPU only: ``use_gpu=False`` raises.
 from __future__ import annotations
 
 import ctypes
+import gc
 import json
 from pathlib import Path
 from typing import Dict, Optional
@@ -540,12 +541,21 @@ class _DeviceModel:
             side = torch.cuda.Stream(self.device)
             side.wait_stream(torch.cuda.current_stream(self.device))
             g = torch.cuda.CUDAGraph()
-            with torch.cuda.stream(side):
-                g.capture_begin(capture_error_mode="thread_local")
-                try:
-                    self._enqueue(1, pos_base=1 << 30, out_cap=0)
-                finally:
-                    g.capture_end()
+            # A dropped model's plans and weights are freed by the cyclic collector (the model and
+            # its device half refer to each other), with calls that a capture on this thread does
+            # not survive: no collection until it has ended (collecting first costs 70 ms).
+            collecting = gc.isenabled()
+            gc.disable()
+            try:
+                with torch.cuda.stream(side):
+                    g.capture_begin(capture_error_mode="thread_local")
+                    try:
+                        self._enqueue(1, pos_base=1 << 30, out_cap=0)
+                    finally:
+                        g.capture_end()
+            finally:
+                if collecting:
+                    gc.enable()
             st["step"] = g
         return st["step"]
 

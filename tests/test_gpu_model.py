@@ -866,6 +866,33 @@ def test_forward_step_leaves_the_callers_stream_bound(hip, monkeypatch):
             step()
 
 
+@pytest.mark.filterwarnings("ignore:The CUDA Graph is empty")
+def test_step_capture_is_not_interrupted_by_the_collector(hip, monkeypatch):
+    """No cyclic collection while the step is captured (it could free a dropped model's plans, whose
+    frees a capture does not survive); collection as before afterwards, also if the capture raised."""
+    import gc
+
+    params = O.make_bitnet_params(23, WIDE16, 96)
+    model = _device_model(hip, params, WIDE16, 96)
+    dev = model._dev
+    _, c = model.forward(np.arange(3, 10, dtype=np.int32), return_logits=False, use_cache=True)
+    seen, enqueue = [], dev._enqueue
+
+    def watched(M, **k):
+        seen.append(gc.isenabled())
+        if len(seen) == 1:
+            raise RuntimeError("refused")
+        return enqueue(M, **k)
+
+    monkeypatch.setattr(dev, "_enqueue", watched)
+    assert gc.isenabled()
+    with pytest.raises(RuntimeError, match="refused"):
+        model.forward(np.array([7], np.int32), past_kv_cache=c, use_cache=True)
+    assert gc.isenabled()
+    model.forward(np.array([7], np.int32), past_kv_cache=c, use_cache=True)
+    assert seen == [False, False] and gc.isenabled()
+
+
 @pytest.mark.parametrize("shape", [(1, 5), (2048, 1024), (2048, 1025), (5, 1 << 20), (3, 1999999)])
 def test_to_host_stages_large_results(small_model, shape):
     """The staged copy to the host (8 MB chunks through two buffers): one chunk or less, one
