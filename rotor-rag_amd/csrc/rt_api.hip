@@ -1368,16 +1368,18 @@ int rt_plan_attach_attention(rt_plan* plan, float* k_cache, float* v_cache, cons
     // err
     const size_t bytes = (words + pwords) * sizeof(unsigned long long) + 256;
     // a launch of this plan may still be in flight on the caller's stream: wait for it
-    // before the hand-off state is freed or reset
+    // before the hand-off state is freed or reset.  The attention is off until all of it is
+    // there, and the flag comes before att_mem, whose presence stands for both.
     if (plan->att_mem) RT_HIP(hipDeviceSynchronize());
+    plan->att_on = false;
+    if (!plan->att_flag) RT_HIP(hipHostMalloc(&plan->att_flag, sizeof(int), hipHostMallocMapped));
+    void* flag_dev = nullptr;
+    RT_HIP(hipHostGetDevicePointer(&flag_dev, plan->att_flag, 0));
     if (plan->att_mem && plan->att_bytes != bytes) {
         RT_HIP(hipFree(plan->att_mem));
         plan->att_mem = nullptr;
     }
     if (!plan->att_mem) RT_HIP(hipMalloc(&plan->att_mem, bytes));
-    if (!plan->att_flag) RT_HIP(hipHostMalloc(&plan->att_flag, sizeof(int), hipHostMallocMapped));
-    void* flag_dev = nullptr;
-    RT_HIP(hipHostGetDevicePointer(&flag_dev, plan->att_flag, 0));
     plan->att_bytes = bytes;
     AttnTail& t = plan->att;
     t.tagged = static_cast<unsigned long long*>(plan->att_mem);

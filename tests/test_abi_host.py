@@ -11,6 +11,7 @@
 import ctypes
 import re
 import subprocess
+import sys
 from pathlib import Path
 
 import numpy as np
@@ -171,3 +172,104 @@ def test_missing_library_raises():
     finally:
         del os.environ["ROTOR_HIP_LIB"]
         _hip._lib = old
+
+
+# ---------------------------------------------------------------- failing allocations
+
+# A HIP runtime on host memory, which a child process loads ahead of the real one: allocations and copies
+# work, launches do nothing, and the n-th call of a chosen allocator from now on fails.
+FAKE_HIP = r"""
+#define __HIP_PLATFORM_AMD__ 1
+#include <hip/hip_runtime_api.h>
+#include <stdlib.h>
+#include <string.h>
+static int fail_malloc = 0, fail_host = 0;
+void fake_fail(int device_call, int host_call) { fail_malloc = device_call; fail_host = host_call; }
+static hipError_t give(void** p, size_t n, int* countdown) {
+    if (*countdown && --*countdown == 0) return hipErrorOutOfMemory;
+    return (*p = calloc(1, n + 1)) ? hipSuccess : hipErrorOutOfMemory;
+}
+hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
+hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
+hipError_t hipSetDevice(int d) { (void)d; return hipSuccess; }
+hipError_t hipGetDeviceProperties(hipDeviceProp_t* p, int d) {
+    (void)d; memset(p, 0, sizeof *p); strcpy(p->gcnArchName, "gfx950"); return hipSuccess;
+}
+hipError_t hipFuncSetAttribute(const void* f, hipFuncAttribute a, int v) { (void)f; (void)a; (void)v; return hipSuccess; }
+hipError_t hipGetSymbolAddress(void** p, const void* s) { (void)s; static char b[64]; *p = b; return hipSuccess; }
+hipError_t hipMalloc(void** p, size_t n) { return give(p, n, &fail_malloc); }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned f) { (void)f; return give(p, n, &fail_host); }
+hipError_t hipFree(void* p) { free(p); return hipSuccess; }
+hipError_t hipHostFree(void* p) { free(p); return hipSuccess; }
+hipError_t hipHostGetDevicePointer(void** d, void* h, unsigned f) { (void)f; *d = h; return hipSuccess; }
+hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind k) { (void)k; memcpy(d, s, n); return hipSuccess; }
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind k, hipStream_t q) {
+    (void)q; return hipMemcpy(d, s, n, k);
+}
+hipError_t hipMemset(void* d, int v, size_t n) { memset(d, v, n); return hipSuccess; }
+hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t q) { (void)q; return hipMemset(d, v, n); }
+hipError_t hipDeviceSynchronize(void) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t q) { (void)q; return hipSuccess; }
+hipError_t hipGetLastError(void) { return hipSuccess; }
+hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void** a, size_t l, hipStream_t q) {
+    (void)f; (void)g; (void)b; (void)a; (void)l; (void)q; return hipSuccess;
+}
+"""
+
+FAKE_CHILD = r"""
+import ctypes, sys
+sys.path.insert(0, sys.argv[1])
+from rotor import _hip
+fake = ctypes.CDLL(sys.argv[2], ctypes.RTLD_GLOBAL)  # the library's HIP calls resolve to it
+lib, P = _hip.load(), ctypes.c_void_p
+ok = lambda rc: _hip.check(rc, "setup")
+ctx = P()
+ok(lib.rt_ctx_create(0, ctypes.byref(ctx)))
+H, Hkv, hd, D, Lmax = 16, 4, 128, 2048, 96
+mem = (ctypes.c_double * (4 << 20))()  # every buffer the plan only keeps a pointer to
+buf = ctypes.addressof(mem) + 15 & ~15
+ws = []
+for n in (H * hd, Hkv * hd, Hkv * hd):
+    w, rows = P(), (ctypes.c_uint8 * (n * D // 4))()
+    ok(lib.rt_weights_upload(ctx, rows, n, D, 1.0, ctypes.byref(w)))
+    ws.append(w)
+src = _hip.RtSrc(_hip.SRC_RMSNORM, buf, buf, None, 1e-6, 0, 0)
+plan = P()
+ok(lib.rt_plan_create_fused(ctx, 3, (P * 3)(*ws), ctypes.byref(src), (P * 3)(buf, buf, buf), None, ctypes.byref(plan)))
+attach = lambda L: lib.rt_plan_attach_attention(plan, buf, buf, buf, H, Hkv, hd, L, buf, buf, 1 << 40)
+
+def timeouts():
+    n = ctypes.c_int(-1)
+    assert lib.rt_plan_attention_timeouts(plan, ctypes.byref(n)) == 0 and n.value == 0
+
+def off():  # nothing of a failed attach is left for a launch to use
+    timeouts()
+    assert lib.rt_plan_attention_combine(plan, buf, buf) == -1 and "attach the attention first" in _hip.last_error()
+
+for device_call, host_call in ((0, 1), (1, 0)):
+    fake.fake_fail(device_call, host_call)
+    assert attach(Lmax) == -2, _hip.last_error()
+    off()
+ok(attach(Lmax))
+timeouts()
+fake.fake_fail(1, 0)  # attached again at another length: the old state is freed before the new one is there
+assert attach(Lmax + 64) == -2
+off()
+ok(attach(Lmax + 64))
+timeouts()
+ok(lib.rt_plan_free(plan))
+print("done")
+"""
+
+
+def test_attach_attention_survives_failed_allocations(tmp_path):
+    """Each allocation of rt_plan_attach_attention refused in turn: an error status, the attention
+    off, and rt_plan_attention_timeouts still answering."""
+    (tmp_path / "fake_hip.c").write_text(FAKE_HIP)
+    so = tmp_path / "fake_hip.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", "-I/opt/rocm/include", "-o", str(so), str(tmp_path / "fake_hip.c")],
+                   check=True, capture_output=True)
+    (tmp_path / "child.py").write_text(FAKE_CHILD)
+    r = subprocess.run([sys.executable, str(tmp_path / "child.py"), str(ROOT / "rotor-rag_amd"), str(so)],
+                       capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and r.stdout.strip() == "done", (r.returncode, r.stdout, r.stderr[-2000:])
