@@ -53,6 +53,10 @@ struct AttnRun {
     float alpha, m, z, pad;
 };
 typedef __attribute__((address_space(3))) AttnRun lds_run;
+// alpha of a block that adds nothing, and of the first that adds something after such blocks
+// (the sums start again: what theirs hold, 0 times the values, may be NaN).  Telling them apart
+// costs the launch 0.1 us (20 heads of 128 at position 1537 of 2048: 16.3 -> 16.4).
+constexpr float kAttnSkip = -2.0f, kAttnFirst = -1.0f;
 
 // The tile's LDS is reached through a local-address-space pointer: through a generic one,
 // a select between an LDS value and a register of the key block (the new key) becomes a
@@ -346,14 +350,28 @@ __device__ __forceinline__ void attn_tile2(SRC qh, SRC kn, SRC vn, float c, floa
             float sc = lane < nk
                            ? (((sm->part[0][lane] + sm->part[1][lane]) + (sm->part[2][lane] + sm->part[3][lane])) * scale)
                            : -INFINITY;
-            const float mx = fmaxf(mrun, lane63(wave_reduce63(sc, -INFINITY, [](float x, float y) { return fmaxf(x, y); })));
-            const float p = lane < nk ? expf(sc - mx) : 0.0f;
+            const float bm = lane63(wave_reduce63(sc, -INFINITY, [](float x, float y) { return fmaxf(x, y); }));
+            float mx = fmaxf(mrun, bm), p = lane < nk ? expf(sc - mx) : 0.0f;
+            float al = r > 0 ? expf(mrun - mx) : 0.0f;  // (the first block's sums start from zero)
+            if (!(bm > -INFINITY)) {
+                // all scores -inf: the block adds nothing, as an empty partial in the combine.  A
+                // NaN makes the sums NaN, and the maximum too where there is no other (one of
+                // -inf would have the combine leave the split out).
+                if (!__any(sc != sc)) {
+                    mx = mrun;
+                    p = 0.0f;
+                    al = kAttnSkip;
+                } else if (mx == -INFINITY) {
+                    mx = __builtin_nanf("");
+                }
+            } else if (r > 0 && mrun == -INFINITY) {
+                al = kAttnFirst;
+            }
             const float z = wave_reduce63(p, 0.0f, [](float x, float y) { return x + y; });
             sm->pr[lane] = p;
-            if (r > 0) {  // (the first block's sums start from zero)
-                const float al = expf(mrun - mx);
+            if (r > 0) {
                 if (lane == 63) run->alpha = al;
-                zrun = fmaf(zrun, al, z);
+                zrun = fmaf(zrun, al == kAttnSkip ? 1.0f : al, z);
             } else {
                 zrun = z;
             }
@@ -362,13 +380,19 @@ __device__ __forceinline__ void attn_tile2(SRC qh, SRC kn, SRC vn, float c, floa
         attn_lds_barrier();
         // unnormalised output: attn_tile's sums, scaled to the new maximum first
         if (live) {
+            bool skip = false;
             if (r > 0) {
                 const float al = run->alpha;
-                o0 *= al;
-                o1 *= al;
+                skip = al == kAttnSkip;
+                if (al >= 0.0f || al != al) {
+                    o0 *= al;
+                    o1 *= al;
+                } else if (!skip) {
+                    o0 = o1 = 0.0f;
+                }
             }
             // the new key, the block's last, is added after the cached ones (the same order)
-            const int nc = holds_new ? lp : nk;
+            const int nc = skip ? 0 : holds_new ? lp : nk;
 #pragma unroll
             for (int c0 = 0; c0 < VN; c0 += CH) {
                 const int first = g + c0 * G, last = g + (c0 + CH - 1) * G;
@@ -388,7 +412,7 @@ __device__ __forceinline__ void attn_tile2(SRC qh, SRC kn, SRC vn, float c, floa
                     }
                 }
             }
-            if (holds_new) {
+            if (holds_new && !skip) {
                 // its slot among this thread's keys g, g + G, .. (g and lp uniform over the wave)
                 const int rel = __builtin_amdgcn_readfirstlane(lp - g);
                 if (rel >= 0 && rel % G == 0) {
@@ -409,11 +433,13 @@ __device__ __forceinline__ void attn_tile2(SRC qh, SRC kn, SRC vn, float c, floa
     if (tile == 0 && g == 0) {
         float o = sm->ored[d];
         for (int gg = 1; gg < G; ++gg) o += sm->ored[gg * HD + d];
-        // tile 0 holds the split's first block; tile 1 may hold none (m = -inf)
+        // either tile may have no block that counts (m = -inf, z = 0)
         const float m0 = run->m, m1 = run1->m, m = fmaxf(m0, m1);
-        const float f0 = expf(m0 - m), f1 = m1 == -INFINITY ? 0.0f : expf(m1 - m);
+        const float f0 = m0 == -INFINITY ? 0.0f : expf(m0 - m), f1 = m1 == -INFINITY ? 0.0f : expf(m1 - m);
         float ob = sm1->ored[d];
         for (int gg = 1; gg < G; ++gg) ob += sm1->ored[gg * HD + d];
+        if (m0 == -INFINITY) o = 0.0f;
+        if (m1 == -INFINITY) ob = 0.0f;
         wp[d] = fmaf(f1, ob, f0 * o);
         if (d == 0) {
             wp[HD] = m;

@@ -445,6 +445,50 @@ def test_qkv_plan_with_attention_long(hip, H, Hkv, pos0, Lmax):
     test_qkv_plan_with_attention_equals_separate_launches(hip, H, Hkv, pos0, Lmax)
 
 
+# blocks of 64 keys whose scores are all -inf (overflowed products), of ten (one a split) and of 21:
+# the first of a split's tile 0 (0), of its tile 1 (10), a later one (20), both tiles' first, every one
+# of split 0, all but the last
+@pytest.mark.parametrize("pos0,Lmax,blocks", [(600, 640, (0,)), (600, 640, (3, 4)), (600, 640, tuple(range(9))),
+                                              (1300, 1344, (0,)), (1300, 1344, (10,)), (1300, 1344, (20,)),
+                                              (1300, 1344, (0, 10)), (1300, 1344, (0, 10, 20)),
+                                              (1300, 1344, (3, 13)), (1300, 1344, tuple(range(20)))])
+@pytest.mark.parametrize("H,Hkv,hd", [(8, 2, 128), (8, 2, 64)])
+def test_attention_decode_blocks_without_scores(hip, H, Hkv, hd, pos0, Lmax, blocks):
+    """Such blocks add nothing, whatever their values hold: the result is the softmax over the
+    other keys.  With NaN instead, every output is NaN."""
+    lib, chk = _lib()
+    import torch
+
+    rng = np.random.default_rng(len(blocks) + hd)
+    K = rng.standard_normal((Hkv, pos0 + 1, hd)).astype(np.float32)
+    V = rng.standard_normal((Hkv, pos0 + 1, hd)).astype(np.float32)
+    q = rng.standard_normal((H, hd)).astype(np.float32)
+    q[:, 0] = 1.0
+    keep = ~np.isin(np.arange(pos0 + 1) // 64, blocks)
+    # f64 reference over the keys that count
+    k4, v4 = (np.repeat(a[:, keep].astype(np.float64), H // Hkv, axis=0) for a in (K, V))
+    sc = np.einsum("hd,hkd->hk", q.astype(np.float64), k4) / np.sqrt(hd)
+    p = np.exp(sc - sc.max(1, keepdims=True))
+    o = np.einsum("hk,hkd->hd", p / p.sum(1, keepdims=True), v4)
+    nbytes = lib.rt_attention_decode_workspace(H, hd, Lmax)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+    qd, out = torch.from_numpy(q).cuda(), torch.empty(H * hd, device="cuda")
+    pos = torch.tensor([pos0], dtype=torch.int32, device="cuda")
+    for bad in (-np.inf, np.nan):
+        K[:, ~keep, 0] = bad
+        V[:, ~keep, ::3] = np.inf if np.isinf(bad) else 0.0
+        kc, vc = torch.zeros(Hkv, hd, Lmax, device="cuda"), torch.zeros(Hkv, Lmax, hd, device="cuda")
+        kc[:, :, :pos0 + 1] = torch.from_numpy(K.transpose(0, 2, 1).copy())
+        vc[:, :pos0 + 1] = torch.from_numpy(V)
+        hip._bind_stream()
+        chk(lib.rt_attention_decode(hip.ctx, qd.data_ptr(), kc.data_ptr(), vc.data_ptr(), out.data_ptr(), H, Hkv, hd,
+                                    Lmax, pos.data_ptr(), ws.data_ptr(), nbytes))
+        if np.isinf(bad):
+            np.testing.assert_allclose(out.cpu().numpy().reshape(H, hd), o, atol=2e-5, rtol=1e-4)
+        else:
+            assert out.isnan().all()
+
+
 def test_attach_attention_rejects_other_plans(hip):
     """Plans the attention cannot join (one problem; 2 query heads per KV head) are refused
     with the library's message, and stay usable."""
