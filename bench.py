@@ -691,7 +691,7 @@ def main():
             "frac": round(value / HBM_PEAK_GBS, 4),
             "traffic": int(prof["traffic_bytes_per_launch"]) if G == 128 and "traffic_bytes_per_launch" in prof else None,
             "traffic_source": "profiles/gemv_2560x6912_m1_g128.md (rocprofv3 FETCH_SIZE+WRITE_SIZE, copy-calibrated)",
-            "kernel": "rt::gemv_rows_kernel<1, 1>",
+            "kernel": "rt::gemv_rows_kernel<1>",
             "bytes_per_launch": bytes_step,
             "avg_launch_ms": round(step_ms, 5),
             "timing": "HIP events around the timed region's back-to-back launches (one launch per step)",
@@ -705,7 +705,7 @@ def main():
         "two_launch_form": {
             "step_ms": round(two_step_ms, 5),
             "gemv_kernel_avg_ms": round(gemv_avg, 5),
-            "gemv_kernel": "rt::gemv_rows_kernel<1, 0>",
+            "gemv_kernel": "rt::gemv_rows_kernel<0>",
             "gemv_GB_per_s": round(G * gemv_bytes(1, N_OUT, K_IN) / (gemv_avg * 1e-3) / 1e9, 1),
             "step_GB_per_s": round(G * gemv_bytes(1, N_OUT, K_IN) / (two_step_ms * 1e-3) / 1e9, 1),
         },

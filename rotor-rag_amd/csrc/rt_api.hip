@@ -436,7 +436,7 @@ static int launch_matrix(rt_ctx* ctx, const rt_weights* w, const int8_t* qx, con
     a.M = M;
     a.out_i32 = out_i32 ? 1 : 0;
     a.total_rb = w->Np / kRowBlock;
-    a.p = GemvProb{w->tiles, qx, sx, row_scale, out, w->scale, w->N, w->C, w->N, 0, res};
+    a.p = GemvProb{w->tiles, qx, sx, row_scale, out, w->scale, w->N, w->C, 0, res};
     const GemvShape shape = gemv_shape(a.total_rb, w->C);
     RT_HIP(launch_gemv(a, shape, ctx->stream));
     return RT_OK;
@@ -450,7 +450,7 @@ static int linear_m1_prologue(rt_ctx* ctx, const rt_weights* w, const float* x, 
     a.G = 1;
     a.M = 1;
     a.total_rb = w->Np / kRowBlock;
-    a.p = GemvProb{w->tiles, nullptr, nullptr, row_scale, out, w->scale, w->N, w->C, w->N, 0, nullptr, x, w->K};
+    a.p = GemvProb{w->tiles, nullptr, nullptr, row_scale, out, w->scale, w->N, w->C, 0, nullptr, x, w->K};
     const QuantProb src{x, nullptr, nullptr, nullptr, nullptr, w->K, w->Kp, kQuant, nullptr, 0.0f, nullptr,
                         nullptr, 0, 0, 0};
     const int nb = a.total_rb;
@@ -742,7 +742,7 @@ int rt_plan_create(rt_ctx* ctx, int G, const rt_weights* const* w, const float* 
     for (int g = 0; g < G; ++g) {
         const int u = which[g];
         p->probs[g] = GemvProb{w[g]->tiles, p->quant[u].qx, p->quant[u].sx, nullptr, y[g], w[g]->scale,
-                               w[g]->N, w[g]->C, w[g]->N, wg};
+                               w[g]->N, w[g]->C, wg};
         wg += w[g]->Np / kRowBlock;
         if (w[g]->C < minC) minC = w[g]->C;
     }
@@ -1025,7 +1025,7 @@ int rt_plan_create_act(rt_ctx* ctx, int G, const rt_weights* const* w, const rt_
     p->probs.resize(G);
     for (int g = 0; g < G; ++g) {
         p->probs[g] = GemvProb{w[g]->tiles, act[g]->qx, act[g]->sx, nullptr, y[g], w[g]->scale,
-                               w[g]->N, w[g]->C, w[g]->N, wg};
+                               w[g]->N, w[g]->C, wg};
         wg += w[g]->Np / kRowBlock;
         if (w[g]->C < minC) minC = w[g]->C;
         if (M > kGemvMaxM)
@@ -1072,7 +1072,7 @@ int rt_plan_create_act_gate_up(rt_ctx* ctx, const rt_weights* w_gu, float s_gate
     p->acts.assign(1, act);
     p->pair_gemm = true;
     const int F = w_gu->N / 2;
-    p->probs.assign(1, GemvProb{w_gu->tiles, act->qx, act->sx, nullptr, a_out, 1.0f, w_gu->N, w_gu->C, F, 0});
+    p->probs.assign(1, GemvProb{w_gu->tiles, act->qx, act->sx, nullptr, a_out, 1.0f, w_gu->N, w_gu->C, 0});
     p->total_rb = w_gu->Np / kRowBlock;
     GemmArgs ga{w_gu->tiles, act->qx, act->sx, nullptr, nullptr, 1.0f, M, w_gu->N, w_gu->Np, w_gu->C, F, 0};
     ga.pair_a = a_out;
@@ -1258,7 +1258,7 @@ int rt_plan_create_fused(rt_ctx* ctx, int G, const rt_weights* const* w, const r
     int wg = 0, minC = 1 << 30;
     p->probs.resize(G);
     for (int g = 0; g < G; ++g) {
-        p->probs[g] = GemvProb{w[g]->tiles, nullptr, nullptr, nullptr, y[g], w[g]->scale, w[g]->N, w[g]->C, w[g]->N, wg,
+        p->probs[g] = GemvProb{w[g]->tiles, nullptr, nullptr, nullptr, y[g], w[g]->scale, w[g]->N, w[g]->C, wg,
                                residual ? residual[g] : nullptr};
         wg += w[g]->Np / kRowBlock;
         if (w[g]->C < minC) minC = w[g]->C;
@@ -1309,8 +1309,7 @@ int rt_plan_create_gate_up(rt_ctx* ctx, const rt_weights* w_gu, float s_gate, fl
     p->fused = true;
     p->pro = QuantProb{src->x, nullptr, nullptr, nullptr, nullptr, K, Kp, src->mode, src->aux, src->eps, nullptr,
                        src->aux2, 0, 0};
-    p->probs = {GemvProb{w_gu->tiles, nullptr, nullptr, nullptr, nullptr, w_gu->scale, w_gu->N, w_gu->C, w_gu->N,
-                         0, nullptr}};
+    p->probs = {GemvProb{w_gu->tiles, nullptr, nullptr, nullptr, nullptr, w_gu->scale, w_gu->N, w_gu->C, 0, nullptr}};
     p->pair_sg = s_gate;
     p->pair_su = s_up;
     p->total_rb = Nb;

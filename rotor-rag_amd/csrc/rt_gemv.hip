@@ -6,7 +6,7 @@
 //   * a wave owns one 64-row block of one problem; lane r accumulates row 64*rb + r,
 //     so no cross-lane reduction is needed;
 //   * each chunk step is one coalesced 16-byte-per-lane (1 KiB per wave) non-temporal
-//     buffer load of rotor bytes; loads run one batch of U chunks ahead of the math;
+//     buffer load of rotor bytes; loads run one batch of kU chunks ahead of the math;
 //   * the activations of a chunk are the same for all 64 lanes, so they are read
 //     with scalar loads into SGPRs and fed to v_dot4_i32_i8 as the scalar operand.
 // Two launch shapes share the body:
@@ -24,7 +24,7 @@
 // accP and 4 sum g x into accQ, and, with g = w + 1,
 //     sum w x = accP + accQ / 4 - sum x.
 // sum x over the same k range (padding activations are 0) is the same for every lane:
-// each wave computes it once from the activation row (slice_sums), or, where a prologue
+// each wave computes it once from the activation row (slice_sum), or, where a prologue
 // quantised the row, the prologue leaves the row's total and one wave subtracts it.
 #include <algorithm>
 #include <type_traits>
@@ -38,6 +38,7 @@
 namespace rt {
 
 constexpr int kAuxNT = 2;                 // cache policy: non-temporal (streamed once)
+constexpr int kU = 4;                     // chunks per batch
 
 // The activations are read-only for the whole launch, so the constant address space
 // lets uniform reads become s_load; a prologue-quantised row is read from LDS.
@@ -61,7 +62,7 @@ __device__ __forceinline__ GemvProb find_prob(const GemvArgs& a, int rbg) {
     }
     if (!a.dev) return a.p;
     const cprob* q = (cprob*)a.dev + ((cidx*)a.rb2p)[rbg];
-    return GemvProb{q->w, q->qx, q->sx, q->rs, q->out, q->s_w, q->N, q->C, q->ldo, q->wg_begin, q->res, q->xs, q->K};
+    return GemvProb{q->w, q->qx, q->sx, q->rs, q->out, q->s_w, q->N, q->C, q->wg_begin, q->res, q->xs, q->K};
 }
 
 // floor(a / nw) from m = ceil(2^31 / nw), for 1 <= nw <= 16 and 0 <= a < 2^23 (a = wave * C
@@ -108,9 +109,8 @@ __device__ __forceinline__ QuantProb own_source(const GemvProb& P) {
                      nullptr, 0, 0, 0};
 }
 
-template <int MT, typename XP>
-__device__ __forceinline__ void chunk_step(const v4u v, XP* __restrict__ xc, const int ldx,
-                                           int (&accP)[MT], int (&accQ)[MT]) {
+template <typename XP>
+__device__ __forceinline__ void chunk_step(const v4u v, XP* __restrict__ xc, int& accP, int& accQ) {
     int d[16];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -122,51 +122,42 @@ __device__ __forceinline__ void chunk_step(const v4u v, XP* __restrict__ xc, con
         d[4 * j + 3] = (int)(h & 0x0C0C0C0Cu);
     }
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        XP* __restrict__ xm = xc + m * ldx;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            accP[m] = __builtin_amdgcn_sdot4(d[4 * j + 0], xm[4 * j + 0], accP[m], false);
-            accQ[m] = __builtin_amdgcn_sdot4(d[4 * j + 1], xm[4 * j + 1], accQ[m], false);
-            accP[m] = __builtin_amdgcn_sdot4(d[4 * j + 2], xm[4 * j + 2], accP[m], false);
-            accQ[m] = __builtin_amdgcn_sdot4(d[4 * j + 3], xm[4 * j + 3], accQ[m], false);
-        }
+    for (int j = 0; j < 4; ++j) {
+        accP = __builtin_amdgcn_sdot4(d[4 * j + 0], xc[4 * j + 0], accP, false);
+        accQ = __builtin_amdgcn_sdot4(d[4 * j + 1], xc[4 * j + 1], accQ, false);
+        accP = __builtin_amdgcn_sdot4(d[4 * j + 2], xc[4 * j + 2], accP, false);
+        accQ = __builtin_amdgcn_sdot4(d[4 * j + 3], xc[4 * j + 3], accQ, false);
     }
 }
 
-// sum x over activation dwords [d0, d1) (multiples of 4) of each of the MT rows at xq
-// (row stride ldx dwords): lane l takes the 16-byte units d0 / 4 + l + 64 i, all loads
-// issued before the first v_dot4 (against 0x01010101), then the wave adds the lanes up.
-template <int MT, typename XP>
-__device__ __forceinline__ void slice_sums(XP* __restrict__ xq, const int ldx, const int d0, const int d1,
-                                           int (&sx)[MT]) {
+// sum x over activation dwords [d0, d1) (multiples of 4) of the row at xq: lane l takes the
+// 16-byte units d0 / 4 + l + 64 i, all loads issued before the first v_dot4 (against
+// 0x01010101), then the wave adds the lanes up.
+template <typename XP>
+__device__ __forceinline__ int slice_sum(XP* __restrict__ xq, const int d0, const int d1) {
     constexpr int R = 4;  // units per lane per round: one round covers K <= 16384
     const int lane = threadIdx.x & 63, u0 = d0 >> 2, u1 = d1 >> 2;
+    int t = 0;
+    for (int u = u0 + lane; u < u1 + lane; u += 64 * R) {
+        v4u x[R];
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        XP* __restrict__ xm = xq + m * ldx;
-        int t = 0;
-        for (int u = u0 + lane; u < u1 + lane; u += 64 * R) {
-            v4u x[R];
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const int ur = u + 64 * r;
-                if (ur < u1) {
-                    x[r][0] = xm[4 * ur + 0];
-                    x[r][1] = xm[4 * ur + 1];
-                    x[r][2] = xm[4 * ur + 2];
-                    x[r][3] = xm[4 * ur + 3];
-                } else {
-                    x[r] = v4u{0u, 0u, 0u, 0u};
-                }
+        for (int r = 0; r < R; ++r) {
+            const int ur = u + 64 * r;
+            if (ur < u1) {
+                x[r][0] = xq[4 * ur + 0];
+                x[r][1] = xq[4 * ur + 1];
+                x[r][2] = xq[4 * ur + 2];
+                x[r][3] = xq[4 * ur + 3];
+            } else {
+                x[r] = v4u{0u, 0u, 0u, 0u};
             }
-#pragma unroll
-            for (int r = 0; r < R; ++r)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) t = __builtin_amdgcn_sdot4((int)x[r][j], 0x01010101, t, false);
         }
-        sx[m] = wave_sum(t);
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) t = __builtin_amdgcn_sdot4((int)x[r][j], 0x01010101, t, false);
     }
+    return wave_sum(t);
 }
 
 // sum w x of one row from the two accumulators and the slice's sum x
@@ -176,23 +167,21 @@ __device__ __forceinline__ int row_dot(int accP, int accQ, int sx) { return accP
 // ends at chunk ce (num_records = ce KiB).  The chunk offset goes into the VGPR offset,
 // which the buffer unit range-checks (the SGPR offset is not checked), so the loads
 // that run past the range come back as zeros without touching memory.  That keeps
-// every load unconditional -- two batches of U chunks in flight -- while the math on
-// chunks >= ce is skipped.  The first two batches (A: chunks cb.., B: cb + U..) are
+// every load unconditional -- two batches of kU chunks in flight -- while the math on
+// chunks >= ce is skipped.  The first two batches (A: chunks cb.., B: cb + kU..) are
 // issued by gemv_preload, which a caller may run before other work (a prologue) to
 // overlap the weight latency with it.
-template <int U>
 __device__ __forceinline__ v4u gemv_load(__amdgpu_buffer_rsrc_t rsrc, const int lane_off, int c) {
     return __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(rsrc, lane_off + c * 1024, 0, kAuxNT));
 }
 
-template <int U>
 __device__ __forceinline__ void gemv_preload(__amdgpu_buffer_rsrc_t rsrc, const int lane_off, const int cb,
-                                             v4u (&A)[U], v4u (&B)[U], bool second = true) {
+                                             v4u (&A)[kU], v4u (&B)[kU], bool second = true) {
 #pragma unroll
-    for (int i = 0; i < U; ++i) A[i] = gemv_load<U>(rsrc, lane_off, cb + i);
+    for (int i = 0; i < kU; ++i) A[i] = gemv_load(rsrc, lane_off, cb + i);
     if (second) {
 #pragma unroll
-        for (int i = 0; i < U; ++i) B[i] = gemv_load<U>(rsrc, lane_off, cb + U + i);
+        for (int i = 0; i < kU; ++i) B[i] = gemv_load(rsrc, lane_off, cb + kU + i);
     }
 }
 
@@ -200,24 +189,24 @@ __device__ __forceinline__ void gemv_preload(__amdgpu_buffer_rsrc_t rsrc, const 
 // past ce is not issued (its loads would return zeros, but the wave still waits for them
 // before reusing the registers and at the closing barrier: decode 1.074 -> 1.055 ms/token).
 // Long streams (the rows kernel) issue every batch unconditionally (3 % faster there).
-template <int MT, int U, typename XP, bool SHORT = false>
+template <typename XP, bool SHORT = false>
 __device__ __forceinline__ void gemv_body(__amdgpu_buffer_rsrc_t rsrc, const int lane_off, XP* __restrict__ xq,
-                                          const int ldx, const int cb, const int ce, int (&accP)[MT],
-                                          int (&accQ)[MT], v4u (&A)[U], v4u (&B)[U]) {
-    for (int c = cb; c < ce; c += 2 * U) {
+                                          const int cb, const int ce, int& accP, int& accQ, v4u (&A)[kU],
+                                          v4u (&B)[kU]) {
+    for (int c = cb; c < ce; c += 2 * kU) {
 #pragma unroll
-        for (int i = 0; i < U; ++i)
-            if (c + i < ce) chunk_step<MT, XP>(A[i], xq + (c + i) * 16, ldx, accP, accQ);
-        if (!SHORT || c + 2 * U < ce) {
+        for (int i = 0; i < kU; ++i)
+            if (c + i < ce) chunk_step(A[i], xq + (c + i) * 16, accP, accQ);
+        if (!SHORT || c + 2 * kU < ce) {
 #pragma unroll
-            for (int i = 0; i < U; ++i) A[i] = gemv_load<U>(rsrc, lane_off, c + 2 * U + i);
+            for (int i = 0; i < kU; ++i) A[i] = gemv_load(rsrc, lane_off, c + 2 * kU + i);
         }
 #pragma unroll
-        for (int i = 0; i < U; ++i)
-            if (c + U + i < ce) chunk_step<MT, XP>(B[i], xq + (c + U + i) * 16, ldx, accP, accQ);
-        if (!SHORT || c + 3 * U < ce) {
+        for (int i = 0; i < kU; ++i)
+            if (c + kU + i < ce) chunk_step(B[i], xq + (c + kU + i) * 16, accP, accQ);
+        if (!SHORT || c + 3 * kU < ce) {
 #pragma unroll
-            for (int i = 0; i < U; ++i) B[i] = gemv_load<U>(rsrc, lane_off, c + 3 * U + i);
+            for (int i = 0; i < kU; ++i) B[i] = gemv_load(rsrc, lane_off, c + 3 * kU + i);
         }
     }
 }
@@ -236,28 +225,26 @@ __device__ __forceinline__ float emit1(const GemvProb& P, int rb, int r, int acc
 }
 
 // sx_pro: the token scale computed by a prologue (used instead of P.sx when >= 0)
-__device__ __forceinline__ void emit(const GemvArgs& a, const GemvProb& P, int rb, int m0, int m, int r, int acc,
+__device__ __forceinline__ void emit(const GemvArgs& a, const GemvProb& P, int rb, int r, int acc,
                                      float sx_pro = -1.0f) {
-    const int n = rb * kRowBlock + r, mg = m0 + m;
-    if (n >= P.N || mg >= a.M) return;
+    const int n = rb * kRowBlock + r;
+    if (n >= P.N) return;
     if (a.out_i32) {
-        static_cast<int*>(P.out)[(size_t)mg * P.ldo + n] = acc;
+        static_cast<int*>(P.out)[n] = acc;
     } else {
         const float sw = P.rs ? P.rs[n] : P.s_w;
-        const size_t o = (size_t)mg * P.ldo + n;
-        const float sx = sx_pro >= 0.0f ? sx_pro : P.sx[mg];
+        const float sx = sx_pro >= 0.0f ? sx_pro : P.sx[0];
         const float y = ((float)acc * sx) * sw;
-        static_cast<float*>(P.out)[o] = P.res ? P.res[o] + y : y;
+        static_cast<float*>(P.out)[n] = P.res ? P.res[n] + y : y;
     }
 }
 
-// PRO 0: activations quantised beforehand (qx); PRO 1 (M = 1): the workgroup first
+// PRO 0: activations quantised beforehand (qx); PRO 1: the workgroup first
 // quantises its problem's own fp32 row into LDS.  With PRO the host sizes workgroups so
 // that nw divides every problem's row-block count: all waves of a workgroup are live and
 // serve one problem (the prologue synchronises the workgroup).
-template <int MT, int PRO>
+template <int PRO>
 __global__ void __launch_bounds__(1024) gemv_rows_kernel(GemvArgs a) {
-    constexpr int U = MT == 1 ? 4 : 2;
     extern __shared__ __attribute__((aligned(16))) v4u lds_row[];
     const int lane = threadIdx.x & 63, nw = blockDim.x >> 6;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
@@ -267,16 +254,12 @@ __global__ void __launch_bounds__(1024) gemv_rows_kernel(GemvArgs a) {
     if (PRO == 0 && rbg >= a.total_rb) return;
     const GemvProb P = find_prob(a, rbg);
     const int rb = rbg - P.wg_begin;
-    const int m0 = blockIdx.y * MT;
-    const int C = P.C, ldx = C * 16;
+    const int C = P.C;
     const __amdgpu_buffer_rsrc_t rsrc =
         __builtin_amdgcn_make_buffer_rsrc((void*)(P.w + (size_t)rb * C * kRowBlock), 0, C * 1024, kBufDword3);
-    int accP[MT], accQ[MT], sx[MT];
-#pragma unroll
-    for (int m = 0; m < MT; ++m) accP[m] = accQ[m] = 0;
-    v4u A[U], B[U];
+    int accP = 0, accQ = 0;
+    v4u A[kU], B[kU];
     if constexpr (PRO != 0) {
-        static_assert(MT == 1, "the prologue quantises one token");
         // Several workgroups share a CU, most of them streaming: the waves of one in its
         // prologue issue first until the row is in LDS (metric plan 6.17 -> 6.28 TB/s).  Both
         // weight batches go out before the prologue (the loop holds both; same registers):
@@ -286,25 +269,24 @@ __global__ void __launch_bounds__(1024) gemv_rows_kernel(GemvArgs a) {
         RowRegs rr;
         const bool early = row_fits1(Q, blockDim.x);
         if (early) row_load1(Q, 0, rr);
-        gemv_preload<U>(rsrc, lane * 16, 0, A, B, true);
+        gemv_preload(rsrc, lane * 16, 0, A, B, true);
         RowSmem* sm = reinterpret_cast<RowSmem*>(lds_row + (Q.Kp >> 4));
         const QxRow qrow{lds_row, 4, 1};
         const float s_pro = early ? row_finish1(Q, rr, qrow, nullptr, nullptr, sm)
                                   : row_quantize<1>(Q, 0, qrow, nullptr, nullptr, sm);
         __syncthreads();
         __builtin_amdgcn_s_setprio(0);
-        slice_sums<MT, lint>((lint*)lds_row, ldx, 0, ldx, sx);
-        gemv_body<MT, U, lint>(rsrc, lane * 16, (lint*)lds_row, ldx, 0, C, accP, accQ, A, B);
-        emit(a, P, rb, 0, 0, lane, row_dot(accP[0], accQ[0], sx[0]), s_pro);
+        const int sx = slice_sum((lint*)lds_row, 0, C * 16);
+        gemv_body(rsrc, lane * 16, (lint*)lds_row, 0, C, accP, accQ, A, B);
+        emit(a, P, rb, lane, row_dot(accP, accQ, sx), s_pro);
     } else {
-        cint* xq = (cint*)(reinterpret_cast<const int*>(P.qx) + (size_t)m0 * ldx);
+        cint* xq = (cint*)(reinterpret_cast<const int*>(P.qx));
         // the activation loads for sum x go out before the weights, so waiting for them
         // does not wait for the weight batches
-        slice_sums<MT, cint>(xq, ldx, 0, ldx, sx);
-        gemv_preload<U>(rsrc, lane * 16, 0, A, B);
-        gemv_body<MT, U, cint>(rsrc, lane * 16, xq, ldx, 0, C, accP, accQ, A, B);
-#pragma unroll
-        for (int m = 0; m < MT; ++m) emit(a, P, rb, m0, m, lane, row_dot(accP[m], accQ[m], sx[m]));
+        const int sx = slice_sum(xq, 0, C * 16);
+        gemv_preload(rsrc, lane * 16, 0, A, B);
+        gemv_body(rsrc, lane * 16, xq, 0, C, accP, accQ, A, B);
+        emit(a, P, rb, lane, row_dot(accP, accQ, sx));
     }
 }
 
@@ -313,7 +295,7 @@ __global__ void __launch_bounds__(1024) gemv_rows_kernel(GemvArgs a) {
 // lane (at 16 waves the budget is 128 and the partials would spill to scratch).
 constexpr int kAttnMaxThreads = 640;
 
-// LDS of the KSPLIT kernel: [nw][MT][64] int partial sums, then (prologue) the
+// LDS of the KSPLIT kernel: [nw][64] int partial sums, then (prologue) the
 // quantised input row (Kp bytes) and the reduction scratch of the prologue.
 // PRO: 0 no prologue; 1 prologue quantising a row source (plain, RMSNorm, relu²·up,
 // relu²·up + sub-norm), 16 elements per thread; 3 / 4 the same with 4 / 8 consecutive
@@ -324,7 +306,7 @@ constexpr int kAttnMaxThreads = 640;
 // workgroup's row block holds both inputs of 32 outputs: it writes the FFN activation
 // a = relu(g)^2 * u of those 32 (g and u rounded as emit rounds y) and their f64 sum of
 // squares, the two inputs of the down projection's sub-norm.
-// Tail = AttnTail (M = 1, fp32 outputs): the attention partials of the token run in the
+// Tail = AttnTail (fp32 outputs): the attention partials of the token run in the
 // same launch (qkv_attn_block): the GEMV's outputs are also stored as epoch-tagged
 // device-coherent words, which the attention workgroups poll.
 struct NoTail {};
@@ -337,7 +319,7 @@ __device__ __forceinline__ void qkv_attn_block(const AttnTail& at, int total_rb)
 __device__ __forceinline__ unsigned attn_epoch(const AttnTail& at) {
     return __hip_atomic_load(at.done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) / at.natt + 1u;
 }
-template <int MT, int PRO, bool PAIR = false, typename Tail = NoTail>
+template <int PRO, bool PAIR = false, typename Tail = NoTail>
 __global__ void __launch_bounds__(PRO == 2 ? kAttnMaxThreads : 1024)
     gemv_ksplit_kernel(const float* pro_x, const float* pro_aux, const float* pro_aux2, int pro_K, int pro_mode,
                        float pro_eps, unsigned shape, unsigned nw_m, const v4u* w1, GemvArgs a, Tail at) {
@@ -345,7 +327,7 @@ __global__ void __launch_bounds__(PRO == 2 ? kAttnMaxThreads : 1024)
     if constexpr (SIG) {
         // the GEMV's workgroup count rides in the shape word (a launch of inline problems
         // has no C1), so the GEMV workgroups start without a kernel-argument load
-        static_assert(MT == 1 && !PAIR, "attention partials follow the one-token qkv GEMV");
+        static_assert(!PAIR, "attention partials follow the one-token qkv GEMV");
         const int total_rb = (int)(shape >> 8);
         if ((int)blockIdx.x >= total_rb) {
             qkv_attn_block<128, std::is_same<Tail, AttnTailLong>::value ? 2 : 1>(at, total_rb);
@@ -367,11 +349,9 @@ __global__ void __launch_bounds__(PRO == 2 ? kAttnMaxThreads : 1024)
     pro.K = pro_K;
     pro.mode = pro_mode;
     pro.eps = pro_eps;
-    constexpr int U = MT == 1 ? 4 : 2;
     extern __shared__ __attribute__((aligned(16))) int red[];
     const int lane = threadIdx.x & 63, nw = (int)(shape & 31u);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int m0 = blockIdx.y * MT;
     // With a prologue whose row fits one group per thread, the row's loads go out first
     // (they do not depend on the problem); then the problem, the weight resource and the
     // first weight batches, which stream in during the prologue's arithmetic.
@@ -391,20 +371,18 @@ __global__ void __launch_bounds__(PRO == 2 ? kAttnMaxThreads : 1024)
         early = attn_fits1(pro, blockDim.x);
         if (early) attn_load1(pro, rr);
     }
-    static_assert(!PAIR || (VEC && MT == 1), "the pair epilogue follows an E-element prologue");
+    static_assert(!PAIR || VEC, "the pair epilogue follows an E-element prologue");
     const WStream ws = w1 ? WStream{w1, C1, 0, 0} : find_stream(a, ninl, blockIdx.x);
     const int rb = blockIdx.x - ws.wg_begin;
-    const int C = ws.C, ldx = C * 16;
+    const int C = ws.C;
     // the wave's chunks [cb, ce): wave-uniform, in SGPRs (the buffer resource must not be
     // per-lane)
     const int cb = div_nw(wave * C, nw_m);
     const int ce = div_nw((wave + 1) * C, nw_m);
     const __amdgpu_buffer_rsrc_t rsrc =
         __builtin_amdgcn_make_buffer_rsrc((void*)(ws.w + (size_t)rb * C * kRowBlock), 0, ce * 1024, kBufDword3);
-    v4u A[U], B[U];
-    int accP[MT], accQ[MT], sx[MT];
-#pragma unroll
-    for (int m = 0; m < MT; ++m) accP[m] = accQ[m] = 0;
+    v4u A[kU], B[kU];
+    int accP = 0, accQ = 0, sx = 0;
     // The rest of the descriptor (epilogue): for inline problems the one at the index the
     // stream lookup chose; otherwise the table lookup.
     const int pj = __builtin_amdgcn_readfirstlane(ws.j);
@@ -419,16 +397,16 @@ __global__ void __launch_bounds__(PRO == 2 ? kAttnMaxThreads : 1024)
     }
     // sum x of the wave's slice: without a prologue its activation loads go out before
     // the weights (waiting for them then does not wait for the weight batches)
-    cint* xq = (cint*)(reinterpret_cast<const int*>(P.qx) + (size_t)m0 * ldx);
-    if constexpr (PRO == 0) slice_sums<MT, cint>(xq, ldx, cb * 16, ce * 16, sx);
+    cint* xq = (cint*)(reinterpret_cast<const int*>(P.qx));
+    if constexpr (PRO == 0) sx = slice_sum(xq, cb * 16, ce * 16);
     // With a prologue only the first batch is in flight during it (register budget); the
     // attention prologue holds its partials in registers first and issues it after their
     // combine.
-    if (PRO != 2 || !early) gemv_preload<U>(rsrc, lane * 16, cb, A, B, PRO == 0 && cb + U < ce);
-    // one token with a prologue: the residual and scale of wave 0's rows (the epilogue's),
+    if (PRO != 2 || !early) gemv_preload(rsrc, lane * 16, cb, A, B, PRO == 0 && cb + kU < ce);
+    // with a prologue: the residual and scale of wave 0's rows (the epilogue's),
     // requested now so that the epilogue does not wait for them
     float res_v = 0.0f, sw_v = P.s_w;
-    if constexpr (MT == 1 && PRO != 0 && !PAIR) {
+    if constexpr (PRO != 0 && !PAIR) {
         const int n = rb * kRowBlock + lane;
         if (wave == 0 && n < P.N) {
             if (P.res) res_v = P.res[n];
@@ -447,7 +425,7 @@ __global__ void __launch_bounds__(PRO == 2 ? kAttnMaxThreads : 1024)
     }
     float sx_pro = -1.0f;
     if constexpr (PRO != 0) {
-        v4u* lq = reinterpret_cast<v4u*>(red + nw * MT * kRowBlock);
+        v4u* lq = reinterpret_cast<v4u*>(red + nw * kRowBlock);
         RowSmem* sm = reinterpret_cast<RowSmem*>(lq + (pro.Kp >> 4));
         sm->fac = (lfloat*)(sm + 1);  // kAttnNorm factors follow
         const QxRow qrow{lq, 4, 1};
@@ -458,12 +436,12 @@ __global__ void __launch_bounds__(PRO == 2 ? kAttnMaxThreads : 1024)
             float v[4];
             attn_combine1(pro, rr, v);
             const float w[4] = {rr.w[0], rr.w[1], rr.w[2], rr.w[3]};
-            gemv_preload<U>(rsrc, lane * 16, cb, A, B, false);
+            gemv_preload(rsrc, lane * 16, cb, A, B, false);
             sx_pro = attn_norm1(pro, v, w, rr.live, lq, sm);
         }
-        if (cb + U < ce) {
+        if (cb + kU < ce) {
 #pragma unroll
-            for (int i = 0; i < U; ++i) B[i] = gemv_load<U>(rsrc, lane * 16, cb + U + i);
+            for (int i = 0; i < kU; ++i) B[i] = gemv_load(rsrc, lane * 16, cb + kU + i);
         }
         __syncthreads();
         if (VEC || (PRO == 2 && early)) {
@@ -471,16 +449,15 @@ __global__ void __launch_bounds__(PRO == 2 ? kAttnMaxThreads : 1024)
             // wave 0 subtracts the row's total, the other waves nothing (the epilogue adds
             // the waves)
             const int nq = VEC ? (pro.K / E + 63) >> 6 : nw;
-            sx[0] = wave == 0 ? slots_reduce(sm->qs, nq, [](int x, int y) { return x + y; }) : 0;
+            sx = wave == 0 ? slots_reduce(sm->qs, nq, [](int x, int y) { return x + y; }) : 0;
         } else {
-            slice_sums<MT, lint>((lint*)lq, ldx, cb * 16, ce * 16, sx);
+            sx = slice_sum((lint*)lq, cb * 16, ce * 16);
         }
-        gemv_body<MT, U, lint, true>(rsrc, lane * 16, (lint*)lq, ldx, cb, ce, accP, accQ, A, B);
+        gemv_body<lint, true>(rsrc, lane * 16, (lint*)lq, cb, ce, accP, accQ, A, B);
     } else {
-        gemv_body<MT, U, cint, true>(rsrc, lane * 16, xq, ldx, cb, ce, accP, accQ, A, B);
+        gemv_body<cint, true>(rsrc, lane * 16, xq, cb, ce, accP, accQ, A, B);
     }
-#pragma unroll
-    for (int m = 0; m < MT; ++m) red[(wave * MT + m) * kRowBlock + lane] = row_dot(accP[m], accQ[m], sx[m]);
+    red[wave * kRowBlock + lane] = row_dot(accP, accQ, sx);
     __syncthreads();
     if constexpr (PAIR) {
         if (threadIdx.x < kRowBlock) {  // wave 0; lanes 32.. only pad the reduction
@@ -505,7 +482,7 @@ __global__ void __launch_bounds__(PRO == 2 ? kAttnMaxThreads : 1024)
         }
         return;
     }
-    if (MT == 1 && PRO != 0 && !a.out_i32) {  // one token, fp32 outputs
+    if (PRO != 0 && !a.out_i32) {  // fp32 outputs
         if (threadIdx.x < kRowBlock) {
             const int r = threadIdx.x;
             int s = 0;
@@ -523,11 +500,11 @@ __global__ void __launch_bounds__(PRO == 2 ? kAttnMaxThreads : 1024)
         }
         return;
     }
-    for (int idx = threadIdx.x; idx < MT * kRowBlock; idx += blockDim.x) {
-        const int m = idx / kRowBlock, r = idx % kRowBlock;
+    if (threadIdx.x < kRowBlock) {
+        const int r = threadIdx.x;
         int s = 0;
-        for (int w = 0; w < nw; ++w) s += red[(w * MT + m) * kRowBlock + r];
-        emit(a, P, rb, m0, m, r, s, sx_pro);
+        for (int w = 0; w < nw; ++w) s += red[w * kRowBlock + r];
+        emit(a, P, rb, r, s, sx_pro);
     }
 }
 
@@ -736,12 +713,12 @@ int vec_elements(int K, int threads) {
 // problem count and the chunks per row of a one-problem launch, C <= 2^16), nw's reciprocal
 // and the weight tiles of a one-problem launch (null otherwise).
 static_assert(kInlineProbs <= 7, "the inline problem count takes 3 bits of the shape word");
-template <int MT, int PRO, bool PAIR = false>
+template <int PRO, bool PAIR = false>
 static void launch_ksplit(dim3 grid, int nw, size_t lds, hipStream_t s, const GemvArgs& a) {
     const QuantProb& P = a.pro;
     const bool one = a.ninl == 1;
     const unsigned shape = (unsigned)nw | ((unsigned)a.ninl << 5) | (one ? (unsigned)a.inl[0].C << 8 : 0u);
-    hipLaunchKernelGGL((gemv_ksplit_kernel<MT, PRO, PAIR>), grid, dim3((unsigned)(64 * nw)), lds, s, P.x, P.aux, P.aux2,
+    hipLaunchKernelGGL((gemv_ksplit_kernel<PRO, PAIR>), grid, dim3((unsigned)(64 * nw)), lds, s, P.x, P.aux, P.aux2,
                        P.K, P.mode, P.eps, shape, nw_reciprocal(nw), one ? a.inl[0].w : nullptr, a, NoTail{});
 }
 
@@ -762,7 +739,7 @@ hipError_t launch_gemv(const GemvArgs& args, GemvShape shape, hipStream_t s) {
         if (shape.ksplit || a.total_rb % shape.nw) return hipErrorInvalidValue;
         const dim3 grid((unsigned)(a.total_rb / shape.nw), 1);
         const size_t lds = (size_t)a.pro.Kp + sizeof(RowSmem);  // pro.Kp: the largest Kp of the problems
-        hipLaunchKernelGGL((gemv_rows_kernel<1, 1>), grid, block, lds, s, a);
+        hipLaunchKernelGGL((gemv_rows_kernel<1>), grid, block, lds, s, a);
     } else if (a.has_pro && a.pair_a) {  // gate/up pair: an E-element prologue
         const QuantProb& P = a.pro;
         const int E = vec_elements(P.K, 64 * shape.nw);
@@ -771,9 +748,9 @@ hipError_t launch_gemv(const GemvArgs& args, GemvShape shape, hipStream_t s) {
             return hipErrorInvalidValue;
         const dim3 grid((unsigned)a.total_rb, 1);
         const size_t lds = (size_t)shape.nw * kRowBlock * sizeof(int) + (size_t)P.Kp + sizeof(RowSmem);
-        if (E == 4) launch_ksplit<1, 3, true>(grid, shape.nw, lds, s, a);
-        else if (E == 8) launch_ksplit<1, 4, true>(grid, shape.nw, lds, s, a);
-        else launch_ksplit<1, 6, true>(grid, shape.nw, lds, s, a);
+        if (E == 4) launch_ksplit<3, true>(grid, shape.nw, lds, s, a);
+        else if (E == 8) launch_ksplit<4, true>(grid, shape.nw, lds, s, a);
+        else launch_ksplit<6, true>(grid, shape.nw, lds, s, a);
     } else if (a.has_pro) {  // single token, prologue-quantised input: KSPLIT shape only
         if (!shape.ksplit) return hipErrorInvalidValue;
         const dim3 grid((unsigned)a.total_rb, 1);
@@ -783,19 +760,19 @@ hipError_t launch_gemv(const GemvArgs& args, GemvShape shape, hipStream_t s) {
         const bool vec = P.K % 64 == 0 && aligned16(P.x) && aligned16(P.aux) && aligned16(P.aux2);
         if (a.pro.mode == kAttnNorm) {
             lds += (size_t)(a.pro.K / a.pro.attn_hd) * (a.pro.attn_S + 1) * sizeof(float);
-            launch_ksplit<1, 2>(grid, nw, lds, s, a);
+            launch_ksplit<2>(grid, nw, lds, s, a);
         } else if (const int E = vec ? vec_elements(P.K, (int)block.x) : 0) {
-            if (E == 4) launch_ksplit<1, 3>(grid, nw, lds, s, a);
-            else if (E == 8) launch_ksplit<1, 4>(grid, nw, lds, s, a);
-            else launch_ksplit<1, 6>(grid, nw, lds, s, a);
+            if (E == 4) launch_ksplit<3>(grid, nw, lds, s, a);
+            else if (E == 8) launch_ksplit<4>(grid, nw, lds, s, a);
+            else launch_ksplit<6>(grid, nw, lds, s, a);
         } else {
-            launch_ksplit<1, 1>(grid, nw, lds, s, a);
+            launch_ksplit<1>(grid, nw, lds, s, a);
         }
     } else if (shape.ksplit) {
-        launch_ksplit<1, 0>(dim3((unsigned)a.total_rb), shape.nw, (size_t)shape.nw * kRowBlock * sizeof(int), s, a);
+        launch_ksplit<0>(dim3((unsigned)a.total_rb), shape.nw, (size_t)shape.nw * kRowBlock * sizeof(int), s, a);
     } else {
         const dim3 grid((unsigned)((a.total_rb + shape.nw - 1) / shape.nw));
-        hipLaunchKernelGGL((gemv_rows_kernel<1, 0>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((gemv_rows_kernel<0>), grid, block, 0, s, a);
     }
     return hipGetLastError();
 }
@@ -805,7 +782,7 @@ static void launch_qkv_attn(dim3 grid, int nw, size_t lds, hipStream_t s, const 
     const QuantProb& P = a.pro;
     const unsigned shape = (unsigned)nw | ((unsigned)a.ninl << 5) | ((unsigned)a.total_rb << 8);
     auto go = [&](auto tail) {
-        hipLaunchKernelGGL((gemv_ksplit_kernel<1, PRO, false, decltype(tail)>), grid, dim3((unsigned)(64 * nw)), lds, s,
+        hipLaunchKernelGGL((gemv_ksplit_kernel<PRO, false, decltype(tail)>), grid, dim3((unsigned)(64 * nw)), lds, s,
                            P.x, P.aux, P.aux2, P.K, P.mode, P.eps, shape, nw_reciprocal(nw),
                            static_cast<const v4u*>(nullptr), a, tail);
     };
@@ -849,9 +826,9 @@ hipError_t gemv_attn_capacity(int K, int Kp, int nw, int Gq, int* workgroups) {
     if (E == 0) return hipErrorInvalidValue;
     const size_t lds = std::max((size_t)nw * kRowBlock * sizeof(int) + (size_t)Kp + sizeof(RowSmem),
                                 (size_t)Gq * (sizeof(AttnTileLds<128>) + sizeof(AttnRun)) + (size_t)(Gq + 2) * 128 * sizeof(float));
-    const void* k = E == 4   ? reinterpret_cast<const void*>(&gemv_ksplit_kernel<1, 3, false, AttnTail>)
-                    : E == 8 ? reinterpret_cast<const void*>(&gemv_ksplit_kernel<1, 4, false, AttnTail>)
-                             : reinterpret_cast<const void*>(&gemv_ksplit_kernel<1, 6, false, AttnTail>);
+    const void* k = E == 4   ? reinterpret_cast<const void*>(&gemv_ksplit_kernel<3, false, AttnTail>)
+                    : E == 8 ? reinterpret_cast<const void*>(&gemv_ksplit_kernel<4, false, AttnTail>)
+                             : reinterpret_cast<const void*>(&gemv_ksplit_kernel<6, false, AttnTail>);
     int per_cu = 0, dev = 0, cus = 0;
     hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, 64 * nw, lds);
     if (e == hipSuccess) e = hipGetDevice(&dev);

@@ -99,17 +99,17 @@ struct QuantProb {
     int blocked;         // qx layout: 0 rows, else the rows of a block (see qx_blocked)
 };
 
-// ---- one GEMV problem (a ternary matrix applied to M tokens) -------------------
+// ---- one GEMV problem (a ternary matrix applied to one token) ------------------
 struct GemvProb {
     const v4u* w;        // weight tiles
-    const int8_t* qx;    // quantised activations [Mpad][Kp] (layout above)
-    const float* sx;     // [Mpad] per-token scales (unused for int32 output)
+    const int8_t* qx;    // quantised activations [Kp] (layout above)
+    const float* sx;     // the token's scale (unused for int32 output)
     const float* rs;     // [N] per-row scales or nullptr (then s_w)
-    void* out;           // float y[M][ldo] or int32 acc[M][ldo]
+    void* out;           // float y[N] or int32 acc[N]
     float s_w;
-    int N, C, ldo;
+    int N, C;
     int wg_begin;        // first global row block of this problem (prefix sum over problems)
-    const float* res;    // optional fp32 [M][ldo] added to y (may alias out)
+    const float* res;    // optional fp32 [N] added to y (may alias out)
     const float* xs;     // has_pro == 2: the problem's own fp32 input row [K] (quantised in the prologue)
     int K;               // has_pro == 2: its length
 };
@@ -211,7 +211,7 @@ struct QuantArgs {
 // ---- one GEMM problem (int8 MFMA path, M > kGemvMaxM) ---------------------------
 struct GemmArgs {
     const v4u* w;        // weight tiles (Np rows, C chunks)
-    const int8_t* qx;    // [Mpad][Kp], Mpad a multiple of gemm_bm(M)
+    const int8_t* qx;    // [Mpad][Kp], Mpad a multiple of gemm_bm(M) (M <= 8: of qx_block_rows(M))
     const float* sx;     // [Mpad]
     const float* rs;     // [N] per-row scales or nullptr (then s_w)
     void* out;           // float y[M][ldo] or int32 acc[M][ldo]
@@ -325,8 +325,8 @@ inline bool skinny_ok(int M, int units, bool split) {
 inline __host__ __device__ int qx_block_rows(int M) { return M <= 2 ? 2 : M <= 4 ? 4 : M <= kSkinnyRows ? 8 : 16; }
 inline int qx_blocked(int M) { return M > kGemvMaxM ? qx_block_rows(M) : 0; }
 
-// rows of the GEMM workgroup tile for M tokens (the activations are padded to it past 8 tokens)
-inline int gemm_bm(int M) { return M <= kSkinnyRows ? 16 : M <= 64 ? 64 : M <= 128 ? 128 : 256; }
+// rows of the GEMM workgroup tile for M > 8 tokens (the activations are padded to it)
+inline int gemm_bm(int M) { return M <= 64 ? 64 : M <= 128 ? 128 : 256; }
 // The GEMM epilogues address one row tile of the output (and residual) with 32-bit byte
 // offsets and buffer ranges: a tile of gemm_bm(M) rows of ldo floats must span < 2^31 bytes.
 // (The skinny kernel addresses its outputs row by row.)

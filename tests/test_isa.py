@@ -105,7 +105,7 @@ def test_no_inline_asm_lane_reads(gemv, gemm):
 
 
 def test_gemv_rows_reads_activations_with_scalar_loads(gemv):
-    (n,) = [n for n in gemv if "gemv_rows_kernelILi1ELi0E" in n]
+    (n,) = [n for n in gemv if "gemv_rows_kernelILi0E" in n]
     t = gemv[n]
     assert "s_load_dwordx16" in t or "s_load_dwordx8" in t
     # the only per-lane activation loads are the 16-byte ones of the sum-x pass (one
