@@ -569,10 +569,9 @@ class _DeviceModel:
         if M == 1 and self.trace is None:
             st = self._state(1)
             try:
-                step = self._step_graph(st)
-            finally:  # not the capture's stream, nor an earlier caller's: as after an eager forward
-                self.hip._bind_stream()
-            step.replay()
+                self._step_graph(st).replay()
+            finally:  # (while the step runs) the caller's stream, as after an eager forward: not
+                self.hip._bind_stream()  # the capture's, nor an earlier caller's
         else:
             st = self._enqueue(M, pos_base=1 << 30, out_cap=0)
         if M == 1:
