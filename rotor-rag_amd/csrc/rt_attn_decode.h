@@ -382,13 +382,15 @@ __device__ __forceinline__ void attn_tile2(SRC qh, SRC kn, SRC vn, float c, floa
         if (live) {
             bool skip = false;
             if (r > 0) {
-                const float al = run->alpha;
-                skip = al == kAttnSkip;
-                if (al >= 0.0f || al != al) {
+                // (uniform, in an SGPR: the branches below stay scalar)
+                const int ab = __builtin_amdgcn_readfirstlane(__float_as_int(run->alpha));
+                skip = ab == __builtin_bit_cast(int, kAttnSkip);
+                if (ab == __builtin_bit_cast(int, kAttnFirst)) {
+                    o0 = o1 = 0.0f;
+                } else if (!skip) {
+                    const float al = __int_as_float(ab);
                     o0 *= al;
                     o1 *= al;
-                } else if (!skip) {
-                    o0 = o1 = 0.0f;
                 }
             }
             // the new key, the block's last, is added after the cached ones (the same order)
