@@ -139,9 +139,9 @@ int rt_linear_f32(rt_ctx* ctx, const rt_weights* w, const float* x, int M, float
  * grown on demand), this entry point stages them in a static device buffer of
  * RT_NOALLOC_SCRATCH_BYTES (16 MiB) that every device holds from the library's load until
  * the process ends; M = 1 needs none (one launch quantises in the GEMV prologue).  Inputs
- * whose staged activations, Mpad * round_up(K, 64) + 4 * Mpad bytes (Mpad = M rounded up to
- * the GEMV token group or GEMM tile: 2048 x 6912 fits), exceed the buffer are rejected with
- * RT_EINVAL.  All calls on one device share its buffer: calls that overlap on one GPU (two
+ * whose staged activations, Mpad * round_up(K, 64) + 4 * Mpad bytes, exceed the buffer are
+ * rejected with RT_EINVAL; Mpad is M rounded up to 2, 4 or 8 for M <= 8, to 64 for M <= 64, to
+ * 128 for M <= 128 and to a multiple of 256 past that (2048 x 6912 fits).  All calls on one device share its buffer: calls that overlap on one GPU (two
  * streams, two host threads) race, so the caller serialises them. */
 #define RT_NOALLOC_SCRATCH_BYTES (16u << 20)
 int rt_linear_f32_noalloc(rt_ctx* ctx, const rt_weights* w, const float* x, int M, float* y);
@@ -318,9 +318,9 @@ int rt_attention(rt_ctx* ctx, const float* q, const float* k_cache, const float*
                  int Hkv, int hd, int Lmax, const int* pos);
 
 /* Decode form of rt_attention for one query (M = 1, flash-decoding): the keys, in blocks of
- * 64, are dealt to at most 10 workgroups per query head; each writes a partial softmax result to `workspace` (at least
- * rt_attention_decode_workspace(H, hd, Lmax) bytes of device memory, no initialisation
- * needed), then a second launch combines them into out [H*hd].  head_dim 64 or 128.
+ * 64, are dealt to at most 10 workgroups per query head; each writes a partial softmax result
+ * to `workspace` (at least rt_attention_decode_workspace(H, hd, Lmax) bytes of device memory,
+ * no initialisation needed), then a second launch combines them into out [H*hd].  head_dim 64 or 128.
  * rt_attention_decode_partials stops after the first launch; a fused plan with source
  * RT_SRC_ATTN_NORM then combines the partials in its prologue. */
 size_t rt_attention_decode_workspace(int H, int hd, int Lmax);

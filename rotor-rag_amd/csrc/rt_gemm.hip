@@ -1186,7 +1186,11 @@ hipError_t launch_gemm(const GemmArgs& a, hipStream_t s) {
     // tiles / this: 2560 x 2560 at 128 / 300 / 512 tokens 13.7 / 11.5 / 12.1 -> 7.4 / 8.1 / 11.4 us,
     // 2560 x 6912 at 201 / 512 22.2 / 23.9 -> 13.9 / 20.9, 640 x 2560 at 1024 11.2 -> 8.1; past the
     // line they lose (6912 x 2560 at 512, 864 tiles: 18.2 -> 21.0), and for long prompts of
-    // narrow matrices the line is one a CU (1111 x 2050 at 1024, 288 tiles: 10.6 -> 10.8).
+    // narrow matrices the line is one a CU (1111 x 2050 at 1024, 288 tiles: 10.6 -> 10.8).  Single
+    // problems only: a plan's launch has no row tiles of this kind, and takes the larger ones also
+    // where they are slower (a plan of one problem / this, launch alone: 2560 x 2560 at 100 / 300
+    // tokens 13.9 / 10.9 against 7.1 / 7.3 us, 2560 x 6912 29.3 / 21.6 against 12.3 / 12.6, 6912 x
+    // 2560 14.3 / 15.4 against 7.5 / 15.2).
     const long long tiles64 = (long long)units * ((a.M + 63) / 64);
     if (a.M <= 64 || tiles64 <= kSplitkOneRound / 2 || (tiles64 <= kSplitkOneRound && a.M <= 768)) {
         GemmArgs one = a;

@@ -308,7 +308,10 @@ __device__ __forceinline__ int wave_sum(int v) {
 }
 constexpr int kGemvMaxM = 1;  // one token: VALU GEMV; beyond: MFMA GEMM
 // gemm_skinny_kernel's launches.  Up to 8 tokens always.  Up to 16 unless a long problem of the
-// group is to be cut into split-K parts (what rt_plan_describe reports of such a plan is kept).
+// group is to be cut into split-K parts: there the line is not where the times cross (launch
+// alone, 20 layers in rotation, split-K / this at 9 and 16 tokens: the seven projections of a
+// 2560 / 6912 layer 12.3 / 9.4 and 12.3 / 9.6 us, o and down 9.5 / 6.1 and 9.5 / 6.2, a 1024 / 4096
+// layer 8.6 / 5.0 and 8.7 / 5.1), but where the plans' tests have the parts.
 // Up to 32 with at most one workgroup per CU (two 16-row blocks a workgroup; launch alone, 20
 // layers in rotation, split-K / this: q/k/v 7.2 / 6.3, down 12.6 / 8.7 us, but a layer's 356
 // row blocks 12.6 / 15.8).
@@ -378,8 +381,6 @@ long long gemm_tile_count(int cfg, int M, int N);
 // problem), tile2p [total_tiles] problem of every tile, cfg from gemm_tile_cfg.
 hipError_t launch_gemm_tiles(const GemmArgs* dev, const int* tile2p, const int* bnd, int nb, int total_tiles, int cfg,
                              hipStream_t s);
-// M <= 64 (gemm_bm(M) == 64): G problems in one launch over all their row blocks;
-// dev [G] (wg_begin set), rb2p [total_rb] problem of every global row block.
 // The M = 1 qkv plan (three inline problems, E-element RMSNorm prologue, 256 Gq threads per
 // workgroup) with the attention partials of its token in the same launch.
 hipError_t launch_gemv_attn(const GemvArgs& args, const AttnTail& at, int Hkv, int hd, GemvShape shape,
@@ -387,11 +388,13 @@ hipError_t launch_gemv_attn(const GemvArgs& args, const AttnTail& at, int Hkv, i
 // Workgroups of that launch (source row of K elements, nw waves, Gq query heads per KV head)
 // that the current device holds at once.
 hipError_t gemv_attn_capacity(int K, int Kp, int nw, int Gq, int* workgroups);
+// 1 < M <= 64: the split-K launch of G problems over all their row blocks (or parts of them): dev
+// (wg_begin set), rb2p [total_rb] descriptor of every unit.
+hipError_t launch_gemm_group(const GemmArgs* dev, const int* rb2p, const int* bnd, int nb, int total_rb,
+                             hipStream_t s);
 // The same for gemm_skinny_kernel (skinny_ok; minC, maxC: the fewest and most chunks of a problem).
 hipError_t launch_gemm_skinny(const GemmArgs* dev, const int* rb2p, const int* bnd, int nb, int M, int units, int minC,
                               int maxC, hipStream_t s);
-hipError_t launch_gemm_group(const GemmArgs* dev, const int* rb2p, const int* bnd, int nb, int total_rb,
-                             hipStream_t s);
 // Once per device (current) before any launch: the function attributes the GEMM kernels
 // and the prefill attention need (dynamic LDS above 64 KiB).
 hipError_t gemm_prepare_device();

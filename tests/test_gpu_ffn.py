@@ -51,8 +51,8 @@ def test_act_rmsnorm_quantize_bit_exact(hip, M, K):
 
 @pytest.mark.parametrize("M,K", [(1, 2560), (9, 2560), (300, 6912), (2, 4160), (3, 8192), (2, 8256)])
 def test_act_quantize_without_value_outputs(hip, M, K):
-    """Without the fp32 value outputs the quantiser takes its vectorised row kernel (K % 64
-    == 0, K <= 8192, 4 or 8 elements per thread); q and s stay bit-exact."""
+    """Without the fp32 value outputs the quantiser takes its wide row kernel up to K = 8192 (any
+    width; wider rows the general one); q and s stay bit-exact."""
     import torch
 
     rng = np.random.default_rng(11 * K + M)
@@ -427,8 +427,7 @@ def test_output_ssq_rejects_other_plans(hip):
 
 
 # (M, F, K): the tile the pair epilogue runs on -- 128 x 128 (M <= 128), 64 x 128 promoted to
-# 128 x 128 (few tiles), 192 x 128, 256 x 128 (the 512-token prefill), and 256 x 256 taken as
-# 256 x 128 (M = 2048)
+# 128 x 128 (few tiles), 192 x 128, 256 x 128 (the 512-token prefill) and 256 x 256 (M = 2048)
 @pytest.mark.parametrize("M,F,K", [(70, 256, 128), (200, 512, 256), (300, 1024, 640), (512, 6912, 2560),
                                    (2048, 6912, 2560)])
 def test_act_gate_up_pair_equals_separate(hip, M, F, K):

@@ -171,7 +171,7 @@ def test_rope_append_parts(hip, M, pos0, H, Hkv, hd):
                                                 (511, 20, 5, 128, 640), (639, 20, 5, 128, 640), (100, 4, 4, 64, 130),
                                                 (527, 20, 5, 128, 640), (528, 20, 5, 128, 640), (600, 20, 5, 128, 640),
                                                 (606, 20, 5, 128, 640), (95, 8, 2, 64, 200),
-                                                (700, 8, 2, 64, 1000)])  # 16 blocks: general prologue path
+                                                (700, 8, 2, 64, 1000)])  # 16 blocks, two to a split
 def test_attention_decode_split(hip, pos0, H, Hkv, hd, Lmax):
     """Flash-decoding form equals the single-workgroup form; the workspace is reusable."""
     import torch
@@ -719,7 +719,7 @@ def test_stale_kv_cache_rejected(small_model):
         model.forward(np.array([6], np.int32), past_kv_cache=d1)
 
 
-# ---- prompts longer than the GEMV's 8 tokens: the prefill runs the quantiser launches, the
+# ---- prompts longer than the few tokens of gemm_skinny_kernel: the prefill runs the quantiser launches, the
 # grouped split-K / tile GEMM plans, residual-aliased linears and rt_attention (the MFMA
 # prefill kernel for head_dim 128) -------------------------------------------------------
 HD128 = dict(vocab_size=1000, d_model=512, n_layers=2, n_heads=4, n_kv_heads=2, d_ff=1024, rope_theta=500000.0)
