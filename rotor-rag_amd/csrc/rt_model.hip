@@ -165,10 +165,10 @@ __global__ void __launch_bounds__(256) attention_kernel(const float* __restrict_
 // K and V go from memory to registers 16 at a time, so a wave needs no LDS slice and 210
 // registers: two workgroups share a CU and one's softmax, waits and merge run under the
 // other's MFMAs (with K and V in LDS, 32 KiB a wave, each SIMD had one wave).  Before / now, 20
-// heads of 128 over 5: 1024 tokens after 1024 228 -> 199 us (matrix cores busy 74 % of the CUs'
-// cycles), 512 / 256 / 64 tokens from an empty cache 32.5 / 19.7 / 11.7 -> 30.2 / 15.1 / 9.0, 2
-// tokens after 1400 70 -> 56; V by one 16-byte load for the four blocks of O^T instead of four
-// 4-byte ones 207 -> 199.
+// heads of 128 over 5: 1024 tokens after 1024 228 -> 199 us (matrix cores 74 % busy in the busy
+// CUs; 640 workgroups fill the 512 slots 69 % of the launch), 512 / 256 / 64 tokens from an empty
+// cache 32.5 / 19.7 / 11.7 -> 30.2 / 15.1 / 9.0, 2 tokens after 1400 70 -> 56; V by one 16-byte
+// load for the four blocks of O^T instead of four 4-byte ones 207 -> 199.
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(3))) void lds_void;
