@@ -20,6 +20,8 @@
 // use the operation order of attn_combine_element, so they give identical values.
 #pragma once
 
+#include <cfloat>
+
 #include "rt_internal.h"
 
 namespace rt {
@@ -53,9 +55,12 @@ struct AttnRun {
     float alpha, m, z, pad;
 };
 typedef __attribute__((address_space(3))) AttnRun lds_run;
-// alpha of a block that adds nothing, and of the first that adds something after such blocks
-// (the sums start again: what theirs hold, 0 times the values, may be NaN).  Telling them apart
-// costs the launch 0.1 us (20 heads of 128 at position 1537 of 2048: 16.3 -> 16.4).
+// alpha of a block whose scores are all -inf: it adds nothing, as an empty partial in the combine;
+// and of the first block that adds something after such ones: the sums start again (theirs, 0 times
+// the values, may be NaN).  The running maximum starts at -FLT_MAX, so that such a block's
+// exponentials are 0, and NaN scores leave a maximum that the combine takes, with sums of NaN.
+// As selects and one scalar mark this costs the joint launch 12.28 -> 12.36 us (20 heads of 128 at
+// position 1537 of 2048); as branches 12.6, as a second, careful pass where one is needed 12.8.
 constexpr float kAttnSkip = -2.0f, kAttnFirst = -1.0f;
 
 // The tile's LDS is reached through a local-address-space pointer: through a generic one,
@@ -320,7 +325,7 @@ __device__ __forceinline__ void attn_tile2(SRC qh, SRC kn, SRC vn, float c, floa
         for (int e = t; e < HD; e += 256) sm->qs[e] = qh[e];
     }
     attn_lds_barrier();
-    float o0 = 0.f, o1 = 0.f, mrun = -INFINITY, zrun = 0.f;  // mrun, zrun: wave 0's (zrun in lane 63)
+    float o0 = 0.f, o1 = 0.f, mrun = -FLT_MAX, zrun = 0.f;  // mrun, zrun: wave 0's (zrun in lane 63)
     for (int r = 0; r < rounds; ++r, j0 += step) {
         const bool live = j0 <= pos;                   // the tile's block holds a key
         const bool more = j0 + step <= pos;            // and so does its next one
@@ -351,27 +356,14 @@ __device__ __forceinline__ void attn_tile2(SRC qh, SRC kn, SRC vn, float c, floa
                            ? (((sm->part[0][lane] + sm->part[1][lane]) + (sm->part[2][lane] + sm->part[3][lane])) * scale)
                            : -INFINITY;
             const float bm = lane63(wave_reduce63(sc, -INFINITY, [](float x, float y) { return fmaxf(x, y); }));
-            float mx = fmaxf(mrun, bm), p = lane < nk ? expf(sc - mx) : 0.0f;
-            float al = r > 0 ? expf(mrun - mx) : 0.0f;  // (the first block's sums start from zero)
-            if (!(bm > -INFINITY)) {
-                // all scores -inf: the block adds nothing, as an empty partial in the combine.  A
-                // NaN makes the sums NaN, and the maximum too where there is no other (one of
-                // -inf would have the combine leave the split out).
-                if (!__any(sc != sc)) {
-                    mx = mrun;
-                    p = 0.0f;
-                    al = kAttnSkip;
-                } else if (mx == -INFINITY) {
-                    mx = __builtin_nanf("");
-                }
-            } else if (r > 0 && mrun == -INFINITY) {
-                al = kAttnFirst;
-            }
+            const float mx = fmaxf(mrun, bm);
+            const float p = lane < nk ? expf(sc - mx) : 0.0f;
             const float z = wave_reduce63(p, 0.0f, [](float x, float y) { return x + y; });
             sm->pr[lane] = p;
-            if (r > 0) {
-                if (lane == 63) run->alpha = al;
-                zrun = fmaf(zrun, al == kAttnSkip ? 1.0f : al, z);
+            if (r > 0) {  // (the first block's sums start from zero)
+                const float al = expf(mrun - mx);
+                if (lane == 63) run->alpha = bm == -INFINITY ? kAttnSkip : mrun == -FLT_MAX ? kAttnFirst : al;
+                zrun = fmaf(zrun, al, z);
             } else {
                 zrun = z;
             }
@@ -382,16 +374,10 @@ __device__ __forceinline__ void attn_tile2(SRC qh, SRC kn, SRC vn, float c, floa
         if (live) {
             bool skip = false;
             if (r > 0) {
-                // (uniform, in an SGPR: the branches below stay scalar)
-                const int ab = __builtin_amdgcn_readfirstlane(__float_as_int(run->alpha));
-                skip = ab == __builtin_bit_cast(int, kAttnSkip);
-                if (ab == __builtin_bit_cast(int, kAttnFirst)) {
-                    o0 = o1 = 0.0f;
-                } else if (!skip) {
-                    const float al = __int_as_float(ab);
-                    o0 *= al;
-                    o1 *= al;
-                }
+                const float al = run->alpha;
+                o0 = al < 0.0f ? (al == kAttnFirst ? 0.0f : o0) : o0 * al;
+                o1 = al < 0.0f ? (al == kAttnFirst ? 0.0f : o1) : o1 * al;
+                skip = __builtin_amdgcn_readfirstlane(__float_as_int(al)) == __builtin_bit_cast(int, kAttnSkip);
             }
             // the new key, the block's last, is added after the cached ones (the same order)
             const int nc = skip ? 0 : holds_new ? lp : nk;
@@ -435,13 +421,13 @@ __device__ __forceinline__ void attn_tile2(SRC qh, SRC kn, SRC vn, float c, floa
     if (tile == 0 && g == 0) {
         float o = sm->ored[d];
         for (int gg = 1; gg < G; ++gg) o += sm->ored[gg * HD + d];
-        // either tile may have no block that counts (m = -inf, z = 0)
+        // either tile may have no block that counts (m = -FLT_MAX, z = 0)
         const float m0 = run->m, m1 = run1->m, m = fmaxf(m0, m1);
-        const float f0 = m0 == -INFINITY ? 0.0f : expf(m0 - m), f1 = m1 == -INFINITY ? 0.0f : expf(m1 - m);
+        const float f0 = expf(m0 - m), f1 = expf(m1 - m);
         float ob = sm1->ored[d];
         for (int gg = 1; gg < G; ++gg) ob += sm1->ored[gg * HD + d];
-        if (m0 == -INFINITY) o = 0.0f;
-        if (m1 == -INFINITY) ob = 0.0f;
+        if (m0 == -FLT_MAX) o = 0.0f;
+        if (m1 == -FLT_MAX) ob = 0.0f;
         wp[d] = fmaf(f1, ob, f0 * o);
         if (d == 0) {
             wp[HD] = m;
