@@ -31,12 +31,18 @@ LINEAR_CASES = [
     (3, 77, 130),
     (9, 65, 63),
     (2, 129, 1000),
-    # int8-MFMA GEMM path (M > 8)
+    # int8-MFMA GEMM path (M > 1): few tokens above; split-K, in 64-row tiles past 64 tokens
     (16, 640, 2560),
     (100, 300, 256),
     (129, 2560, 2560),
     (256, 6912, 2560),
     (512, 2560, 6912),
+    # too many 64 x 64 tiles for that: the tile kernel's 128 x 128 (M <= 128 and past it), 64 x 128 and
+    # 256 x 128 tiles
+    (100, 16500, 130),
+    (900, 2500, 320),
+    (800, 1900, 320),
+    (1100, 3400, 200),
     (2048, 6912, 2560),  # cfg 3 (gate/up)
     (2048, 2560, 6912),  # cfg 3 (down): 128 x 160 regions, K split over the waves
     (2000, 2500, 4224),  # regions with rows past M and a last region of 100 columns, 33 chunks per K half
@@ -101,9 +107,12 @@ def test_linear_f32_parity(hip, M, N, K):
     assert np.array_equal(y, y_exact)
 
 
-@pytest.mark.parametrize("M,N,K", [(2048, 2560, 6912), (300, 2560, 2560), (2000, 2500, 4224), (2000, 2500, 4160)])
+# regions, split-K row tiles, and each shape of the tile kernel
+@pytest.mark.parametrize("M,N,K", [(2048, 2560, 6912), (300, 2560, 2560), (2000, 2500, 4224), (2000, 2500, 4160),
+                                   (100, 16500, 130), (900, 2500, 320), (800, 1900, 320), (1100, 3400, 200),
+                                   (2048, 6912, 128)])
 def test_gemm_residual_epilogue(hip, M, N, K):
-    """The GEMM epilogue with a residual (region and tile kernels): y = r + ((acc s_x) s_w),
+    """The GEMM epilogue with a residual (region, split-K and tile kernels): y = r + ((acc s_x) s_w),
     each a separate fp32 operation."""
     import torch
 
@@ -131,7 +140,7 @@ def test_extreme_accumulators(hip):
     assert acc.tolist() == [[-128 * K, 128 * K, 0], [127 * K, -127 * K, 0]]
 
 
-@pytest.mark.parametrize("M", [3, 16, 100])  # GEMV, split-K GEMM, tile GEMM
+@pytest.mark.parametrize("M", [1, 3, 16, 33, 100])  # GEMV, skinny GEMM, split-K GEMM and its row tiles
 def test_error_codes_in_weights_decode_to_zero(hip, M):
     import torch
 

@@ -99,9 +99,10 @@ def test_noalloc_few_tokens_of_long_rows(hip, M, K):
 # The allocation-free call captured in a HIP graph: every replay, each on a new input written
 # in place between replays (with the process's own eager launches and synchronisations in
 # between), equals the eager rt_linear_f32 bit for bit.  The child process captures each
-# shape BEFORE any launch of its kernels in that process (the tile GEMM, the split-K GEMM, the
-# 128 x 160 region GEMM, the one-launch M = 1 GEMV): the first launch of a kernel then happens
-# under the capture.
+# shape BEFORE any launch of its kernels in that process (the split-K GEMM in row tiles and on 37
+# tokens, the 128 x 160 region GEMM, the one-launch M = 1 GEMV, the tile GEMM, the skinny GEMM of up to
+# 16 and of 32 tokens and on weights past the L2s): the first launch of a kernel then happens under
+# the capture.
 _CAPTURE_CHILD = r"""
 import sys
 sys.path[:0] = [sys.argv[1] + "/rotor-rag_amd", sys.argv[1]]
@@ -111,7 +112,8 @@ from rotor import _hip
 from rotor.gpu_ternary import HIPTernaryOps
 hip = HIPTernaryOps(0)
 lib = _hip.load()
-for i, (M, N, K) in enumerate([(300, 640, 2560), (37, 640, 2560), (2048, 2560, 6912), (1, 6912, 2560)]):
+for i, (M, N, K) in enumerate([(300, 640, 2560), (37, 640, 2560), (2048, 2560, 6912), (1, 6912, 2560),
+                               (1024, 2560, 640), (5, 640, 2560), (20, 640, 2560), (3, 16384, 8256)]):
     print(f"capture case {i}: M={M} N={N} K={K}", flush=True)
     x, W, scale = O.make_linear_case(200 + i, M, N, K)
     w = hip.upload(O.pack_rotor(W), K, scale)
